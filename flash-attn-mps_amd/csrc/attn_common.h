@@ -68,3 +68,8 @@ FA_DEV float descale_of(const float* p, const int64_t* st, int64_t b, int kh) {
 
 // Host-side argument checks shared by fa_attn_fwd / fa_decode_fwd / fa_prefill_fwd.
 int fa_validate_attn(const fa_attn_args* a, const char* who);
+
+// The fp32 matrix-core kernel (attn_f32.hip): whether it takes these
+// (validated) arguments, and its launch with fa_attn_fwd's split partials.
+bool fa_f32_supported(const fa_attn_args& a);
+int fa_f32_launch(const fa_attn_args& a, void* stream);

@@ -1,0 +1,468 @@
+// Attention in single precision on the matrix cores: fp32 queries, keys and
+// values, one kernel for prefill and for decode (counterpart of the
+// reference's fp32 use of its fast and decode kernels,
+// flash_attn_mps/_attention.py:134-158, with the features of its tiled one,
+// kernels/attention.metal:29-51).
+//
+// What bounds it: v_mfma_f32_32x32x2_f32 does 64 FLOP per SIMD and clock
+// (157 TFLOP/s), 1/16 of the bf16 rate, so a 32-key x 32-column stage at d128
+// is 128 MFMAs = 8192 cycles against ~300 VALU instructions of softmax and
+// 32 KiB of K/V: prefill is MFMA-bound, and every score feature (softcap with
+// tanhf, ALiBi, masks) is a run-time branch that hides behind the MFMAs.
+// Decode is HBM-bound: a stage reads its 32 KiB in 8192 cycles per SIMD,
+// 1024 SIMDs x 32 KiB / 3.4 us = 9.8 TB/s, above what HBM delivers.  All
+// products, probabilities and sums are fp32, as in the generic kernel.
+//
+// * A workgroup takes 32 columns, (query head, query row) pairs of one KV
+//   head: 32 rows of one head in prefill, the group's heads at one row each
+//   in decode, or R rows of 32 / R heads between.  Its four waves take the
+//   32-key stages j = w, w + 4, ... (by absolute key, so a row's order of
+//   summation does not depend on the rest of the batch) and combine (m, l, O)
+//   through LDS at the end.  Splitting the keys over the waves, rather than
+//   giving each wave its own rows, quarters the longest chain of a causal
+//   block and lets a grid of 32-row blocks fill the 1024 SIMDs.
+// * S^T = K Q^T: lane (key l32, half hh) loads its key row 16 bytes at a
+//   time straight from global memory (dims 8 t + 4 hh .. +4 feed four MFMAs;
+//   the contraction order is free), Q^T comes from LDS in operand order.
+//   S^T's accumulator i then holds key 8 (i / 4) + 4 hh + i % 4 of the lane's
+//   column, which is the B operand of O^T += V^T P^T as it stands when V's
+//   lanes load that key's row: no shuffle, no LDS trip, no rounding of P.
+//   V lane m holds dims 4 m .. 4 m + 3 (one 16-byte load feeds four MFMAs,
+//   each of its own 32-dim block {4 m + n}).
+// * K and V move in halves (the row's first and second dims; the stage's
+//   first and last 16 keys), each loaded one half ahead of its MFMAs (2048
+//   cycles at d128, twice that with two waves on the SIMD).  Lifetimes of two
+//   halves let K and V share 64 registers, so two waves per SIMD fit without
+//   spills; whole K and V tiles in flight (128 registers) spilled 35.
+//   K/V go through registers: at 16 bytes per clock and CU they leave the
+//   load path three quarters idle, and LDS tiles would only add barriers.
+#include "attn_common.h"
+
+#include <climits>
+
+namespace {
+
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr int F32_COLS = 32, F32_STAGE = 32, F32_WAVES = 4;
+constexpr int F32_ROUND = F32_STAGE * F32_WAVES;   // keys per pass of the four waves
+
+struct F32Shape {
+  int log2_rows;    // a column block holds 2^log2_rows query rows of each of `heads` heads
+  int heads;        // query heads per workgroup
+  int tiles;        // workgroups per KV head: ceil(group / heads)
+  int n_qblocks;
+  int log2_page;    // >= 0: page size 2^log2_page; -1: any other page size; packed K/V unused
+  int vec_out;      // fp32 output rows take 16-byte stores
+};
+
+// 32-dim blocks of O^T (one, two, four or eight).
+template <int DV> constexpr int f32_blocks() { return DV <= 32 ? 1 : DV <= 64 ? 2 : DV <= 128 ? 4 : 8; }
+template <int DQ, int DV> constexpr size_t f32_lds_bytes() {
+  const size_t q = (size_t)(DQ / 8) * 64 * 16;
+  const size_t combine = (size_t)F32_WAVES * F32_COLS * (32 * f32_blocks<DV>() + 4 + 2) * 4;
+  return q > combine ? q : combine;
+}
+
+FA_DEV float f32_sum_hh(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+FA_DEV float f32_max_hh(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+FA_DEV uint64_t shfl_u64(uint64_t x, int src) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)(uint32_t)x);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)(uint32_t)(x >> 32));
+  return (uint64_t)hi << 32 | lo;
+}
+
+// DQ, DV: the tensors' head dims (multiples of 8).  V columns past DV inside
+// the 32-dim blocks re-read real columns and are not stored.
+template <int DQ, int DV, int MINB>
+__global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa_attn_args a, const F32Shape shp) {
+  static_assert(DQ % 8 == 0 && DV % 8 == 0 && DQ <= 256 && DV <= 256, "head dims");
+  constexpr int KT = DQ / 8;                       // 16-byte key pieces per lane
+  constexpr int NB = f32_blocks<DV>();
+  constexpr int VW = NB < 4 ? NB : 4;              // dims per lane and V load (one per block)
+  constexpr int VL = NB / VW;                      // V loads per key: 32 VW dims each
+  typedef __attribute__((ext_vector_type(VW))) float vpiece;
+
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // Work order: KV heads fastest (a KV head of a multiple of 8 stays on one
+  // XCD, whose L2 then serves all its query blocks), then head tiles,
+  // requests and splits; query blocks last to first, since causal ones are
+  // the longest.
+  const int S = a.num_splits, hk = (int)a.heads_k, group = (int)(a.heads_q / a.heads_k);
+  int64_t id = blockIdx.x;
+  const int kh = (int)(id % hk);
+  id /= hk;
+  const int tile = (int)(id % shp.tiles);
+  id /= shp.tiles;
+  const int64_t b = id % a.batch;
+  id /= a.batch;
+  const int split = (int)(id % S);
+  const int qb = shp.n_qblocks - 1 - (int)(id / S);
+  const RequestInfo r = load_request(a, b);
+  const int rl = shp.log2_rows, R = 1 << rl, q0 = qb << rl;
+  if (q0 >= r.q_len) return;
+  const int t0 = tile * shp.heads, nheads = min(shp.heads, group - t0);
+  const int h0 = kh * group + t0;
+
+  // This lane's column: head h0 + chead, query row q0 + crow, and the keys it
+  // sees, [lo, hi) (mask kinds: [0, hi), refined per key below).
+  const int chead = l32 >> rl, crow = l32 & (R - 1);
+  const bool col_ok = chead < nheads && q0 + crow < r.q_len;
+  const int qa = q0 + crow + r.k_len - r.q_len;
+  const int64_t tq = (int64_t)r.q_begin + q0 + (col_ok ? crow : 0);
+  const int hq = h0 + (col_ok ? chead : 0);
+  int lo = INT_MAX, hi = INT_MIN, mlo = -1, mhi = -1, mwin = -1;
+  if (col_ok) {
+    lo = 0, hi = r.k_len;
+    if (a.mask_kind == 0) {
+      if (r.causal) hi = min(hi, qa + 1);
+      if (a.window_right >= 0) hi = min(hi, qa + a.window_right + 1);
+      if (a.window_left >= 0) lo = max(qa - a.window_left, 0);
+    } else if (a.mask_kind == 1) {
+      mlo = a.mask_ranges[tq * a.ranges_stride[0]];
+      mhi = a.mask_ranges[tq * a.ranges_stride[0] + a.ranges_stride[1]];
+      mwin = a.mask_window;
+      hi = min(hi, max(qa, mlo >= 0 ? mhi : -1) + 1);
+    } else {
+      mhi = a.mask_prefix[b * a.prefix_stride];
+      mwin = a.mask_window_len[0];
+      hi = min(hi, qa + 1);
+    }
+    if (hi <= lo) lo = INT_MAX, hi = INT_MIN;   // a row without keys bounds nothing
+  }
+  // Keys of the workgroup, [kbeg, kend), and those every column sees.
+  const int kbeg = __builtin_amdgcn_readfirstlane(wave_min_i(lo));
+  const int kend = __builtin_amdgcn_readfirstlane(wave_max_i(hi));
+  const bool bounds = col_ok && hi > lo;
+  const int full_lo = __builtin_amdgcn_readfirstlane(wave_max_i(bounds ? lo : INT_MIN));
+  const int full_hi = __builtin_amdgcn_readfirstlane(wave_min_i(bounds ? hi : INT_MAX));
+  // A column without keys among columns that have some: masked everywhere.
+  const bool any_empty = __any(col_ok && !bounds) || a.mask_kind != 0;
+  // This split's rounds of 128 keys.
+  const int rnd0 = kbeg < kend ? kbeg / F32_ROUND : 0;
+  const int nrnd = kbeg < kend ? (kend + F32_ROUND - 1) / F32_ROUND - rnd0 : 0;
+  const int rb = rnd0 + (int)((int64_t)nrnd * split / S), re = rnd0 + (int)((int64_t)nrnd * (split + 1) / S);
+
+  // Q^T operands in LDS: piece t of lane (column l32, half hh) is dims
+  // 8 t + 4 hh .. +4 of the column's query (zeros for columns without one).
+  f32x4* const qs = (f32x4*)smem;
+  {
+    const float* qp = (const float*)a.q + tq * a.q_stride[0] + (int64_t)hq * a.q_stride[1] + 4 * hh;
+    for (int t = wave; t < KT; t += F32_WAVES) qs[t * 64 + lane] = col_ok ? *(const f32x4*)(qp + 8 * t) : f32x4{0, 0, 0, 0};
+  }
+  __syncthreads();
+
+  const float scale = a.softmax_scale * descale_of(a.q_descale, a.q_descale_stride, b, kh) *
+                      descale_of(a.k_descale, a.k_descale_stride, b, kh);
+  const float slope = a.alibi ? a.alibi[b * a.alibi_stride[0] + (int64_t)hq * a.alibi_stride[1]] : 0.0f;
+  const bool plain = a.softcap <= 0.0f && !a.alibi;
+  const float c_scale = scale * LOG2E;   // raw dot -> log2 units
+  const float cap = a.softcap, cap_in = cap > 0.0f ? scale / cap : 0.0f;
+
+  // A sink logit seeds the state of one wave of split 0 (max = sink, sum = 1).
+  const float sink = (a.sinks && split == 0 && wave == 0 && col_ok) ? a.sinks[(int64_t)hq * a.sink_stride] * LOG2E : -INFINITY;
+  float m_run = sink, l_run = sink > -INFINITY && hh == 0 ? 1.0f : 0.0f;
+  f32x16 o[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[n][i] = 0.0f;
+
+  const float* const khead = (const float*)a.k + (int64_t)kh * a.k_stride[2];
+  const float* const vhead = (const float*)a.v + (int64_t)kh * a.v_stride[2];
+  const int P = (int)a.page_size, lp = shp.log2_page;
+  const int32_t* const trow = P ? a.block_table + b * a.bt_stride[0] : nullptr;
+  // Row offsets (elements) of key k0 + l32 in K and V.  Keys outside
+  // [kbeg, kend) take a row inside it: what lies there is never read.
+  auto rows_of = [&](int k0, uint64_t& kr, uint64_t& vr) {
+    const int key = min(max(k0 + l32, kbeg), kend - 1);
+    const int64_t pos = (int64_t)r.k_base + r.left + key;
+    if (P) {
+      const int page = lp >= 0 ? (int)pos >> lp : (int)pos / P;
+      const int64_t blk = trow[(int64_t)page * a.bt_stride[1]];
+      const int64_t slot = (int)pos - page * P;
+      kr = (uint64_t)(blk * a.k_stride[0] + slot * a.k_stride[1]);
+      vr = (uint64_t)(blk * a.v_stride[0] + slot * a.v_stride[1]);
+    } else {
+      kr = (uint64_t)(pos * a.k_stride[1]);
+      vr = (uint64_t)(pos * a.v_stride[1]);
+    }
+  };
+  // K and V halves: the first KA key pieces and the rest, the stage's first
+  // and last eight V rows per lane half.
+  constexpr int KA = KT / 2;
+  f32x4 ka[KA], kb[KT - KA];
+  vpiece va[8][VL], vb[8][VL];
+  auto load_k = [&](uint64_t kr, auto& k, int t0) {
+    const float* p = khead + kr + 4 * hh + 8 * t0;
+#pragma unroll
+    for (int t = 0; t < (int)(sizeof(k) / 16); ++t) k[t] = *(const f32x4*)(p + 8 * t);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Element 4 m + n of the row feeds block n (VW = 4; likewise 2 m + n, m);
+  // lanes past the row's end re-read its last piece.
+  int vcol[VL];
+#pragma unroll
+  for (int u = 0; u < VL; ++u) vcol[u] = min(32 * VW * u + VW * l32, DV - VW);
+  auto load_v = [&](uint64_t vr, vpiece (&v)[8][VL], int half) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float* p = vhead + shfl_u64(vr, 16 * half + 8 * (i >> 2) + 4 * hh + (i & 3));
+#pragma unroll
+      for (int u = 0; u < VL; ++u) v[i][u] = *(const vpiece*)(p + vcol[u]);
+      if (i % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  if (rb < re) {
+    uint64_t kr, vr, kn, vn;
+    rows_of(F32_ROUND * rb + F32_STAGE * wave, kr, vr);
+    load_k(kr, ka, 0);
+    for (int rnd = rb; rnd < re; ++rnd) {
+      const int k0 = F32_ROUND * rnd + F32_STAGE * wave;
+      rows_of(k0 + F32_ROUND, kn, vn);   // the next stage's rows (past the last one: clamped, unused)
+      load_k(kr, kb, KA);
+      f32x16 s;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+      auto qk = [&](auto& k, int t0) {
+#pragma unroll
+        for (int t = 0; t < (int)(sizeof(k) / 16); ++t) {
+          const f32x4 q = qs[(t0 + t) * 64 + lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[t][e], q[e], s, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      qk(ka, 0);
+      load_v(vr, va, 0);
+      qk(kb, KA);
+      // s[i] = score of key k0 + 8 (i / 4) + 4 hh + i % 4.
+      const int key0 = k0 + 4 * hh;
+      if (plain) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] *= c_scale;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          float x = s[i] * scale;
+          if (cap > 0.0f) x = cap * tanhf(s[i] * cap_in);
+          x -= slope * (float)abs(qa - (key0 + 8 * (i >> 2) + (i & 3)));
+          s[i] = x * LOG2E;
+        }
+      }
+      const bool edge = k0 < kbeg || k0 + F32_STAGE > kend;
+      if (k0 < full_lo || k0 + F32_STAGE > full_hi || any_empty) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = key0 + 8 * (i >> 2) + (i & 3);
+          bool see = key >= lo && key < hi;
+          if (a.mask_kind == 1) {
+            const int diff = qa - key;
+            const bool in_win = mwin < 0 || diff < mwin;
+            see = see && ((diff >= 0 && in_win) || (mlo >= 0 && key >= mlo && key <= mhi && (!a.mask_clamp || in_win)));
+          } else if (a.mask_kind == 2) {
+            see = see && (key < mhi || qa - key < mwin);
+          }
+          s[i] = see ? s[i] : -INFINITY;
+        }
+      }
+      float mx = s[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+      const float m_new = fmaxf(m_run, f32_max_hh(mx));
+      const float mref = m_new == -INFINITY ? 0.0f : m_new;
+      if (__any(m_new != m_run)) {
+        const float f = fast_exp2(m_run - mref);   // 1 where the maximum stays
+        l_run *= f;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[n][i] *= f;
+      }
+      m_run = m_new;
+      float psum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[i] = fast_exp2(s[i] - mref);
+        psum += s[i];
+      }
+      l_run += psum;
+      auto pv = [&](vpiece (&v)[8][VL], int half) {
+        if (edge) {   // rows that are not the stage's own: no value of theirs may reach O
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int key = key0 + 16 * half + 8 * (i >> 2) + (i & 3);
+            const bool own = key >= kbeg && key < kend;
+#pragma unroll
+            for (int u = 0; u < VL; ++u)
+#pragma unroll
+              for (int n = 0; n < VW; ++n) v[i][u][n] = own ? v[i][u][n] : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int u = 0; u < VL; ++u)
+#pragma unroll
+            for (int n = 0; n < VW; ++n)
+              o[u * VW + n] =
+                  __builtin_amdgcn_mfma_f32_32x32x2f32(v[i][u][n], s[8 * half + i], o[u * VW + n], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(vr, vb, 1);
+      pv(va, 0);
+      kr = kn, vr = vn;
+      load_k(kr, ka, 0);
+      pv(vb, 1);
+    }
+  }
+
+  // Combine the four waves: per column m (log2 units), l and O^T through LDS.
+  const float lt = f32_sum_hh(l_run);
+  __syncthreads();   // every wave is done with the queries
+  float* const cm = (float*)smem;              // [4][32]
+  float* const cl = cm + F32_WAVES * F32_COLS; // [4][32]
+  constexpr int ROW = 32 * NB + 4;             // padded: one instruction's stores fall on distinct bank groups
+  float* const co = cl + F32_WAVES * F32_COLS; // [4][32][ROW]
+  if (hh == 0) {
+    cm[wave * F32_COLS + l32] = m_run;
+    cl[wave * F32_COLS + l32] = lt;
+  }
+  // o[u VW + n][i]: column l32, dim 32 VW u + VW (8 (i / 4) + 4 hh + i % 4) + n.
+  float* const row = co + (wave * F32_COLS + l32) * ROW;
+#pragma unroll
+  for (int u = 0; u < VL; ++u)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      vpiece w;
+#pragma unroll
+      for (int n = 0; n < VW; ++n) w[n] = o[u * VW + n][i];
+      *(vpiece*)(row + 32 * VW * u + VW * (8 * (i >> 2) + 4 * hh + (i & 3))) = w;
+    }
+  __syncthreads();
+  // Once per column: the waves' weights times the output scale (over cm) and
+  // the LSE (over cl's first row).
+  if (tid < F32_COLS) {
+    float M = cm[tid];
+#pragma unroll
+    for (int w = 1; w < F32_WAVES; ++w) M = fmaxf(M, cm[w * F32_COLS + tid]);
+    const float ref = M == -INFINITY ? 0.0f : M;
+    float fw[F32_WAVES], L = 0.0f;
+#pragma unroll
+    for (int w = 0; w < F32_WAVES; ++w) {
+      fw[w] = fast_exp2(cm[w * F32_COLS + tid] - ref);
+      L += cl[w * F32_COLS + tid] * fw[w];
+    }
+    const float norm = L > 0.0f ? descale_of(a.v_descale, a.v_descale_stride, b, kh) / L : 0.0f;
+#pragma unroll
+    for (int w = 0; w < F32_WAVES; ++w) cm[w * F32_COLS + tid] = fw[w] * norm;
+    cl[tid] = L > 0.0f ? M * LN2 + logf(L) : -INFINITY;
+  }
+  __syncthreads();
+  constexpr int D4 = DV / 4;
+  for (int idx = tid; idx < F32_COLS * D4; idx += 64 * F32_WAVES) {
+    const int c = idx / D4, d = 4 * (idx - c * D4);
+    const int ch = c >> rl, cr = q0 + (c & (R - 1));
+    if (ch >= nheads || cr >= r.q_len) continue;
+    f32x4 O = {0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < F32_WAVES; ++w) O += *(const f32x4*)(co + (w * F32_COLS + c) * ROW + d) * cm[w * F32_COLS + c];
+    const int64_t t = (int64_t)r.q_begin + cr, h = h0 + ch;
+    if (S > 1) {   // partials [S][T][Hq][Dv], LSEs [S][Hq][T], as the generic kernel's
+      *(f32x4*)(a.partial_out + ((split * a.total_q + t) * a.heads_q + h) * DV + d) = O;
+      if (d == 0) a.partial_lse[(split * a.heads_q + h) * a.total_q + t] = cl[c];
+    } else {
+      const int64_t off = t * a.out_stride[0] + h * a.out_stride[1] + (int64_t)d * a.out_stride[2];
+      if (shp.vec_out) {
+        *(f32x4*)((float*)a.out + off) = O;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_any(a.out, off + e * a.out_stride[2], a.out_dtype, O[e]);
+      }
+      if (d == 0) a.lse[h * a.lse_stride[0] + t * a.lse_stride[1]] = cl[c];
+    }
+  }
+}
+
+using F32Kernel = void (*)(fa_attn_args, F32Shape);
+struct F32Choice {
+  F32Kernel kern;
+  size_t lds;
+};
+
+// Workgroups per CU: 256 registers a wave at two (d128: K, V and O^T hold 64
+// each, S 16), 512 at one.
+template <int DQ, int DV, int MINB> F32Choice f32_choice() {
+  return F32Choice{attn_f32_kernel<DQ, DV, MINB>, f32_lds_bytes<DQ, DV>()};
+}
+
+F32Choice pick_f32(int64_t dq, int64_t dv) {
+  if (dq == 192 && dv == 128) return f32_choice<192, 128, 1>();
+  if (dq != dv) return F32Choice{nullptr, 0};
+  switch (dq) {
+    case 32: return f32_choice<32, 32, 4>();
+    case 64: return f32_choice<64, 64, 3>();
+    case 72: return f32_choice<72, 72, 2>();
+    case 80: return f32_choice<80, 80, 2>();
+    case 96: return f32_choice<96, 96, 2>();
+    case 128: return f32_choice<128, 128, 2>();
+    case 256: return f32_choice<256, 256, 1>();
+    default: return F32Choice{nullptr, 0};
+  }
+}
+
+// Every 16-byte piece of a Q, K or V row starts on a 16-byte boundary.
+bool rows_aligned(const void* p, const int64_t* st, int n) {
+  if ((uintptr_t)p & 15) return false;
+  for (int i = 0; i < n; ++i)
+    if (st[i] % 4) return false;
+  return st[n] == 1;
+}
+
+}  // namespace
+
+bool fa_f32_supported(const fa_attn_args& a) {
+  if (a.q_dtype != FA_F32 || a.k_dtype != FA_F32 || a.v_dtype != FA_F32) return false;
+  if (a.heads_k < 1 || a.heads_q % a.heads_k) return false;
+  if (!pick_f32(a.head_dim_qk, a.head_dim_v).kern) return false;
+  return rows_aligned(a.q, a.q_stride, 2) && rows_aligned(a.k, a.k_stride, 3) && rows_aligned(a.v, a.v_stride, 3);
+}
+
+int fa_f32_launch(const fa_attn_args& a, void* stream) {
+  const F32Choice ch = pick_f32(a.head_dim_qk, a.head_dim_v);
+  const int64_t group = a.heads_q / a.heads_k;
+  F32Shape shp;
+  shp.log2_rows = 0;
+  while (shp.log2_rows < 5 && (1ll << shp.log2_rows) < a.max_seqlen_q) ++shp.log2_rows;
+  shp.heads = F32_COLS >> shp.log2_rows;
+  if (shp.heads > group) shp.heads = (int)group;
+  shp.tiles = (int)fa_ceil_div(group, shp.heads);
+  const int64_t qblocks = fa_ceil_div(a.max_seqlen_q, 1ll << shp.log2_rows);
+  const int64_t blocks = a.heads_k * shp.tiles * a.batch * a.num_splits * qblocks;
+  FA_REQUIRE(qblocks <= 0x7fffffffll && blocks <= 0x7fffffffll, "fa_attn_fwd: grid too large");
+  shp.n_qblocks = (int)qblocks;
+  shp.log2_page = -1;
+  if (a.page_size && (a.page_size & (a.page_size - 1)) == 0)
+    for (shp.log2_page = 0; (1ll << shp.log2_page) < a.page_size; ++shp.log2_page) {}
+  shp.vec_out = a.out_dtype == FA_F32 && a.out_stride[2] == 1 && a.out_stride[0] % 4 == 0 && a.out_stride[1] % 4 == 0 &&
+                ((uintptr_t)a.out & 15) == 0;
+  const hipError_t err = hipFuncSetAttribute((const void*)ch.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ch.lds);
+  if (err != hipSuccess) {
+    fa_set_error("fa_attn_fwd: cannot reserve %zu bytes of LDS: %s", ch.lds, hipGetErrorString(err));
+    return FA_ERR_LAUNCH;
+  }
+  hipLaunchKernelGGL(ch.kern, dim3((unsigned)blocks), dim3(64 * F32_WAVES), ch.lds, (hipStream_t)stream, a, shp);
+  return fa_check_launch("fa_attn_fwd");
+}

@@ -158,11 +158,17 @@ extern "C" int fa_attn_fwd(const fa_attn_args* a, void* stream) {
   const dim3 grid((unsigned)fa_ceil_div(a->max_seqlen_q, GEN_WAVES), (unsigned)a->heads_q,
                   (unsigned)(a->batch * a->num_splits));
   hipStream_t s = (hipStream_t)stream;
-  switch (a->k_dtype) {
-    case FA_F16: rc = launch_generic_v<F16T>(*a, grid, s); break;
-    case FA_BF16: rc = launch_generic_v<BF16T>(*a, grid, s); break;
-    case FA_E4M3: rc = launch_generic_v<E4M3T>(*a, grid, s); break;
-    default: rc = launch_generic_v<F32T>(*a, grid, s); break;
+  // fp32 at the matrix-core kernel's head dims and alignment (any feature):
+  // dense causal 2 x 1024 tokens, 16/8 heads, d128 4940 us here.
+  if (fa_f32_supported(*a)) {
+    rc = fa_f32_launch(*a, stream);
+  } else {
+    switch (a->k_dtype) {
+      case FA_F16: rc = launch_generic_v<F16T>(*a, grid, s); break;
+      case FA_BF16: rc = launch_generic_v<BF16T>(*a, grid, s); break;
+      case FA_E4M3: rc = launch_generic_v<E4M3T>(*a, grid, s); break;
+      default: rc = launch_generic_v<F32T>(*a, grid, s); break;
+    }
   }
   if (rc || a->num_splits == 1) return rc;
   fa_merge_partials_args m;

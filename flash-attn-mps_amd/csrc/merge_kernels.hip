@@ -88,6 +88,58 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(const MergePartials
   if (lane == 0) p.lse[h * p.ls[0] + t * p.ls[1]] = empty ? -INFINITY : peak + logf(denom);
 }
 
+// fp32 partial rows contiguous over the head dimension, Dv <= 64 DIMS: split
+// weights once per wave (split s0 + j on lane j, broadcast with readlane)
+// and GROUP partial rows in flight, where the kernel above recomputes every
+// weight from memory for each 64 dims and waits for one row at a time.
+// Splits are added in order.
+template <int DIMS, int GROUP>
+__global__ __launch_bounds__(256) void merge_rows_kernel(const MergePartialsParams p) {
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= p.tokens * p.heads) return;
+  const int64_t t = row / p.heads, h = row - t * p.heads;
+  const int S = (int)p.splits, dim = (int)p.dim;
+  const float* const lse = p.plse + h * p.pls[1] + t * p.pls[2];
+  const float* const part = (const float*)p.part + t * p.ps[1] + h * p.ps[2];
+  const float lse0 = lane < S ? lse[lane * p.pls[0]] : -INFINITY;
+  float peak = lse0;
+  for (int s = lane + 64; s < S; s += 64) peak = fmaxf(peak, lse[s * p.pls[0]]);
+  peak = wave_max(peak);
+  float acc[DIMS], denom = 0.0f;
+#pragma unroll
+  for (int k = 0; k < DIMS; ++k) acc[k] = 0.0f;
+  for (int s0 = 0; s0 < S; s0 += 64) {
+    const float l = s0 == 0 ? lse0 : s0 + lane < S ? lse[(s0 + lane) * p.pls[0]] : -INFINITY;
+    const float w = merge_weight(l, peak);
+    denom += w;
+    const int cnt = min(64, S - s0);
+    for (int j = 0; j < cnt; j += GROUP) {
+      float x[GROUP][DIMS];
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u)
+#pragma unroll
+        for (int k = 0; k < DIMS; ++k)
+          x[u][k] = j + u < cnt && lane + 64 * k < dim ? part[(int64_t)(s0 + j + u) * p.ps[0] + lane + 64 * k] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) {
+        const float ws = j + u < cnt ? readlane_f(w, j + u) : 0.0f;
+#pragma unroll
+        for (int k = 0; k < DIMS; ++k) acc[k] = ws > 0.0f ? fmaf(ws, x[u][k], acc[k]) : acc[k];
+      }
+    }
+  }
+  denom = wave_sum(denom);
+  const bool empty = peak == -INFINITY;
+#pragma unroll
+  for (int k = 0; k < DIMS; ++k) {
+    const int d = lane + 64 * k;
+    if (d < dim)
+      store_any(p.out, t * p.os[0] + h * p.os[1] + d * p.os[2], p.out_dtype, empty ? 0.0f : acc[k] / denom);
+  }
+  if (lane == 0) p.lse[h * p.ls[0] + t * p.ls[1]] = empty ? -INFINITY : peak + logf(denom);
+}
+
 }  // namespace
 
 extern "C" int fa_merge_pair(const fa_merge_pair_args* a, void* stream) {
@@ -129,7 +181,9 @@ extern "C" int fa_merge_partials(const fa_merge_partials_args* a, void* stream) 
   const int64_t rows = p.tokens * p.heads;
   if (rows == 0) return FA_OK;
   FA_REQUIRE(fa_ceil_div(rows, 4) <= 0x7fffffffll, "fa_merge_partials: too many rows");
-  hipLaunchKernelGGL(merge_partials_kernel, dim3((unsigned)fa_ceil_div(rows, 4)), dim3(256), 0,   // a wave per row
-                     (hipStream_t)stream, p);
+  void (*kern)(MergePartialsParams) = merge_partials_kernel;
+  if (p.part_dtype == FA_F32 && p.ps[3] == 1 && p.dim <= 256 && p.splits >= 1 && p.splits <= 0x7fffffffll)
+    kern = p.dim <= 64 ? merge_rows_kernel<1, 16> : p.dim <= 128 ? merge_rows_kernel<2, 8> : merge_rows_kernel<4, 4>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)fa_ceil_div(rows, 4)), dim3(256), 0, (hipStream_t)stream, p);   // a wave per row
   return fa_check_launch("fa_merge_partials");
 }

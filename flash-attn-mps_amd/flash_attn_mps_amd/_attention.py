@@ -13,9 +13,11 @@ a HIP graph:
    K/V, E4M3 queries, ALiBi and per-request causality); in a batch of
    several requests the single-query ones go to the decode kernel first and
    fa_prefill_fwd skips them (FA_FLAG_SKIP_SINGLE_QUERY);
-3. everything else -> fa_attn_fwd, the generic kernel, with the reference's
-   split rule: deterministic -> 1, else num_splits, else min(32, ceil(max_k /
-   256)) when the row is decode-like or d > 256 (_attention.py:159-161).
+3. everything else -> fa_attn_fwd: fp32 calls at its head dims on the fp32
+   matrix-core kernel (split by f32_splits), the rest on the generic kernel
+   with the reference's split rule: deterministic -> 1, else num_splits, else
+   min(32, ceil(max_k / 256)) when the row is decode-like or d > 256
+   (_attention.py:159-161).
 
 Deterministic calls (vLLM's num_splits=1, the reference's fixed
 batch-invariant path, docs/contracts.md:76-79) take route 2 for every
@@ -135,6 +137,32 @@ def _partials(p, a, shape_out, shape_lse):
     pl = torch.empty(shape_lse, dtype=torch.float32, device=p.device)
     p.keep += [po, pl]
     a.partial_out, a.partial_lse = po.data_ptr(), pl.data_ptr()
+
+
+# Head dims of the fp32 matrix-core kernel (attn_f32.hip, which fa_attn_fwd
+# picks by itself) and the shape of its grid: 32 (head, row) columns per
+# workgroup, two workgroups per compute unit, rounds of 128 keys.
+_F32_DIMS = {(d, d) for d in (32, 64, 72, 80, 96, 128, 256)} | {(192, 128)}
+_F32_COLUMNS = 32
+_F32_WORKGROUPS = 512
+_F32_ROUND = 128
+
+
+def f32_splits(p):
+    """Key splits of an fp32 call on the matrix-core kernel: enough to put two
+    workgroups on every compute unit, each with a round of 128 keys or more;
+    None for calls of other types or head dims (the generic kernel's rule)."""
+    f32 = torch.float32
+    if not (p.q.dtype == p.k.dtype == p.v.dtype == f32 and (p.dim_qk, p.dim_v) in _F32_DIMS):
+        return None
+    rows = 1
+    while rows < _F32_COLUMNS and rows < p.max_q:
+        rows *= 2
+    group = p.heads // p.kv_heads
+    tiles = -(-group // min(group, _F32_COLUMNS // rows))
+    row_blocks = min(p.batch * -(-p.max_q // rows), p.tokens // rows + p.batch)
+    blocks = max(1, row_blocks * p.kv_heads * tiles)
+    return max(1, min(-(-_F32_WORKGROUPS // blocks), -(-p.visible_max // _F32_ROUND)))
 
 
 _SIDE = {}
@@ -263,7 +291,7 @@ def solve(p):
     if p.deterministic:
         splits = 1
     else:
-        splits = p.splits or (min(32, max(1, -(-p.max_k // 256))) if per_row else 1)
+        splits = p.splits or f32_splits(p) or (min(32, max(1, -(-p.max_k // 256))) if per_row else 1)
     if splits > 1:
         _partials(p, a, (splits, p.tokens, p.heads, p.dim_v), (splits, p.heads, p.tokens))
     a.num_splits = splits

@@ -17,7 +17,7 @@ num_splits is honoured.  fa_decode_fwd_noalloc plans the same way in C.
 import torch
 
 from . import _lib
-from ._attention import _partials, build_args
+from ._attention import _partials, build_args, f32_splits
 
 _MIN_WORKGROUPS = 1024
 _START_SPAN = 4096
@@ -143,15 +143,15 @@ def decode(p, out, splits=None):
 
     Returns (out, lse).  The split-KV kernels handle 16-bit queries over
     16-bit or FP8 caches at their compiled head dims; other dtype/dim/stride
-    combinations run the generic kernel with the reference's split rule
-    (_decode.py:63-64).
+    combinations run fa_attn_fwd: fp32 its matrix-core kernel, the rest the
+    generic kernel with the reference's split rule (_decode.py:63-64).
     """
     lse = torch.empty((p.heads, p.tokens), dtype=torch.float32, device=p.device)
     a = build_args(p, out, lse, max_q=1)
     a.causal, a.causal_by_batch = 0, None   # a right-aligned single query has no future keys
     if _run_split_kv(p, a, 1, splits):
         return out, lse
-    splits = splits or p.splits or max(1, min(32, -(-p.visible_max // 256)))
+    splits = splits or p.splits or f32_splits(p) or max(1, min(32, -(-p.visible_max // 256)))
     if splits > 1:
         _partials(p, a, (splits, p.tokens, p.heads, p.dim_v), (splits, p.heads, p.tokens))
     a.num_splits = splits

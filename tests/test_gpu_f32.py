@@ -1,0 +1,109 @@
+"""fp32 attention on the fp32 matrix-core kernel against the float64 oracle:
+edges of its 32-row blocks, 32-key stages and 128-key rounds, every head dim,
+packed (head, row) columns, splits, and the features it evaluates at run time.
+
+Tolerance: with |v| <= 5 and scores of standard deviation ~1, a score's fp32
+dot product over <= 256 dims is within ~16 * 2^-24 * |q||k| / sqrt(d) ~ 2e-6,
+a probability within twice that relative, and an output within 2 * 4e-6 *
+max|v| = 4e-5 (softcaps and ALiBi add terms of the same size).
+"""
+import pytest
+import torch
+
+from flash_attn_mps_amd import vllm
+from harness import assert_parity, attention, offsets, oracle_attention, seeded
+
+pytestmark = pytest.mark.gpu
+
+BAR = 4e-5
+
+
+def _packed(device, q_lens, k_lens, heads, kv_heads, dq, dv, seed):
+    q = seeded((sum(q_lens), heads, dq), seed, torch.float32, device)
+    k = seeded((sum(k_lens), kv_heads, dq), seed + 1, torch.float32, device)
+    v = seeded((sum(k_lens), kv_heads, dv), seed + 2, torch.float32, device)
+    return q, k, v, offsets(q_lens, device), offsets(k_lens, device)
+
+
+@pytest.mark.parametrize("dq,dv", [(32, 32), (64, 64), (72, 72), (80, 80), (96, 96), (128, 128), (192, 128), (256, 256)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_head_dims_and_tile_edges(device, dq, dv, causal):
+    """Row blocks of 1, 31, 32, 33 rows over 0, 1, 127, 128, 129, 300 keys."""
+    q_lens, k_lens = [1, 31, 32, 33, 2, 70], [0, 1, 127, 128, 129, 300]
+    q, k, v, cu_q, cu_k = _packed(device, q_lens, k_lens, 4, 2, dq, dv, 900)
+    got, lse = attention(q, k, v, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=70, max_seqlen_k=300,
+                         causal=causal)
+    ref, ref_lse = oracle_attention(q, k, v, cu_q, cu_k, causal=causal)
+    assert_parity(got, lse, ref, ref_lse, out_bar=BAR)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 16, 17])
+@pytest.mark.parametrize("heads,kv_heads", [(2, 2), (6, 2), (80, 2)])
+@pytest.mark.parametrize("splits", [0, 1, 3])
+def test_head_row_columns_over_paged_cache(device, rows, heads, kv_heads, splits):
+    """Groups of 1, 3 and 40 heads (tiles that a group does not fill), 1..17
+    rows per request, left padding, pages of 48, unread storage NaN."""
+    page, k_lens, left = 48, [max(rows, 1), 131, 700], [0, 5, 47]
+    cols = -(-(max(k_lens) + max(left)) // page)
+    table = torch.randperm(3 * cols, generator=torch.Generator().manual_seed(7)).reshape(3, cols).int()
+    k = torch.full((3 * cols, page, kv_heads, 64), float("nan"), device=device)
+    v = torch.full((3 * cols, page, kv_heads, 64), float("nan"), device=device)
+    for b, (n, pad) in enumerate(zip(k_lens, left)):
+        pos = torch.arange(pad, pad + n)
+        at = (table[b, pos // page].long(), pos % page)
+        k[at] = seeded((n, kv_heads, 64), 910 + b, torch.float32, device)
+        v[at] = seeded((n, kv_heads, 64), 920 + b, torch.float32, device)
+    q = seeded((3 * rows, heads, 64), 930, torch.float32, device)
+    sinks = seeded((heads,), 931, torch.float32, device)
+    cu_q, used = offsets([rows] * 3, device), torch.tensor(k_lens, dtype=torch.int32, device=device)
+    got, lse = attention(q, k, v, cu_seqlens_q=cu_q, seqused_k=used, max_seqlen_q=rows, max_seqlen_k=700,
+                         block_table=table.to(device), leftpad_k=torch.tensor(left, dtype=torch.int32, device=device),
+                         causal=True, s_aux=sinks, num_splits=splits)
+    ref, ref_lse = oracle_attention(q, k.nan_to_num(0), v.nan_to_num(0), cu_q, used_k=used, block_table=table,
+                                    leftpad=torch.tensor(left), causal=True, sinks=sinks)
+    assert_parity(got, lse, ref, ref_lse, out_bar=BAR)
+
+
+@pytest.mark.parametrize("feature", ["window", "right", "softcap", "alibi", "causal_flags", "descales", "prefix", "rolling"])
+def test_score_features(device, feature):
+    q_lens, k_lens = [40, 1, 100, 5], [40, 260, 100, 3]
+    q, k, v, cu_q, cu_k = _packed(device, q_lens, k_lens, 4, 2, 128, 128, 940)
+    kw = dict(causal=True)
+    if feature == "window":
+        kw.update(window_size=(33, 0))
+    elif feature == "right":
+        kw.update(causal=False, window_size=(70, 5))
+    elif feature == "softcap":
+        kw.update(softcap=2.0)
+    elif feature == "alibi":
+        kw.update(alibi_slopes=torch.tensor([0.5, 0.25, 0.0, 1.0], device=device), softcap=3.0)
+    elif feature == "causal_flags":
+        kw.update(causal=torch.tensor([True, False, False, True], device=device))
+    elif feature == "descales":
+        kw.update({n: seeded((4, 2), 950 + i, torch.float32, device).abs() + 0.1
+                   for i, n in enumerate(("q_descale", "k_descale", "v_descale"))})
+    elif feature == "prefix":
+        ranges = torch.full((146, 2), -1, dtype=torch.int32)
+        ranges[10:30] = torch.tensor([5, 35], dtype=torch.int32)
+        ranges[60:140] = torch.tensor([50, 99], dtype=torch.int32)
+        kw.update(mask_mod=vllm.mm_prefix_mask(20), aux_tensors=[ranges.to(device), cu_q])
+    else:
+        aux = [torch.tensor([3, 100, 0, 2], dtype=torch.int32, device=device),
+               torch.tensor([16], dtype=torch.int32, device=device)]
+        kw.update(mask_mod=vllm.rswa_mask(), aux_tensors=aux)
+    names = dict(window_size="window", alibi_slopes="alibi", mask_mod="mask", aux_tensors="aux")
+    okw = {names.get(n, n): x for n, x in kw.items()}
+    got, lse = attention(q, k, v, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=100, max_seqlen_k=260, **kw)
+    ref, ref_lse = oracle_attention(q, k, v, cu_q, cu_k, **okw)
+    assert_parity(got, lse, ref, ref_lse, out_bar=BAR)
+
+
+def test_rows_do_not_depend_on_the_batch(device):
+    """num_splits=1: a windowed request's rows are bit-identical alone (8 rows,
+    packed columns) and beside a longer one (32-row blocks)."""
+    q, k, v, cu_q, cu_k = _packed(device, [8, 90], [500, 333], 4, 2, 64, 64, 960)
+    run = dict(causal=True, window_size=(150, 0), num_splits=1, deterministic=True)
+    both, lse = attention(q, k, v, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=90, max_seqlen_k=500, **run)
+    alone, lse1 = attention(q[:8], k[:500], v[:500], cu_seqlens_q=cu_q[:2], cu_seqlens_k=cu_k[:2], max_seqlen_q=8,
+                            max_seqlen_k=500, **run)
+    assert torch.equal(both[:8], alone) and torch.equal(lse[:, :8], lse1)
