@@ -29,16 +29,24 @@
 //   lanes load that key's row: no shuffle, no LDS trip, no rounding of P.
 //   V lane m holds dims 4 m .. 4 m + 3 (one 16-byte load feeds four MFMAs,
 //   each of its own 32-dim block {4 m + n}).
-// * K and V move in halves (the row's first and second dims; the stage's
-//   first and last 16 keys), each loaded one half ahead of its MFMAs (2048
-//   cycles at d128, twice that with two waves on the SIMD).  Lifetimes of two
-//   halves let K and V share 64 registers, so two waves per SIMD fit without
-//   spills; whole K and V tiles in flight (128 registers) spilled 35.
+// * K and V move in quarters (of the row's dims; of the stage's keys), each
+//   loaded one quarter ahead of its MFMAs (1024 cycles at d128, three times
+//   that with three waves on the SIMD).  K and V then share 32 registers and
+//   three workgroups fit a CU at d128, four at d64.  Same process against
+//   halves (64 registers, two workgroups): 2 x 4096 tokens 16/8 heads d128
+//   2338 -> 2238 us (123 TFLOP/s; a 8192^3 fp32 matrix product of the library
+//   154), 2 x 1024 causal d64 68.1 -> 61.8, d128 unchanged at 111; whole tiles
+//   in flight (128 registers) spilled 35.
 //   K/V go through registers: at 16 bytes per clock and CU they leave the
 //   load path three quarters idle, and LDS tiles would only add barriers.
+//   Two accumulators for S^T instead of one chain: no change.
+// * Measured (generic kernel before): 2 x 1024 tokens causal, 16/8 heads,
+//   d128 4971 -> 111 us (77 TFLOP/s; 1024 workgroups for 256 CUs); decode of
+//   4 requests x 2048 keys 252 + 14 (merge) -> 16 + 4 us.
 #include "attn_common.h"
 
 #include <climits>
+#include <type_traits>
 
 namespace {
 
@@ -61,7 +69,7 @@ struct F32Shape {
 template <int DV> constexpr int f32_blocks() { return DV <= 32 ? 1 : DV <= 64 ? 2 : DV <= 128 ? 4 : 8; }
 template <int DQ, int DV> constexpr size_t f32_lds_bytes() {
   const size_t q = (size_t)(DQ / 8) * 64 * 16;
-  const size_t combine = (size_t)F32_WAVES * F32_COLS * (32 * f32_blocks<DV>() + 4 + 2) * 4;
+  const size_t combine = (size_t)F32_COLS * (2 * (32 * f32_blocks<DV>() + 4) + 2 * F32_WAVES) * 4;
   return q > combine ? q : combine;
 }
 
@@ -99,15 +107,15 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   // requests and splits; query blocks last to first, since causal ones are
   // the longest.
   const int S = a.num_splits, hk = (int)a.heads_k, group = (int)(a.heads_q / a.heads_k);
-  int64_t id = blockIdx.x;
-  const int kh = (int)(id % hk);
-  id /= hk;
-  const int tile = (int)(id % shp.tiles);
-  id /= shp.tiles;
-  const int64_t b = id % a.batch;
-  id /= a.batch;
-  const int split = (int)(id % S);
-  const int qb = shp.n_qblocks - 1 - (int)(id / S);
+  uint32_t id = blockIdx.x;   // 32-bit: a 64-bit division costs ~100 instructions
+  const int kh = (int)(id % (uint32_t)hk);
+  id /= (uint32_t)hk;
+  const int tile = (int)(id % (uint32_t)shp.tiles);
+  id /= (uint32_t)shp.tiles;
+  const int64_t b = id % (uint32_t)a.batch;
+  id /= (uint32_t)a.batch;
+  const int split = (int)(id % (uint32_t)S);
+  const int qb = shp.n_qblocks - 1 - (int)(id / (uint32_t)S);
   const RequestInfo r = load_request(a, b);
   const int rl = shp.log2_rows, R = 1 << rl, q0 = qb << rl;
   if (q0 >= r.q_len) return;
@@ -153,15 +161,6 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   const int nrnd = kbeg < kend ? (kend + F32_ROUND - 1) / F32_ROUND - rnd0 : 0;
   const int rb = rnd0 + (int)((int64_t)nrnd * split / S), re = rnd0 + (int)((int64_t)nrnd * (split + 1) / S);
 
-  // Q^T operands in LDS: piece t of lane (column l32, half hh) is dims
-  // 8 t + 4 hh .. +4 of the column's query (zeros for columns without one).
-  f32x4* const qs = (f32x4*)smem;
-  {
-    const float* qp = (const float*)a.q + tq * a.q_stride[0] + (int64_t)hq * a.q_stride[1] + 4 * hh;
-    for (int t = wave; t < KT; t += F32_WAVES) qs[t * 64 + lane] = col_ok ? *(const f32x4*)(qp + 8 * t) : f32x4{0, 0, 0, 0};
-  }
-  __syncthreads();
-
   const float scale = a.softmax_scale * descale_of(a.q_descale, a.q_descale_stride, b, kh) *
                       descale_of(a.k_descale, a.k_descale_stride, b, kh);
   const float slope = a.alibi ? a.alibi[b * a.alibi_stride[0] + (int64_t)hq * a.alibi_stride[1]] : 0.0f;
@@ -198,15 +197,16 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
       vr = (uint64_t)(pos * a.v_stride[1]);
     }
   };
-  // K and V halves: the first KA key pieces and the rest, the stage's first
-  // and last eight V rows per lane half.
-  constexpr int KA = KT / 2;
-  f32x4 ka[KA], kb[KT - KA];
-  vpiece va[8][VL], vb[8][VL];
-  auto load_k = [&](uint64_t kr, auto& k, int t0) {
-    const float* p = khead + kr + 4 * hh + 8 * t0;
+  // Quarters: key pieces [KT q / 4, KT (q + 1) / 4) and the stage's V rows
+  // 8 q + 4 hh .. +4; buffers 0 and 1 take turns.
+  constexpr int KQ = (KT + 3) / 4;
+  f32x4 kq[2][KQ];
+  vpiece vq[2][4][VL];
+  auto load_k = [&](uint64_t kr, auto q) {
+    constexpr int Q = decltype(q)::value, T0 = KT * Q / 4, T1 = KT * (Q + 1) / 4;
+    const float* p = khead + kr + 4 * hh;
 #pragma unroll
-    for (int t = 0; t < (int)(sizeof(k) / 16); ++t) k[t] = *(const f32x4*)(p + 8 * t);
+    for (int t = T0; t < T1; ++t) kq[Q & 1][t - T0] = *(const f32x4*)(p + 8 * t);
     __builtin_amdgcn_sched_barrier(0);
   };
   // Element 4 m + n of the row feeds block n (VW = 4; likewise 2 m + n, m);
@@ -214,39 +214,66 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   int vcol[VL];
 #pragma unroll
   for (int u = 0; u < VL; ++u) vcol[u] = min(32 * VW * u + VW * l32, DV - VW);
-  auto load_v = [&](uint64_t vr, vpiece (&v)[8][VL], int half) {
+  auto load_v = [&](uint64_t vr, auto q) {
+    constexpr int Q = decltype(q)::value;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float* p = vhead + shfl_u64(vr, 16 * half + 8 * (i >> 2) + 4 * hh + (i & 3));
+    for (int i = 0; i < 4; ++i) {
+      const float* p = vhead + shfl_u64(vr, 8 * Q + 4 * hh + i);
 #pragma unroll
-      for (int u = 0; u < VL; ++u) v[i][u] = *(const vpiece*)(p + vcol[u]);
+      for (int u = 0; u < VL; ++u) vq[Q & 1][i][u] = *(const vpiece*)(p + vcol[u]);
       if (i % 2) __builtin_amdgcn_sched_barrier(0);
     }
   };
+  const std::integral_constant<int, 0> q0c;
+  const std::integral_constant<int, 1> q1c;
+  const std::integral_constant<int, 2> q2c;
+  const std::integral_constant<int, 3> q3c;
 
+  // The first keys, then the queries: both round trips to memory run together.
+  uint64_t kr = 0, vr = 0, kn, vn;
   if (rb < re) {
-    uint64_t kr, vr, kn, vn;
     rows_of(F32_ROUND * rb + F32_STAGE * wave, kr, vr);
-    load_k(kr, ka, 0);
+    load_k(kr, q0c);
+  }
+  // Q^T operands in LDS: piece t of lane (column l32, half hh) is dims
+  // 8 t + 4 hh .. +4 of the column's query (zeros for columns without one).
+  f32x4* const qs = (f32x4*)smem;
+  {
+    const float* qp = (const float*)a.q + tq * a.q_stride[0] + (int64_t)hq * a.q_stride[1] + 4 * hh;
+    constexpr int TW = (KT + F32_WAVES - 1) / F32_WAVES;
+    f32x4 x[TW];
+#pragma unroll
+    for (int i = 0; i < TW; ++i) x[i] = *(const f32x4*)(qp + 8 * min(wave + F32_WAVES * i, KT - 1));
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+      if (wave + F32_WAVES * i < KT) qs[(wave + F32_WAVES * i) * 64 + lane] = col_ok ? x[i] : f32x4{0, 0, 0, 0};
+  }
+  __syncthreads();
+  if (rb < re) {
     for (int rnd = rb; rnd < re; ++rnd) {
       const int k0 = F32_ROUND * rnd + F32_STAGE * wave;
       rows_of(k0 + F32_ROUND, kn, vn);   // the next stage's rows (past the last one: clamped, unused)
-      load_k(kr, kb, KA);
       f32x16 s;
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-      auto qk = [&](auto& k, int t0) {
+      auto qk = [&](auto q) {
+        constexpr int Q = decltype(q)::value, T0 = KT * Q / 4, T1 = KT * (Q + 1) / 4;
 #pragma unroll
-        for (int t = 0; t < (int)(sizeof(k) / 16); ++t) {
-          const f32x4 q = qs[(t0 + t) * 64 + lane];
+        for (int t = T0; t < T1; ++t) {
+          const f32x4 x = qs[t * 64 + lane];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[t][e], q[e], s, 0, 0, 0);
+          for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq[Q & 1][t - T0][e], x[e], s, 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       };
-      qk(ka, 0);
-      load_v(vr, va, 0);
-      qk(kb, KA);
+      load_k(kr, q1c);
+      qk(q0c);
+      load_k(kr, q2c);
+      qk(q1c);
+      load_k(kr, q3c);
+      qk(q2c);
+      load_v(vr, q0c);
+      qk(q3c);
       // s[i] = score of key k0 + 8 (i / 4) + 4 hh + i % 4.
       const int key0 = k0 + 4 * hh;
       if (plain) {
@@ -298,91 +325,112 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
         psum += s[i];
       }
       l_run += psum;
-      auto pv = [&](vpiece (&v)[8][VL], int half) {
+      auto pv = [&](auto q) {
+        constexpr int Q = decltype(q)::value;
         if (edge) {   // rows that are not the stage's own: no value of theirs may reach O
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int key = key0 + 16 * half + 8 * (i >> 2) + (i & 3);
-            const bool own = key >= kbeg && key < kend;
+          for (int i = 0; i < 4; ++i) {
+            const bool own = key0 + 8 * Q + i >= kbeg && key0 + 8 * Q + i < kend;
 #pragma unroll
             for (int u = 0; u < VL; ++u)
 #pragma unroll
-              for (int n = 0; n < VW; ++n) v[i][u][n] = own ? v[i][u][n] : 0.0f;
+              for (int n = 0; n < VW; ++n) vq[Q & 1][i][u][n] = own ? vq[Q & 1][i][u][n] : 0.0f;
           }
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int u = 0; u < VL; ++u)
 #pragma unroll
             for (int n = 0; n < VW; ++n)
               o[u * VW + n] =
-                  __builtin_amdgcn_mfma_f32_32x32x2f32(v[i][u][n], s[8 * half + i], o[u * VW + n], 0, 0, 0);
+                  __builtin_amdgcn_mfma_f32_32x32x2f32(vq[Q & 1][i][u][n], s[4 * Q + i], o[u * VW + n], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       };
       __builtin_amdgcn_sched_barrier(0);
-      load_v(vr, vb, 1);
-      pv(va, 0);
+      load_v(vr, q1c);
+      pv(q0c);
+      load_v(vr, q2c);
+      pv(q1c);
+      load_v(vr, q3c);
+      pv(q2c);
       kr = kn, vr = vn;
-      load_k(kr, ka, 0);
-      pv(vb, 1);
+      load_k(kr, q0c);
+      pv(q3c);
     }
   }
 
-  // Combine the four waves: per column m (log2 units), l and O^T through LDS.
+  // Combine the four waves: per column the common max and the sum of the
+  // scaled (l, O^T), O^T pairwise through LDS (waves 2, 3 onto 0, 1, then 1
+  // onto 0), which takes half the room of four at once.
   const float lt = f32_sum_hh(l_run);
   __syncthreads();   // every wave is done with the queries
   float* const cm = (float*)smem;              // [4][32]
   float* const cl = cm + F32_WAVES * F32_COLS; // [4][32]
   constexpr int ROW = 32 * NB + 4;             // padded: one instruction's stores fall on distinct bank groups
-  float* const co = cl + F32_WAVES * F32_COLS; // [4][32][ROW]
+  float* const co = cl + F32_WAVES * F32_COLS; // [2][32][ROW]
   if (hh == 0) {
     cm[wave * F32_COLS + l32] = m_run;
     cl[wave * F32_COLS + l32] = lt;
   }
+  __syncthreads();
+  float M = cm[l32], L = 0.0f;
+#pragma unroll
+  for (int w = 1; w < F32_WAVES; ++w) M = fmaxf(M, cm[w * F32_COLS + l32]);
+  const float ref = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+  for (int w = 0; w < F32_WAVES; ++w) L += cl[w * F32_COLS + l32] * fast_exp2(cm[w * F32_COLS + l32] - ref);
+  const float norm = L > 0.0f ? descale_of(a.v_descale, a.v_descale_stride, b, kh) / L : 0.0f;
+  const float fw = fast_exp2(m_run - ref) * norm;
   // o[u VW + n][i]: column l32, dim 32 VW u + VW (8 (i / 4) + 4 hh + i % 4) + n.
-  float* const row = co + (wave * F32_COLS + l32) * ROW;
+  auto piece = [&](int w, int u, int i) -> vpiece* {
+    return (vpiece*)(co + (w * F32_COLS + l32) * ROW + 32 * VW * u + VW * (8 * (i >> 2) + 4 * hh + (i & 3)));
+  };
+  auto put = [&](int w) {
 #pragma unroll
-  for (int u = 0; u < VL; ++u)
+    for (int u = 0; u < VL; ++u)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      vpiece w;
+      for (int i = 0; i < 16; ++i) {
+        vpiece x;
 #pragma unroll
-      for (int n = 0; n < VW; ++n) w[n] = o[u * VW + n][i];
-      *(vpiece*)(row + 32 * VW * u + VW * (8 * (i >> 2) + 4 * hh + (i & 3))) = w;
-    }
+        for (int n = 0; n < VW; ++n) x[n] = o[u * VW + n][i];
+        *piece(w, u, i) = x;
+      }
+  };
+  auto add = [&](int w) {
+#pragma unroll
+    for (int u = 0; u < VL; ++u)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const vpiece x = *piece(w, u, i);
+#pragma unroll
+        for (int n = 0; n < VW; ++n) o[u * VW + n][i] += x[n];
+      }
+  };
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[n][i] *= fw;
+  if (wave >= 2) put(wave - 2);
   __syncthreads();
-  // Once per column: the waves' weights times the output scale (over cm) and
-  // the LSE (over cl's first row).
-  if (tid < F32_COLS) {
-    float M = cm[tid];
-#pragma unroll
-    for (int w = 1; w < F32_WAVES; ++w) M = fmaxf(M, cm[w * F32_COLS + tid]);
-    const float ref = M == -INFINITY ? 0.0f : M;
-    float fw[F32_WAVES], L = 0.0f;
-#pragma unroll
-    for (int w = 0; w < F32_WAVES; ++w) {
-      fw[w] = fast_exp2(cm[w * F32_COLS + tid] - ref);
-      L += cl[w * F32_COLS + tid] * fw[w];
-    }
-    const float norm = L > 0.0f ? descale_of(a.v_descale, a.v_descale_stride, b, kh) / L : 0.0f;
-#pragma unroll
-    for (int w = 0; w < F32_WAVES; ++w) cm[w * F32_COLS + tid] = fw[w] * norm;
-    cl[tid] = L > 0.0f ? M * LN2 + logf(L) : -INFINITY;
+  if (wave < 2) add(wave);
+  if (wave == 1) put(1);
+  if (wave == 0) put(0);
+  __syncthreads();
+  const float lse = L > 0.0f ? M * LN2 + logf(L) : -INFINITY;
+  if (wave == 0 && hh == 0 && col_ok) {
+    if (S > 1) a.partial_lse[((int64_t)split * a.heads_q + hq) * a.total_q + tq] = lse;
+    else a.lse[hq * a.lse_stride[0] + tq * a.lse_stride[1]] = lse;
   }
-  __syncthreads();
   constexpr int D4 = DV / 4;
   for (int idx = tid; idx < F32_COLS * D4; idx += 64 * F32_WAVES) {
     const int c = idx / D4, d = 4 * (idx - c * D4);
     const int ch = c >> rl, cr = q0 + (c & (R - 1));
     if (ch >= nheads || cr >= r.q_len) continue;
-    f32x4 O = {0, 0, 0, 0};
-#pragma unroll
-    for (int w = 0; w < F32_WAVES; ++w) O += *(const f32x4*)(co + (w * F32_COLS + c) * ROW + d) * cm[w * F32_COLS + c];
+    const f32x4 O = *(const f32x4*)(co + c * ROW + d) + *(const f32x4*)(co + (F32_COLS + c) * ROW + d);
     const int64_t t = (int64_t)r.q_begin + cr, h = h0 + ch;
     if (S > 1) {   // partials [S][T][Hq][Dv], LSEs [S][Hq][T], as the generic kernel's
       *(f32x4*)(a.partial_out + ((split * a.total_q + t) * a.heads_q + h) * DV + d) = O;
-      if (d == 0) a.partial_lse[(split * a.heads_q + h) * a.total_q + t] = cl[c];
     } else {
       const int64_t off = t * a.out_stride[0] + h * a.out_stride[1] + (int64_t)d * a.out_stride[2];
       if (shp.vec_out) {
@@ -391,7 +439,6 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
 #pragma unroll
         for (int e = 0; e < 4; ++e) store_any(a.out, off + e * a.out_stride[2], a.out_dtype, O[e]);
       }
-      if (d == 0) a.lse[h * a.lse_stride[0] + t * a.lse_stride[1]] = cl[c];
     }
   }
 }
@@ -402,22 +449,22 @@ struct F32Choice {
   size_t lds;
 };
 
-// Workgroups per CU: 256 registers a wave at two (d128: K, V and O^T hold 64
-// each, S 16), 512 at one.
+// Workgroups per CU (waves per SIMD): 168 registers at three (d128 spills
+// 14), 128 at four; d256 holds 128 for O^T alone and runs one.
 template <int DQ, int DV, int MINB> F32Choice f32_choice() {
   return F32Choice{attn_f32_kernel<DQ, DV, MINB>, f32_lds_bytes<DQ, DV>()};
 }
 
 F32Choice pick_f32(int64_t dq, int64_t dv) {
-  if (dq == 192 && dv == 128) return f32_choice<192, 128, 1>();
+  if (dq == 192 && dv == 128) return f32_choice<192, 128, 2>();
   if (dq != dv) return F32Choice{nullptr, 0};
   switch (dq) {
     case 32: return f32_choice<32, 32, 4>();
-    case 64: return f32_choice<64, 64, 3>();
-    case 72: return f32_choice<72, 72, 2>();
-    case 80: return f32_choice<80, 80, 2>();
-    case 96: return f32_choice<96, 96, 2>();
-    case 128: return f32_choice<128, 128, 2>();
+    case 64: return f32_choice<64, 64, 4>();
+    case 72: return f32_choice<72, 72, 3>();
+    case 80: return f32_choice<80, 80, 3>();
+    case 96: return f32_choice<96, 96, 3>();
+    case 128: return f32_choice<128, 128, 3>();
     case 256: return f32_choice<256, 256, 1>();
     default: return F32Choice{nullptr, 0};
   }

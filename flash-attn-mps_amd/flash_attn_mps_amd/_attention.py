@@ -141,17 +141,21 @@ def _partials(p, a, shape_out, shape_lse):
 
 # Head dims of the fp32 matrix-core kernel (attn_f32.hip, which fa_attn_fwd
 # picks by itself) and the shape of its grid: 32 (head, row) columns per
-# workgroup, two workgroups per compute unit, rounds of 128 keys.
+# workgroup, rounds of 128 keys.
 _F32_DIMS = {(d, d) for d in (32, 64, 72, 80, 96, 128, 256)} | {(192, 128)}
 _F32_COLUMNS = 32
-_F32_WORKGROUPS = 512
 _F32_ROUND = 128
 
 
 def f32_splits(p):
-    """Key splits of an fp32 call on the matrix-core kernel: enough to put two
-    workgroups on every compute unit, each with a round of 128 keys or more;
-    None for calls of other types or head dims (the generic kernel's rule)."""
+    """Key splits of an fp32 call on the matrix-core kernel (a round of 128
+    keys or more each); None for calls of other types or head dims (the
+    generic kernel's rule).  One query row per request is bound by memory and
+    wants two workgroups per compute unit (4 x 2048 keys, 16/8 heads: 4 / 8 /
+    16 splits 39.0 / 28.6 / 28.2 us a call; 4 x 8192: 8 / 16 / 32 splits 64.4 /
+    58.3 / 73.5).  More rows are bound by the matrix cores, and partials cost
+    more than idle compute units until most of them idle (2 x 256 tokens, 256
+    workgroups: 1 / 2 splits 19.5 / 29.4 us; 1 x 2048: 177 / 204)."""
     f32 = torch.float32
     if not (p.q.dtype == p.k.dtype == p.v.dtype == f32 and (p.dim_qk, p.dim_v) in _F32_DIMS):
         return None
@@ -162,7 +166,8 @@ def f32_splits(p):
     tiles = -(-group // min(group, _F32_COLUMNS // rows))
     row_blocks = min(p.batch * -(-p.max_q // rows), p.tokens // rows + p.batch)
     blocks = max(1, row_blocks * p.kv_heads * tiles)
-    return max(1, min(-(-_F32_WORKGROUPS // blocks), -(-p.visible_max // _F32_ROUND)))
+    wanted = -(-512 // blocks) if p.max_q == 1 else 256 // blocks
+    return max(1, min(wanted, -(-p.visible_max // _F32_ROUND)))
 
 
 _SIDE = {}
