@@ -35,7 +35,7 @@
 //   XOR-swizzled); K operands are widened in registers after 8-byte reads,
 //   V^T comes through ds_read_b64_tr_b8 and is widened the same way.
 // * Supports 16-bit queries over K/V of their type or E4M3 (with descales),
-//   head dims 64 and 128 (Dqk = Dv), outputs of the query's type, packed or
+//   E4M3 queries over E4M3 K/V (one row per request), head dims 64 and 128 (Dqk = Dv), outputs of the query's type, packed or
 //   paged K/V (page size a multiple of 16), sinks, softcap, windows, 1-16
 //   query rows per request; the host keeps other combinations on the VALU
 //   kernel.  Neighbouring KV heads (64-dim, or 128-dim E4M3) can run in
@@ -127,7 +127,13 @@ FA_DEV void wait_dma_groups(int n) {
 // with each column's probabilities zeroed for the other head's half, so
 // every column accumulates only its own head's values.  Descales are per
 // column (its KV head).
-template <typename T, int D, bool CAP, typename KT = T, int PACK = 1>
+// QF8: E4M3 queries (with E4M3 K/V, T = fp16, which holds both exactly).
+// Probabilities then stay at fp32 accuracy, as in the kernels that compute
+// them on the VALU: P = hi + lo, two fp16 values (22 bits; the remainder is
+// below 2^-24 of the largest), and P.V runs on both.  The matrix cores have
+// the room: 24 MFMAs a stage at d128 are 768 cycles per 8 KiB and SIMD, four
+// times the rate HBM delivers.
+template <typename T, int D, bool CAP, typename KT = T, int PACK = 1, bool QF8 = false>
 __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_attn_args a, const int span) {
   static_assert(D == 64 || D == 128 || D == 256, "rows of 64, 128 or 256 elements");
   static_assert((PACK == 1 && D <= 128) || (PACK == 2 && (D == 128 || (D == 256 && KT::id == FA_E4M3))),
@@ -144,6 +150,8 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
   constexpr int KBYTES = KG * KGROUP, SLOT = gqa_slot_bytes<D, FP8>(), NSLOT = gqa_slots<D, FP8, PACK>();
   static_assert(NSLOT >= 2, "a stage's two slots");
   constexpr bool RING2 = NSLOT == 4;      // slots hold two stages (E4M3, unpaired)
+  static_assert(!QF8 || (FP8 && T::id == FA_F16), "E4M3 queries: E4M3 K/V, fp16 products");
+  constexpr int PT = QF8 ? 2 : 1;         // 16-bit terms of a probability
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
@@ -195,7 +203,17 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
   // query (token ctok, head h0 + chead), dims 16 kk + 8 hh .. +8 (zeros for
   // columns past the group or the request's tokens).
   u32x4 qop[KPH];
-  {
+  if constexpr (QF8) {
+    const uint8_t* qp = (const uint8_t*)a.q + (int64_t)(r.q_begin + (col_ok ? ctok : 0)) * a.q_stride[0] +
+                        (int64_t)(h0 + (col_ok ? chead : 0)) * a.q_stride[1] + 8 * hh;
+#pragma unroll
+    for (int kk = 0; kk < KPH; ++kk) {
+      const u32x2 w = *(const u32x2*)(qp + 16 * kk);
+      const u32x4 x = {widen_fp8_pair<T, false>(w[0]), widen_fp8_pair<T, true>(w[0]), widen_fp8_pair<T, false>(w[1]),
+                       widen_fp8_pair<T, true>(w[1])};
+      qop[kk] = col_ok ? x : u32x4{0u, 0u, 0u, 0u};
+    }
+  } else {
     const uint16_t* qp = (const uint16_t*)a.q + (int64_t)(r.q_begin + (col_ok ? ctok : 0)) * a.q_stride[0] +
                          (int64_t)(h0 + (col_ok ? chead : 0)) * a.q_stride[1] + 8 * hh;
 #pragma unroll
@@ -495,14 +513,22 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
     l_run += psum;
     // P^T operands per head half: a column's probabilities for its own
     // head's half of the V rows, zeros for the other half.
-    u32x4 pop[PACK][2];
+    u32x4 pop[PACK][2][PT];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const uint32_t w = pack2<T>(s[8 * c + 2 * q], s[8 * c + 2 * q + 1]);
+        float x = s[8 * c + 2 * q], y = s[8 * c + 2 * q + 1];
 #pragma unroll
-        for (int u = 0; u < PACK; ++u) pop[u][c][q] = PACK == 1 || cpart == u ? w : 0u;
+        for (int t = 0; t < PT; ++t) {
+          const uint32_t w = pack2<T>(x, y);
+#pragma unroll
+          for (int u = 0; u < PACK; ++u) pop[u][c][t][q] = PACK == 1 || cpart == u ? w : 0u;
+          if constexpr (QF8) {
+            x -= f16_bits_to_f32(w & 0xffffu);
+            y -= f16_bits_to_f32(w >> 16);
+          }
+        }
       }
     // V(i) landed; newer: K(i + 1) with one-stage rings; stage i + 1 and
     // K(i + 2) with two-stage rings.
@@ -530,7 +556,8 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
           const u32x2 hi = lds_read_tr(vb, vrd + 4 * 128);
           av = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
-        o[db % DBH] = mfma32<T>(av, pop[db / DBH][c], o[db % DBH]);
+#pragma unroll
+        for (int t = 0; t < PT; ++t) o[db % DBH] = mfma32<T>(av, pop[db / DBH][c][t], o[db % DBH]);
       }
     wait_lds();   // V reads of stage i done
     if constexpr (RING2) {

@@ -1,6 +1,6 @@
 // Variants of the matrix-core GQA decode kernel (decode_gqa.h) and their
-// selection: 16-bit queries over K/V of the same type or E4M3, Dqk = Dv in
-// {64, 128}, with and without softcap; neighbouring 64-dim heads, and
+// selection: 16-bit queries over K/V of the same type or E4M3, E4M3 queries
+// over E4M3 K/V, Dqk = Dv in {64, 128}, with and without softcap; neighbouring 64-dim heads, and
 // 128-dim E4M3 heads, stored next to each other run two KV heads per
 // workgroup (PACK = 2).
 #include "decode_gqa.h"
@@ -15,21 +15,22 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // head and page strides of K/V (`kvb` bytes per element) and the query's
 // token and head strides.
 bool chunks_aligned(const fa_attn_args& a, int kvb) {
-  if (!aligned16(a.q) || !aligned16(a.k) || !aligned16(a.v)) return false;
+  const bool fp8q = a.q_dtype == FA_E4M3;   // queries in 8-byte pieces
+  if ((fp8q ? (uintptr_t)a.q & 7 : !aligned16(a.q)) || !aligned16(a.k) || !aligned16(a.v)) return false;
   if (a.q_stride[2] != 1 || a.k_stride[3] != 1 || a.v_stride[3] != 1) return false;
   for (int i = 0; i < 2; ++i)
-    if ((a.q_stride[i] * 2) % 16) return false;
+    if (a.q_stride[i] % 8) return false;
   for (int i = 0; i < 3; ++i)
     if ((a.k_stride[i] * kvb) % 16 || (a.v_stride[i] * kvb) % 16 || a.k_stride[i] < 0 || a.v_stride[i] < 0)
       return false;
   return true;
 }
 
-template <typename T, typename KT, int D, int PACK>
+template <typename T, typename KT, int D, int PACK, bool QF8>
 GqaChoice choose(bool cap) {
   GqaChoice c;
-  c.kern = cap ? fa_decode_gqa::decode_gqa_kernel<T, D, true, KT, PACK>
-               : fa_decode_gqa::decode_gqa_kernel<T, D, false, KT, PACK>;
+  c.kern = cap ? fa_decode_gqa::decode_gqa_kernel<T, D, true, KT, PACK, QF8>
+               : fa_decode_gqa::decode_gqa_kernel<T, D, false, KT, PACK, QF8>;
   c.lds = fa_decode_gqa::gqa_lds_bytes<D, KT::id == FA_E4M3, PACK>();
   c.pack = PACK;
   return c;
@@ -60,13 +61,13 @@ bool packable(const fa_attn_args& a) {
          (fp8 || a.heads_k >= 8);
 }
 
-template <typename T, typename KT>
+template <typename T, typename KT, bool QF8 = false>
 GqaChoice choose_dim(const fa_attn_args& a, bool cap) {
-  if (a.head_dim_qk == 64) return packable(a) ? choose<T, KT, 128, 2>(cap) : choose<T, KT, 64, 1>(cap);
+  if (a.head_dim_qk == 64) return packable(a) ? choose<T, KT, 128, 2, QF8>(cap) : choose<T, KT, 64, 1, QF8>(cap);
   if constexpr (KT::id == FA_E4M3) {
-    if (packable(a)) return choose<T, KT, 256, 2>(cap);
+    if (packable(a)) return choose<T, KT, 256, 2, QF8>(cap);
   }
-  return choose<T, KT, 128, 1>(cap);
+  return choose<T, KT, 128, 1, QF8>(cap);
 }
 
 }  // namespace
@@ -80,10 +81,17 @@ GqaChoice pick_decode_gqa(const fa_attn_args& a) {
   if (a.max_seqlen_q > DECODE_GQA_MAX_ROWS) return none;
   if (a.max_seqlen_q <= 1 && a.heads_q / a.heads_k < DECODE_GQA_MIN_GROUP && !(a.head_dim_qk == 64 && packable(a)))
     return none;
-  if (a.q_dtype != FA_BF16 && a.q_dtype != FA_F16) return none;
   // P.V runs on probabilities rounded to the query's type: fp32 outputs
   // (held to fp32 accuracy) take the VALU kernel, which keeps P in fp32.
-  if (a.out_dtype != a.q_dtype) return none;
+  // E4M3 queries (P as two fp16 terms) write either 16-bit type; their
+  // multi-row calls run as prefill.
+  const bool fp8q = a.q_dtype == FA_E4M3;
+  if (fp8q) {
+    if (a.max_seqlen_q > 1 || a.k_dtype != FA_E4M3 || (a.out_dtype != FA_F16 && a.out_dtype != FA_BF16)) return none;
+  } else {
+    if (a.q_dtype != FA_BF16 && a.q_dtype != FA_F16) return none;
+    if (a.out_dtype != a.q_dtype) return none;
+  }
   if (a.k_dtype != a.v_dtype || (a.k_dtype != a.q_dtype && a.k_dtype != FA_E4M3)) return none;
   if (a.head_dim_qk != a.head_dim_v || (a.head_dim_qk != 64 && a.head_dim_qk != 128)) return none;
   if (a.alibi || a.mask_kind != 0) return none;
@@ -94,6 +102,7 @@ GqaChoice pick_decode_gqa(const fa_attn_args& a) {
   for (int i = 0; i < 2; ++i)
     if (a.k_stride[i] * kvb >= (1ll << 31) / 16 || a.v_stride[i] * kvb >= (1ll << 31) / 16) return none;
   const bool cap = a.softcap > 0.0f, fp8 = a.k_dtype == FA_E4M3;
+  if (fp8q) return choose_dim<F16T, E4M3T, true>(a, cap);
   if (a.q_dtype == FA_BF16) return fp8 ? choose_dim<BF16T, E4M3T>(a, cap) : choose_dim<BF16T, BF16T>(a, cap);
   return fp8 ? choose_dim<F16T, E4M3T>(a, cap) : choose_dim<F16T, F16T>(a, cap);
 }

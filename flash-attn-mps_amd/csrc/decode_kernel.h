@@ -426,7 +426,18 @@ __global__ __launch_bounds__(DEC_THREADS, FA_DEC_MINB) void decode_kernel(const 
       const int ep = piece_bytes(KB, j) / KT::bytes, e0 = piece_start(KB, j) / KT::bytes;
       const int d0 = 16 * e0 + ep * lq;
       uint32_t* dst = qp[g] + e0 / 2;
-      if (a.q_stride[2] == 1) {
+      if (CT::id == FA_F16 && KT::id == FA_E4M3 && a.q_dtype == FA_E4M3) {
+        // E4M3 queries (unit stride) widen exactly to fp16.
+        uint32_t w[4];
+        const char* src = (const char*)a.q + q0 + d0;
+        if (ep == 16) load_words<16>(src, w);
+        else if (ep == 8) load_words<8>(src, *(uint32_t(*)[2])w);
+        else load_words<4>(src, *(uint32_t(*)[1])w);
+        for (int i = 0; i < ep / 4; ++i) {
+          dst[2 * i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[i], 1.0f, false));
+          dst[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[i], 1.0f, true));
+        }
+      } else if (a.q_stride[2] == 1) {
         const char* src = (const char*)a.q + (q0 + d0) * 2;
         if (ep == 8) {
           uint32_t w[4];

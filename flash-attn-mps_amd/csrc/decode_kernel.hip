@@ -202,9 +202,15 @@ DecodeKernel select_decode(const fa_attn_args& a, int* gt_out) {
   if (!chunk_aligned(a.k, a.k_stride, 3, esz, (int)(tq / 16) * esz)) return nullptr;
   if (!chunk_aligned(a.v, a.v_stride, 3, esz, (int)(tv / 16) * esz)) return nullptr;
   // Q.K runs on 16-bit pairs of the query's type: 16-bit K must match it,
-  // FP8 K widens exactly to either.
-  if (a.q_dtype != FA_BF16 && a.q_dtype != FA_F16) return nullptr;
-  if (a.q_stride[2] == 1 && !chunk_aligned(a.q, a.q_stride, 2, 2, (int)(tq / 16) * 2)) return nullptr;
+  // FP8 K widens exactly to either, and FP8 queries (over FP8 K/V, 16-bit
+  // output: fp32 output keeps the generic kernel's tanhf softcap) to fp16.
+  const bool fp8q = a.q_dtype == FA_E4M3;
+  if (fp8q) {
+    if (a.out_dtype == FA_F32 || a.k_dtype != FA_E4M3 || a.q_stride[2] != 1 || !chunk_aligned(a.q, a.q_stride, 2, 1, (int)(tq / 16))) return nullptr;
+  } else {
+    if (a.q_dtype != FA_BF16 && a.q_dtype != FA_F16) return nullptr;
+    if (a.q_stride[2] == 1 && !chunk_aligned(a.q, a.q_stride, 2, 2, (int)(tq / 16) * 2)) return nullptr;
+  }
   const int pk = valu_pair(a);
   const int gt = pk == 2 ? 2 * (int)(a.heads_q / a.heads_k) : decode_group_tile(a);
   *gt_out = gt;

@@ -76,8 +76,11 @@ def uses_gqa_kernel(p, rows=None):
     small = p.dim_qk == 64 and gqa_pack(p, 1) == 2   # paired 64-dim heads take groups of 1-2 too
     rows_ok = (p.heads // p.kv_heads >= _GQA_MIN_GROUP or small) if rows <= 1 else rows <= _GQA_MAX_ROWS
     out_dtype = p.out.dtype if p.out is not None else p.output_dtype
-    return (rows_ok and p.q.dtype in (torch.float16, torch.bfloat16) and out_dtype == p.q.dtype
-            and p.k.dtype == p.v.dtype and p.k.dtype in (p.q.dtype, torch.float8_e4m3fn)
+    if p.q.dtype == torch.float8_e4m3fn:
+        types_ok = rows <= 1 and out_dtype in (torch.float16, torch.bfloat16)
+    else:
+        types_ok = p.q.dtype in (torch.float16, torch.bfloat16) and out_dtype == p.q.dtype
+    return (rows_ok and types_ok and p.k.dtype == p.v.dtype and p.k.dtype in (p.q.dtype, torch.float8_e4m3fn)
             and p.dim_qk == p.dim_v and p.dim_qk in (64, 128) and p.alibi is None and p.mask is None
             and page % 16 == 0)
 
@@ -142,7 +145,7 @@ def decode(p, out, splits=None):
     `splits` overrides the split count (1: the fixed-order route).
 
     Returns (out, lse).  The split-KV kernels handle 16-bit queries over
-    16-bit or FP8 caches at their compiled head dims; other dtype/dim/stride
+    16-bit or FP8 caches and FP8 queries over FP8 caches at their compiled head dims; other dtype/dim/stride
     combinations run fa_attn_fwd: fp32 its matrix-core kernel, the rest the
     generic kernel with the reference's split rule (_decode.py:63-64).
     """
