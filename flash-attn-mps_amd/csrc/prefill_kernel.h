@@ -351,8 +351,11 @@ FA_DEV bool compact_item(const fa_attn_args& a, int slot, int xcd, int lane, int
 // MK: vLLM mask kind (a.mask_kind; 0 none): each row's visible keys are at
 // most two key ranges (see mask_ranges below); causality and the window
 // fields do not apply, as in the reference (kernels/attention.metal:29-45).
+// SPLIT: a.num_splits workgroups (blockIdx.y) share each work item's key
+// tiles evenly and write fp32 partials for prefill_merge_kernel: for grids
+// that leave CUs idle (a chunk of a few hundred rows behind a long prefix).
 template <typename T, int DQ, int DV, int W, int NB, int MINB, bool CAUSAL, bool CAP, bool WIN, int DQT = DQ,
-          int DVT = DV, typename KT = T, bool ALIBI = false, typename QT = T, int MK = 0>
+          int DVT = DV, typename KT = T, bool ALIBI = false, typename QT = T, int MK = 0, bool SPLIT = false>
 __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_args a, const PrefillShape shp) {
   static_assert(MK == 0 || (!CAUSAL && !WIN && !ALIBI), "mask kinds carry their own causality and windows");
   constexpr bool GEN = WIN || MK != 0;   // per-stage hot / masked decisions (no closed-form hot loop)
@@ -538,6 +541,14 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
   }
   int n_tiles = kv_end > 0 ? (kv_end + PF_BN - 1) / PF_BN : 0;
   int tile0 = kv_begin / PF_BN;   // first tile with a visible key
+  const int split = SPLIT ? (int)blockIdx.y : 0;
+  if constexpr (SPLIT) {
+    static_assert(MK == 0 && !WIN, "key splits: one run of tiles per work item");
+    const int n = n_tiles;   // tile0 = 0 without windows
+    tile0 = (int)((int64_t)n * split / a.num_splits);
+    n_tiles = (int)((int64_t)n * (split + 1) / a.num_splits);
+    kv_end = min(kv_end, n_tiles * PF_BN);
+  }
 
   // Descales (per request and KV head, 1 when absent): score = scale *
   // q_descale * k_descale * q.k, output * v_descale
@@ -843,13 +854,15 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
   const float sl = ALIBI_FOLD ? slope / kscale : 0.0f;
   const float sl2 = ALIBI_LATE ? slope * LOG2E : 0.0f;
   // A sink logit seeds the running state (max = sink, sum = 1) of every row.
-  const float sink2 = a.sinks ? a.sinks[(int64_t)h * a.sink_stride] * LOG2E : -INFINITY;
+  // (with key splits, the first split's)
+  const bool seed = a.sinks && (!SPLIT || split == 0);
+  const float sink2 = seed ? a.sinks[(int64_t)h * a.sink_stride] * LOG2E : -INFINITY;
   float m_run[NB], l_run[NB];
   f32x16 o[NB][DB];
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     m_run[nb] = sink2;
-    l_run[nb] = (a.sinks && hh == 0) ? 1.0f : 0.0f;
+    l_run[nb] = (seed && hh == 0) ? 1.0f : 0.0f;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1335,6 +1348,21 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
     if (row < r.q_len) {
       const float inv = lt > 0.0f ? vdsc / lt : 0.0f;
       const int64_t tq = (int64_t)r.q_begin + row;
+      if constexpr (SPLIT) {
+        // Partials [S][T][Hq][Dv] (normalised), LSEs [S][Hq][T].
+        const int64_t dv = TWO_PARTS ? 2 * DVT : DVT;
+        float* pp = a.partial_out + ((split * a.total_q + tq) * a.heads_q + h) * dv + (TWO_PARTS ? vpart * DVT : 0) + 4 * hh;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *(float4*)(pp + 32 * db + 8 * g) = float4{o[nb][db][4 * g] * inv, o[nb][db][4 * g + 1] * inv,
+                                                      o[nb][db][4 * g + 2] * inv, o[nb][db][4 * g + 3] * inv};
+        if (hh == 0 && (!TWO_PARTS || vpart == 0))
+          a.partial_lse[((int64_t)split * a.heads_q + h) * a.total_q + tq] =
+              lt > 0.0f ? m_run[nb] * LN2 + logf(lt) : -INFINITY;
+        continue;
+      }
       uint16_t* op = (uint16_t*)a.out + tq * a.out_stride[0] + (int64_t)h * a.out_stride[1] + (TWO_PARTS ? vpart * DVT : 0) + 4 * hh;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -1543,6 +1571,49 @@ PrefillChoice pick_dims_fp8q(int64_t dq, int64_t dv, bool causal, int score, boo
     return causal ? pick_tile_fp8q<T, 256, 128, true>(score, win) : pick_tile_fp8q<T, 256, 128, false>(score, win);
   return PrefillChoice{nullptr, 0, 0, 0};
 }
+
+// Key-split variants: unpadded 64-, 128-, 192/128- and 256-dim heads (256 as
+// V halves) without windows, ALiBi or mask kinds, softcap at 64 and 128.  The
+// workgroups of a CU and the LDS are those of the unsplit tile.
+template <typename T, typename KT, typename QT, int DQ, int DV, bool CAUSAL>
+PrefillChoice pick_tile_split(bool cap) {
+  using S = PrefillTile<DQ, DV>;
+  PrefillChoice c{nullptr, 0, 0, 0, 0};
+  if constexpr (DQ <= 128) {
+    if (cap)
+      c.kern = prefill_kernel<T, DQ, DV, S::W, S::NB, S::MINB, CAUSAL, true, false, DQ, DV, KT, false, QT, 0, true>;
+  }
+  if (!cap) c.kern = prefill_kernel<T, DQ, DV, S::W, S::NB, S::MINB, CAUSAL, false, false, DQ, DV, KT, false, QT, 0, true>;
+  c.bm = 32 * S::NB * S::W;
+  c.threads = 64 * S::W;
+  if constexpr (QT::id == FA_E4M3)
+    c.lds = 2 * (size_t)((DQ + 127) / 128) * PF_GROUP_BYTES + 2 * (size_t)(DV / 64) * PF_GROUP_BYTES + 2 * 64 * (size_t)DV;
+  else
+    c.lds = lds_bytes<DQ, DV>() + (KT::id == FA_E4M3 ? 64 * (size_t)(DQ + DV) : 0);
+  c.vparts = prefill_vparts<DQ, DV>();
+  return c;
+}
+
+template <typename T, typename KT, typename QT = T>
+PrefillChoice pick_split(int64_t dq, int64_t dv, bool causal, bool cap) {
+  if (dq == 64 && dv == 64)
+    return causal ? pick_tile_split<T, KT, QT, 64, 64, true>(cap) : pick_tile_split<T, KT, QT, 64, 64, false>(cap);
+  if (dq == 128 && dv == 128)
+    return causal ? pick_tile_split<T, KT, QT, 128, 128, true>(cap) : pick_tile_split<T, KT, QT, 128, 128, false>(cap);
+  if (dq == 256 && dv == 256)
+    return causal ? pick_tile_split<T, KT, QT, 256, 128, true>(cap) : pick_tile_split<T, KT, QT, 256, 128, false>(cap);
+  if constexpr (KT::id != FA_E4M3) {
+    if (dq == 192 && dv == 128)
+      return causal ? pick_tile_split<T, KT, QT, 192, 128, true>(cap) : pick_tile_split<T, KT, QT, 192, 128, false>(cap);
+  }
+  return PrefillChoice{nullptr, 0, 0, 0, 0};
+}
+
+// Defined in prefill_inst_split_{16,fp8,fp8q}.hip; bf16: the kernel's 16-bit
+// type (the query's, or the output's with E4M3 queries).
+PrefillChoice pick_split_16(bool bf16, int64_t dq, int64_t dv, bool causal, bool cap);
+PrefillChoice pick_split_fp8(bool bf16, int64_t dq, int64_t dv, bool causal, bool cap);
+PrefillChoice pick_split_fp8q(bool bf16, int64_t dq, int64_t dv, bool causal, bool cap);
 
 // Defined in prefill_inst_{bf16,f16}_{small,large}.hip and prefill_inst_fp8q.hip.
 PrefillChoice pick_bf16_small(int64_t dq, int64_t dv, bool causal, int score, bool win, int mk);

@@ -24,12 +24,70 @@ PrefillChoice select_prefill(const fa_attn_args& a) {
   // A right window bounds nothing under causality.
   const bool win = mk == 0 && window_set(a);
   const int64_t dq = a.head_dim_qk, dv = a.head_dim_v;
+  if (a.num_splits > 1) {
+    if (a.q_dtype == FA_E4M3) return pick_split_fp8q(a.out_dtype == FA_BF16, dq, dv, causal, score == 1);
+    return (fp8 ? pick_split_fp8 : pick_split_16)(a.q_dtype == FA_BF16, dq, dv, causal, score == 1);
+  }
   if (a.q_dtype == FA_E4M3) return pick_fp8q(a.out_dtype, dq, dv, causal, score, win);
   const bool bf16 = a.q_dtype == FA_BF16;
   if (!fp8 && dq <= 128)
     return bf16 ? pick_bf16_small(dq, dv, causal, score, win, mk) : pick_f16_small(dq, dv, causal, score, win, mk);
   return bf16 ? pick_bf16_large(dq, dv, causal, score, win, fp8, mk)
               : pick_f16_large(dq, dv, causal, score, win, fp8, mk);
+}
+
+// Calls whose key tiles the kernel can split (pick_split): no windows, ALiBi
+// or mask kinds, unpadded head dims, softcap at 64 and 128 dims.
+bool split_ok(const fa_attn_args& a) {
+  if (a.mask_kind != 0 || a.alibi || window_set(a)) return false;
+  const int64_t dq = a.head_dim_qk, dv = a.head_dim_v;
+  if (dq == dv && (dq == 64 || dq == 128)) return true;
+  return !(a.softcap > 0.0f) && ((dq == 256 && dv == 256) || (dq == 192 && dv == 128));
+}
+
+// Merge of the split partials: one wave per (request, row, head) row, split
+// weights on lanes, GROUP partial rows in flight; DIMS dims per lane.  The
+// rows of single-query requests under FA_FLAG_SKIP_SINGLE_QUERY are the
+// decode kernel's and stay untouched.
+template <int DIMS, int GROUP>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const fa_attn_args a) {
+  const int lane = threadIdx.x & 63, S = a.num_splits, DV = (int)a.head_dim_v;
+  const uint32_t idx = blockIdx.x * 4 + (threadIdx.x >> 6), hq = (uint32_t)a.heads_q;
+  const int64_t b = blockIdx.y;
+  const int64_t q_begin = load_invariant_i32(a.cu_seqlens_q, b * a.cu_q_stride);
+  const int q_len = load_invariant_i32(a.cu_seqlens_q, (b + 1) * a.cu_q_stride) - (int)q_begin;
+  const int row = (int)(idx / hq);
+  const int64_t h = idx - (uint32_t)row * hq;
+  if (row >= q_len || ((a.flags & FA_FLAG_SKIP_SINGLE_QUERY) && q_len == 1)) return;
+  const int64_t tq = q_begin + row;
+  const float* const part = a.partial_out + (tq * a.heads_q + h) * DV;
+  const float* const plse = a.partial_lse + h * a.total_q + tq;
+  const int64_t pitch = a.total_q * a.heads_q * DV, lpitch = a.heads_q * a.total_q;
+  const float lse0 = lane < S ? plse[lane * lpitch] : -INFINITY;   // S <= 64
+  const float peak = wave_max(lse0), ref = peak == -INFINITY ? 0.0f : peak;
+  const float w = lane < S ? expf(lse0 - ref) : 0.0f;
+  float acc[DIMS];
+#pragma unroll
+  for (int k = 0; k < DIMS; ++k) acc[k] = 0.0f;
+  for (int s0 = 0; s0 < S; s0 += GROUP) {
+    float x[GROUP][DIMS];
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u)
+#pragma unroll
+      for (int k = 0; k < DIMS; ++k)
+        x[u][k] = s0 + u < S ? __builtin_nontemporal_load(part + (s0 + u) * pitch + lane + 64 * k) : 0.0f;
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u) {
+      const float ws = s0 + u < S ? readlane_f(w, s0 + u) : 0.0f;
+#pragma unroll
+      for (int k = 0; k < DIMS; ++k) acc[k] = ws > 0.0f ? fmaf(ws, x[u][k], acc[k]) : acc[k];
+    }
+  }
+  const float denom = wave_sum(w), inv = denom > 0.0f ? 1.0f / denom : 0.0f;
+#pragma unroll
+  for (int k = 0; k < DIMS; ++k)
+    store_any(a.out, tq * a.out_stride[0] + h * a.out_stride[1] + lane + 64 * k, a.out_dtype, acc[k] * inv);
+  if (lane == 0) a.lse[h * a.lse_stride[0] + tq * a.lse_stride[1]] = denom > 0.0f ? peak + logf(denom) : -INFINITY;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -76,7 +134,7 @@ bool prefill_ok(const fa_attn_args& a) {
   }
   const int kb = fp8 ? 1 : 2;   // K/V bytes per element
   if (a.window_left < -1 || a.window_right < -1) return false;
-  if (a.num_splits != 1) return false;
+  if (a.num_splits != 1 && (a.num_splits < 1 || a.num_splits > 64 || !split_ok(a))) return false;
   if (a.q_stride[2] != 1 || a.k_stride[3] != 1 || a.v_stride[3] != 1 || a.out_stride[2] != 1) return false;
   if (!aligned16(a.q) || !aligned16(a.k) || !aligned16(a.v) || ((uintptr_t)a.out & 7u)) return false;
   const int qb = fp8q ? 1 : 2;   // query bytes per element
@@ -150,11 +208,25 @@ extern "C" int fa_prefill_fwd(const fa_attn_args* a, void* stream) {
   // multiple of 8, as the kernel's 16-block interleave of the parts needs).
   blocks *= ch.vparts;
   FA_REQUIRE(blocks <= 0x7fffffffll, "fa_prefill_fwd: grid too large");
+  const bool split = a->num_splits > 1;
+  FA_REQUIRE(!split || (a->partial_out && a->partial_lse), "fa_prefill_fwd: splits need partial buffers");
+  FA_REQUIRE(!split || (a->batch <= 65535 && a->max_seqlen_q * a->heads_q <= 0x7fffffffll),
+             "fa_prefill_fwd: split grid too large");
   hipError_t err = hipFuncSetAttribute((const void*)ch.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ch.lds);
   if (err != hipSuccess) {
     fa_set_error("fa_prefill_fwd: cannot reserve %zu bytes of LDS: %s", ch.lds, hipGetErrorString(err));
     return FA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(ch.kern, dim3((unsigned)blocks), dim3(ch.threads), ch.lds, (hipStream_t)stream, *a, shp);
+  // Splits are the slow grid dimension and `blocks` a multiple of 8, so a
+  // work item's splits stay on its XCD.
+  hipLaunchKernelGGL(ch.kern, dim3((unsigned)blocks, (unsigned)(split ? a->num_splits : 1)), dim3(ch.threads), ch.lds,
+                     (hipStream_t)stream, *a, shp);
+  rc = fa_check_launch("fa_prefill_fwd");
+  if (rc || !split) return rc;
+  void (*merge)(const fa_attn_args) = a->head_dim_v == 64    ? prefill_merge_kernel<1, 8>
+                                      : a->head_dim_v == 128 ? prefill_merge_kernel<2, 8>
+                                                             : prefill_merge_kernel<4, 4>;
+  hipLaunchKernelGGL(merge, dim3((unsigned)fa_ceil_div(a->max_seqlen_q * a->heads_q, 4), (unsigned)a->batch), dim3(256), 0,
+                     (hipStream_t)stream, *a);
   return fa_check_launch("fa_prefill_fwd");
 }

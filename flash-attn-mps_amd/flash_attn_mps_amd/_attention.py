@@ -170,6 +170,53 @@ def f32_splits(p):
     return max(1, min(wanted, -(-p.visible_max // _F32_ROUND)))
 
 
+# The MFMA prefill's tiles by query head dim (PrefillTile in prefill_kernel.h):
+# query rows per workgroup, workgroups a compute unit holds, workgroups per
+# work item, and the time of one 64-key tile on a compute unit of its own (us).
+_PREFILL_TILE = {64: (128, 3, 1, 1.0), 128: (128, 2, 1, 1.1), 192: (128, 2, 1, 1.4), 256: (256, 1, 2, 2.2)}
+_COMPUTE_UNITS = 256
+# Below this the estimate keeps one split but for a handful of rows at d256;
+# such calls are bound by the host, where planning would cost 5 of ~27 us.
+_PREFILL_SPLIT_MIN_KEYS = 1024
+
+
+def prefill_splits(p):
+    """Key splits of an MFMA prefill call, for grids that leave at least half
+    of the GPU's workgroup slots empty (the conditions mirror split_ok in
+    prefill_mfma.hip).  The cheapest count by an estimate: the tiles of a
+    split, 1.45 / 1.9 times as long with two / three workgroups on a compute
+    unit, plus 6 us for the merge and the partials written and read back at
+    2.5 TB/s.  Measured (us, 1 split -> the chosen count, bf16, 16-token
+    pages): 512 rows behind 24000 keys, 32/8 heads d128 451 -> 211 (4), 64
+    rows 445 -> 46 (16), 2 x 256 behind 4096, 16/8 94 -> 44 (4), 512 behind
+    8192, 16/8 d256 283 -> 116 (4); where the estimate keeps one: 1 x 2048
+    causal 16/8 44 against 56 with two, 4 x 128 behind 1024 35 / 38."""
+    if p.max_k < _PREFILL_SPLIT_MIN_KEYS:
+        return 1
+    if (p.splits or p.deterministic or p.mask is not None or p.alibi is not None or torch.is_tensor(p.causal)
+            or p.window[0] >= 0 or (not p.causal and p.window[1] >= 0) or p.dim_qk not in _PREFILL_TILE):
+        return 1
+    if p.dim_v != (128 if p.dim_qk == 192 else p.dim_qk) or (p.softcap > 0 and p.dim_qk > 128):
+        return 1
+    rows, per_cu, parts, tile_us = _PREFILL_TILE[p.dim_qk]
+    pair = 2 if p.heads // p.kv_heads % 2 == 0 else 1   # heads per workgroup
+    requests = p.batch if p.tokens >= 2 * p.batch else 1
+    blocks = requests * -(-p.tokens // (requests * (rows // pair))) * (p.heads // pair) * parts
+    most = min(per_cu * _COMPUTE_UNITS // blocks, 16)
+    if most < 2 or p.batch > 65535:
+        return 1
+    keys_us = p.max_k / 64 * tile_us
+    partial_us = p.tokens * p.heads * p.dim_v * 8 / 2.5e6
+    best, best_us = 1, keys_us
+    for n in (2, 3, 4, 6, 8, 12, 16):
+        if n > most:
+            break
+        us = keys_us / n * (0.55 + 0.45 * -(-blocks * n // _COMPUTE_UNITS)) + 6 + n * partial_us
+        if us < best_us:
+            best, best_us = n, us
+    return best
+
+
 _SIDE = {}
 
 # Below this many K/V bytes (an upper bound of what the decode pass of a
@@ -289,6 +336,10 @@ def solve(p):
         # follows the batch).
         self_attention = p.cu_k is p.cu_q and p.used_k is None and not p.paged
         mixed = p.batch > 1 and not self_attention and (not p.deterministic or p.paged)
+        splits = prefill_splits(p)
+        if splits > 1:
+            _partials(p, a, (splits, p.tokens, p.heads, p.dim_v), (splits, p.heads, p.tokens))
+            a.num_splits = splits
         if not (mixed and _mixed_batch(p, a, fixed_order=p.deterministic)):
             _lib.call("fa_prefill_fwd", a, p.device)
         return out, lse
