@@ -373,6 +373,90 @@ __global__ __launch_bounds__(256) void rotary_kernel(const RotaryParams p) {
   }
 }
 
+// -------------------------------------------- rotary embedding and append
+
+// One wave per (token, head) row of q, then of k, then of v: a lane rotates
+// whole pairs, so each element is read once, and the row's position, table
+// row and cache row are found once per wave.  A step of one token is a
+// handful of waves, bound by the round trip lengths -> cos/sin -> store; as
+// separate launches (two rotations, the append, the lengths' update and the
+// two table conversions, 2-3.5 us each and as much again to launch) they were
+// most of a small decode call.
+template <typename XT, bool FP8>
+__global__ __launch_bounds__(256) void step_kernel(const fa_step_args p, const uint32_t q_rows, const uint32_t k_rows) {
+  using S = typename XT::storage;
+  const fa_append_args& c = p.kv;
+  if (blockIdx.x == 0 && p.lengths_out)
+    for (int64_t b = threadIdx.x; b < c.batch; b += 256)
+      p.lengths_out[b] = c.lengths[b] + (int32_t)c.new_tokens - (p.leftpad ? p.leftpad[b * p.leftpad_stride] : 0);
+  const int lane = threadIdx.x & 63;
+  uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int part = w < q_rows ? 0 : w < q_rows + k_rows ? 1 : 2;   // q, k, v
+  if (part == 2 && w >= q_rows + 2 * k_rows) return;
+  w -= part == 0 ? 0 : part == 1 ? q_rows : q_rows + k_rows;
+  const fa_store_desc& d = c.kv[part == 2 ? 1 : 0];
+  const uint32_t heads = (uint32_t)(part == 0 ? p.q_heads : d.heads), seq = (uint32_t)(part == 0 ? p.q_seq : c.new_tokens);
+  const uint32_t bj = w / heads, h = w - bj * heads, b = bj / seq, j = bj - b * seq;
+  const int dim = (int)(part == 0 ? p.q_dim : d.dim);
+  const int64_t pos = (int64_t)c.lengths[b] + (part == 0 && !p.q_advance ? 0 : j);
+  const S* src;
+  int64_t xs;
+  char* dst;
+  int64_t ds = 1;
+  float scale = 1.0f;
+  if (part == 0) {
+    src = (const S*)p.q + b * p.q_stride[0] + j * p.q_stride[1] + h * p.q_stride[2];
+    xs = p.q_stride[3];
+    dst = (char*)((S*)p.q_out + (int64_t)w * dim);
+  } else {
+    src = (const S*)d.x + b * c.x_batch_stride[part - 1] + j * d.x_stride[0] + h * d.x_stride[1];
+    xs = d.x_stride[2];
+    const bool paged = c.block_table != nullptr;
+    const int64_t row = (!paged && c.batch_index) ? (int64_t)c.batch_index[b] : (int64_t)b;
+    const int64_t rows = paged ? c.table_rows : c.num_blocks, limit = paged ? c.table_cols * c.page_size : c.page_size;
+    if (row < 0 || row >= rows || pos < 0 || pos >= limit) return;
+    const int64_t page = paged ? pos / c.page_size : 0;
+    const int64_t block = paged ? (int64_t)c.block_table[row * c.table_cols + page] : row;
+    if (block < 0 || block >= c.num_blocks) return;
+    const int64_t at = block * d.cache_stride[0] + (pos - page * c.page_size) * d.cache_stride[1] + h * d.cache_stride[2];
+    dst = (char*)d.cache + at * (FP8 ? 1 : (int64_t)sizeof(S));
+    ds = d.cache_stride[3];
+    if (FP8) scale = d.scale[h * d.scale_stride];
+  }
+  auto encode = [&](int e, float v) { ((uint8_t*)dst)[e * ds] = f32_to_e4m3(v / scale); };
+  // A rotated value rounds to the input type first, as a separate rotation's
+  // output would.
+  auto put = [&](int e, float v) {
+    if (FP8 && part != 0) {
+      S r;
+      store_elem<XT>(&r, 0, v);
+      encode(e, load_elem<XT>(&r, 0));
+    } else {
+      store_elem<XT>(dst, e * ds, v);
+    }
+  };
+  const int half = p.cos_table && part != 2 ? (int)p.half_rot : 0;
+  // A position without a cos/sin row rotates to NaN, as in rotary_kernel.
+  const bool in_table = pos >= 0 && pos < p.table_rows;
+  for (int i = lane; i < half; i += 64) {
+    const int e0 = p.interleaved ? 2 * i : i, e1 = p.interleaved ? 2 * i + 1 : i + half;
+    float r0 = __builtin_nanf(""), r1 = __builtin_nanf("");
+    if (in_table) {
+      const float cs = load_any(p.cos_table, pos * p.cos_stride[0] + i * p.cos_stride[1], p.trig_dtype);
+      const float sn = load_any(p.sin_table, pos * p.sin_stride[0] + i * p.sin_stride[1], p.trig_dtype);
+      const float x = load_elem<XT>(src, e0 * xs), y = load_elem<XT>(src, e1 * xs);
+      r0 = fmaf(x, cs, -(y * sn));   // rotary_kernel's rounding, bit for bit
+      r1 = fmaf(y, cs, x * sn);
+    }
+    put(e0, r0);
+    put(e1, r1);
+  }
+  for (int e = 2 * half + lane; e < dim; e += 64) {
+    if (FP8 && part != 0) encode(e, load_elem<XT>(src, e * xs));
+    else ((S*)dst)[e * ds] = src[e * xs];
+  }
+}
+
 StoreDescK to_desc(const fa_store_desc& s, int64_t vec) {
   StoreDescK d;
   d.x = s.x;
@@ -526,4 +610,41 @@ extern "C" int fa_rotary(const fa_rotary_args* a, void* stream) {
     default: hipLaunchKernelGGL((rotary_kernel<F32T>), dim3((unsigned)blocks), dim3(256), 0, s, p); break;
   }
   return fa_check_launch("fa_rotary");
+}
+
+extern "C" int fa_rotary_append(const fa_step_args* a, void* stream) {
+  FA_REQUIRE(a && a->size == (int64_t)sizeof(fa_step_args), "fa_rotary_append: null or mismatched arguments");
+  const fa_append_args& c = a->kv;
+  FA_REQUIRE(c.lengths != nullptr, "fa_rotary_append: null lengths");
+  const int xdt = c.kv[0].x_dtype, cdt = c.kv[0].cache_dtype;
+  for (int i = 0; i < 2; ++i) {
+    const fa_store_desc& s = c.kv[i];
+    FA_REQUIRE(s.x && s.cache, "fa_rotary_append: null tensor %d", i);
+    FA_REQUIRE(s.x_dtype == xdt && s.cache_dtype == cdt, "fa_rotary_append: K and V must share dtypes");
+    FA_REQUIRE(s.heads == c.kv[0].heads && s.heads > 0 && s.dim > 0, "fa_rotary_append: bad head counts or dims");
+    FA_REQUIRE(cdt == xdt || (cdt == FA_E4M3 && s.scale), "fa_rotary_append: cache dtype must match input, or E4M3 with a scale");
+  }
+  FA_REQUIRE(xdt == FA_F16 || xdt == FA_BF16 || xdt == FA_F32, "fa_rotary_append: input dtype must be f16/bf16/f32");
+  FA_REQUIRE(c.batch >= 0 && c.new_tokens >= 1 && c.page_size > 0, "fa_rotary_append: bad sizes");
+  FA_REQUIRE(c.block_table == nullptr || c.table_cols > 0, "fa_rotary_append: empty block table");
+  FA_REQUIRE(!a->cos_table == !a->sin_table && !a->q == !a->q_out, "fa_rotary_append: cos/sin and q/q_out come together");
+  if (a->cos_table) {
+    FA_REQUIRE(a->trig_dtype == FA_F16 || a->trig_dtype == FA_BF16 || a->trig_dtype == FA_F32,
+               "fa_rotary_append: cos/sin dtype must be f16/bf16/f32");
+    FA_REQUIRE(2 * a->half_rot <= c.kv[0].dim && (!a->q || 2 * a->half_rot <= a->q_dim),
+               "fa_rotary_append: rotary dim exceeds head dim");
+  }
+  FA_REQUIRE(!a->q || (a->q_seq >= 0 && a->q_heads >= 1 && a->q_dim >= 1), "fa_rotary_append: bad query shape");
+  const int64_t qr = a->q ? c.batch * a->q_seq * a->q_heads : 0, kr = c.batch * c.new_tokens * c.kv[0].heads;
+  if (c.batch == 0) return FA_OK;
+  FA_REQUIRE(qr + 2 * kr <= 0x7fffffffll, "fa_rotary_append: too many rows");
+  const dim3 grid((unsigned)fa_ceil_div(qr + 2 * kr, 4));
+  hipStream_t s = (hipStream_t)stream;
+  const bool fp8 = cdt == FA_E4M3;
+  void (*kern)(const fa_step_args, const uint32_t, const uint32_t) =
+      xdt == FA_F16    ? (fp8 ? step_kernel<F16T, true> : step_kernel<F16T, false>)
+      : xdt == FA_BF16 ? (fp8 ? step_kernel<BF16T, true> : step_kernel<BF16T, false>)
+                       : (fp8 ? step_kernel<F32T, true> : step_kernel<F32T, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, *a, (uint32_t)qr, (uint32_t)kr);
+  return fa_check_launch("fa_rotary_append");
 }

@@ -6,10 +6,13 @@ flash_attn_mps/_cache.py:55-155).
   row = slot % P); negative or out-of-range slots are skipped by the kernel.
 * append_kvcache writes new rows at ``lengths[b] + j`` of a dense cache row
   or through a page table; the lengths themselves are not touched.
+* rotary_append is a generation step's rotary embedding and append in one
+  launch.
 * An FP8 (E4M3FN) cache stores E4M3(x / scale) with scale a scalar or one
   value per KV head; 16-bit and fp32 caches of the input's dtype get the
   input's bits.
 """
+import ctypes
 from functools import lru_cache
 
 import torch
@@ -114,6 +117,16 @@ def append_kvcache(k, v, k_cache, v_cache, cache_seqlens, *, cache_batch_idx=Non
     the table.  cache_leftpad does not move the write: FA2 lengths already
     count the padding (flash_attn_mps/_cache.py:99-127).
     """
+    keep = []
+    args = _append_args(k, v, k_cache, v_cache, cache_seqlens, cache_batch_idx, cache_leftpad, block_table, k_scale,
+                        v_scale, keep)
+    if args is not None:
+        _lib.call("fa_append_kvcache", args, k.device)
+
+
+def _append_args(k, v, k_cache, v_cache, cache_seqlens, cache_batch_idx, cache_leftpad, block_table, k_scale, v_scale,
+                 keep):
+    """The checked fa_append_args of an append (None: nothing to write)."""
     _require_gpu(k=k, v=v, k_cache=k_cache, v_cache=v_cache, block_table=block_table)
     if k.ndim != 4 or v.ndim != 4 or k.shape[:3] != v.shape[:3]:
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} must be [batch, new_tokens, heads, dim] "
@@ -132,8 +145,8 @@ def append_kvcache(k, v, k_cache, v_cache, cache_seqlens, *, cache_batch_idx=Non
     _check_cache_shape(v, v_cache, 2)
     writes = [(x, c, s) for x, c, s in ((k, k_cache, k_scale), (v, v_cache, v_scale)) if x.numel()]
     if not writes:
-        return
-    keep = [lengths, rows, table]
+        return None
+    keep += [lengths, rows, table]
     args = _lib.AppendArgs()
     for i, (x, c, s) in enumerate(writes):
         args.kv[i] = _write_desc(x, c, s, x.stride()[1:], keep)
@@ -144,7 +157,68 @@ def append_kvcache(k, v, k_cache, v_cache, cache_seqlens, *, cache_batch_idx=Non
     args.batch, args.new_tokens = batch, k.shape[1]
     args.page_size, args.num_blocks = k_cache.shape[1], k_cache.shape[0]
     args.table_rows, args.table_cols = (0, 0) if table is None else tuple(table.shape)
-    _lib.call("fa_append_kvcache", args, k.device)
+    return args
+
+
+def rotary_append(q, k, v, k_cache, v_cache, lengths, cos, sin, *, cache_batch_idx=None, cache_leftpad=None,
+                  block_table=None, rotary_interleaved=True, causal=False, window_size=(-1, -1)):
+    """rotary() of q and k (cos / sin None: neither) and append_kvcache() of
+    (k, v), in one launch where q, k and v share a type and nothing is empty.
+
+    Returns (q rotated, the lengths after the append less cache_leftpad)."""
+    one_launch = (q.dtype == k.dtype == v.dtype and q.dtype in _INPUT_TYPES and q.ndim == 4 and k.ndim == 4
+                  and q.numel() and k.numel() and v.numel() and lengths.numel() == k.shape[0]
+                  and (cos is None or (cos.numel() and cos.dtype in _INPUT_TYPES and sin.dtype == cos.dtype
+                                       and cos.device == sin.device == q.device))
+                  and (cache_leftpad is None or (cache_leftpad.dtype == torch.int32 and cache_leftpad.ndim == 1
+                                                 and cache_leftpad.device == q.device)))
+    if not one_launch:
+        if cos is not None:
+            q, k = rotary(q, k, cos, sin, lengths, rotary_interleaved=rotary_interleaved, causal=causal,
+                          window_size=window_size)
+        append_kvcache(k, v, k_cache, v_cache, lengths, cache_batch_idx=cache_batch_idx, cache_leftpad=cache_leftpad,
+                       block_table=block_table)
+        lengths = lengths + k.shape[1]
+        return q, lengths if cache_leftpad is None else lengths - cache_leftpad
+    if cos is not None:
+        _check_rotary(q, k, cos, sin)
+    keep = []
+    append = _append_args(k, v, k_cache, v_cache, lengths, cache_batch_idx, cache_leftpad, block_table, None, None, keep)
+    a = _lib.StepArgs()
+    a.size, a.kv = ctypes.sizeof(_lib.StepArgs), append
+    after = torch.empty(k.shape[0], dtype=torch.int32, device=k.device)
+    a.lengths_out = after.data_ptr()
+    if cache_leftpad is not None:
+        a.leftpad, a.leftpad_stride = cache_leftpad.data_ptr(), cache_leftpad.stride(0)
+    if cos is not None:
+        rotated = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        a.q, a.q_out = q.data_ptr(), rotated.data_ptr()
+        a.q_seq, a.q_heads, a.q_dim = q.shape[1:]
+        a.q_stride[:] = q.stride()
+        a.cos_table, a.sin_table, a.trig_dtype = cos.data_ptr(), sin.data_ptr(), _lib.DTYPE_CODE[cos.dtype]
+        a.cos_stride[:], a.sin_stride[:] = cos.stride(), sin.stride()
+        a.half_rot, a.table_rows = cos.shape[1], cos.shape[0]
+        a.interleaved = int(bool(rotary_interleaved))
+        a.q_advance = int(bool(causal) or tuple(window_size) != (-1, -1))
+        q = rotated
+    _lib.call("fa_rotary_append", a, k.device)
+    return q, after
+
+
+def _check_rotary(q, k, cos, sin):
+    _require_gpu(q=q, k=k, cos=cos, sin=sin)
+    if q.ndim != 4 or (k is not None and (k.ndim != 4 or k.shape[0] != q.shape[0])):
+        raise ValueError("q and k must be [batch, tokens, heads, dim] with one batch")
+    if cos.ndim != 2 or sin.shape != cos.shape or 2 * cos.shape[1] > q.shape[-1]:
+        raise ValueError(f"cos/sin must be [positions, rotary_dim / 2] with rotary_dim <= {q.shape[-1]}; "
+                         f"got {tuple(cos.shape)} / {tuple(sin.shape)}")
+    for x in (q, k):
+        if x is None:
+            continue
+        if x.dtype not in _INPUT_TYPES:
+            raise TypeError(f"rotary embedding takes float16, bfloat16 or float32; got {x.dtype}")
+        if 2 * cos.shape[1] > x.shape[-1]:
+            raise ValueError(f"rotary_dim {2 * cos.shape[1]} exceeds the head dim {x.shape[-1]}")
 
 
 def rotary(q, k, cos, sin, cache_seqlens, *, rotary_interleaved=True, causal=False, window_size=(-1, -1)):
@@ -156,12 +230,7 @@ def rotary(q, k, cos, sin, cache_seqlens, *, rotary_interleaved=True, causal=Fal
     or local attention, else all sit at cache_seqlens[b]
     (flash_attn_mps/_cache.py:130-155).  A position past the table rotates to NaN.
     """
-    _require_gpu(q=q, k=k, cos=cos, sin=sin)
-    if q.ndim != 4 or (k is not None and (k.ndim != 4 or k.shape[0] != q.shape[0])):
-        raise ValueError("q and k must be [batch, tokens, heads, dim] with one batch")
-    if cos.ndim != 2 or sin.shape != cos.shape or 2 * cos.shape[1] > q.shape[-1]:
-        raise ValueError(f"cos/sin must be [positions, rotary_dim / 2] with rotary_dim <= {q.shape[-1]}; "
-                         f"got {tuple(cos.shape)} / {tuple(sin.shape)}")
+    _check_rotary(q, k, cos, sin)
     cos32, sin32 = cos.float().contiguous(), sin.float().contiguous()
     lengths = _per_request(cache_seqlens, q.shape[0], q.device, "cache_seqlens")
     query_moves = bool(causal) or tuple(window_size) != (-1, -1)
@@ -170,10 +239,6 @@ def rotary(q, k, cos, sin, cache_seqlens, *, rotary_interleaved=True, causal=Fal
         if x is None:
             rotated.append(None)
             continue
-        if x.dtype not in _INPUT_TYPES:
-            raise TypeError(f"rotary embedding takes float16, bfloat16 or float32; got {x.dtype}")
-        if 2 * cos.shape[1] > x.shape[-1]:
-            raise ValueError(f"rotary_dim {2 * cos.shape[1]} exceeds the head dim {x.shape[-1]}")
         y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         if x.numel():
             a = _lib.RotaryArgs()

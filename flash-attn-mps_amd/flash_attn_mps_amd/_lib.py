@@ -56,6 +56,14 @@ class RotaryArgs(ctypes.Structure):
                 ("half_rot", _i64), ("table_rows", _i64), ("x_stride", _arr(_i64, 4))]
 
 
+class StepArgs(ctypes.Structure):
+    _fields_ = [("size", _i64), ("kv", AppendArgs), ("q", _p), ("q_out", _p), ("cos_table", _p), ("sin_table", _p),
+                ("trig_dtype", _i32), ("interleaved", _i32), ("q_advance", _i32), ("_pad0", _i32),
+                ("q_seq", _i64), ("q_heads", _i64), ("q_dim", _i64), ("half_rot", _i64), ("table_rows", _i64),
+                ("q_stride", _arr(_i64, 4)), ("cos_stride", _arr(_i64, 2)), ("sin_stride", _arr(_i64, 2)),
+                ("leftpad", _p), ("leftpad_stride", _i64), ("lengths_out", _p)]
+
+
 class AttnArgs(ctypes.Structure):
     _fields_ = [("q", _p), ("k", _p), ("v", _p), ("out", _p), ("lse", _p),
                 ("q_dtype", _i32), ("k_dtype", _i32), ("v_dtype", _i32), ("out_dtype", _i32),
@@ -113,6 +121,7 @@ ENTRY_POINTS = {
     "fa_store_kvcache": (StoreArgs, ctypes.c_int),
     "fa_append_kvcache": (AppendArgs, ctypes.c_int),
     "fa_rotary": (RotaryArgs, ctypes.c_int),
+    "fa_rotary_append": (StepArgs, ctypes.c_int),
     "fa_decode_supported": (AttnArgs, ctypes.c_int),
     "fa_decode_fwd": (AttnArgs, ctypes.c_int),
     "fa_decode_fwd_noalloc": (AttnArgs, ctypes.c_int),

@@ -21,24 +21,30 @@ from ._problem import MaskSpec, Problem, reject_training  # noqa: F401  (MaskSpe
 PAGE_MULTIPLE = 16   # paged caches: page sizes the FlashAttention contract accepts
 
 
-class _UniformOffsets:
-    """int32 offsets 0, L, 2L, ..., B*L on a device, made once per (device, B, L).
+class _Resident:
+    """Small int32 index tensors of (batch, length) on a device, made once per
+    (device, batch, length) by `make`.
 
     Dense layers of one model reuse a handful of shapes, so a small LRU keeps
-    their offsets resident and a call adds no host-to-device copy (which also
-    keeps dense calls capturable in HIP graphs).  Entries are never written
-    after creation.
+    the tensors resident and a call adds no kernel.  Entries are copied from
+    the host, complete when the call that makes them returns (so any stream
+    may read them), and never written again.  While a graph is being captured
+    a missing entry is made by a captured kernel and not kept: its memory
+    belongs to the graph.
     """
 
-    def __init__(self, capacity=64):
+    def __init__(self, make, capacity=64):
+        self._make = make
         self._entries = OrderedDict()
         self._capacity = capacity
 
     def __call__(self, batch, length, device):
-        key = (str(device), batch, length)
+        key = (device.type, device.index, batch, length)
         hit = self._entries.get(key)
         if hit is None:
-            hit = torch.arange(batch + 1, dtype=torch.int32, device=device) * length
+            if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+                return self._make(batch, length, device)
+            hit = self._make(batch, length, "cpu").to(device)
             self._entries[key] = hit
             if len(self._entries) > self._capacity:
                 self._entries.popitem(last=False)
@@ -47,7 +53,10 @@ class _UniformOffsets:
         return hit
 
 
-_offsets = _UniformOffsets()
+# Offsets 0, L, 2 L, ..., B L of a dense batch, and the identity table [B, 1]
+# of a dense cache (request b reads row b).
+_offsets = _Resident(lambda b, n, device: torch.arange(b + 1, dtype=torch.int32, device=device) * n)
+_rows = _Resident(lambda b, n, device: torch.arange(b, dtype=torch.int32, device=device).reshape(b, n))
 
 
 def _check_page_size(k):
@@ -197,24 +206,22 @@ def flash_attn_with_kvcache(
     if rotary_cos is not None:
         if k is None:
             raise ValueError("a rotary embedding is applied to new k/v only; none were given")
-        from ._cache import rotary
-        q, k = rotary(q, k, rotary_cos, rotary_sin, lengths, rotary_interleaved=rotary_interleaved,
-                      causal=causal, window_size=window_size)
     if k is not None:
         if k.ndim != 4 or v.ndim != 4 or k.shape[0] != batch or v.shape[:3] != k.shape[:3]:
             raise ValueError(f"new k {tuple(k.shape)} / v {tuple(v.shape)} must be [{batch}, Snew, Hkv, D]")
-        from ._cache import append_kvcache
-        append_kvcache(k, v, k_cache, v_cache, lengths, cache_batch_idx=cache_batch_idx,
-                       cache_leftpad=cache_leftpad, block_table=block_table)
-        lengths = lengths + k.shape[1]
+        from ._cache import rotary_append
+        q, lengths = rotary_append(q, k, v, k_cache, v_cache, lengths, rotary_cos, rotary_sin,
+                                   cache_batch_idx=cache_batch_idx, cache_leftpad=cache_leftpad, block_table=block_table,
+                                   rotary_interleaved=rotary_interleaved, causal=causal, window_size=window_size)
+    elif cache_leftpad is not None:
+        lengths = lengths - cache_leftpad
     if block_table is not None:
         # Table rows follow the query batch; cache_batch_idx only remaps dense rows.
         table, max_k = block_table, block_table.shape[1] * k_cache.shape[1]
+    elif cache_batch_idx is not None:
+        table, max_k = cache_batch_idx.to(torch.int32).reshape(batch, 1), k_cache.shape[1]
     else:
-        rows = cache_batch_idx if cache_batch_idx is not None else torch.arange(batch, device=q.device)
-        table, max_k = rows.to(torch.int32).reshape(batch, 1), k_cache.shape[1]
-    if cache_leftpad is not None:
-        lengths = lengths - cache_leftpad
+        table, max_k = _rows(batch, 1, q.device), k_cache.shape[1]
     problem = Problem(q.flatten(0, 1), k_cache, v_cache, _offsets(batch, sq, q.device), sq, max_k,
                       used_k=lengths, table=table, leftpad=cache_leftpad, scale=softmax_scale,
                       causal=causal, window=tuple(window_size), softcap=softcap, alibi=alibi_slopes,

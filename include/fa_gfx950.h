@@ -119,6 +119,26 @@ typedef struct fa_rotary_args {
   int64_t x_stride[4];
 } fa_rotary_args;
 
+/* One generation step's work before attention, in one launch: rotary
+ * embedding of the queries into q_out and of the new keys on their way into
+ * the cache, the append of K and V, and the lengths after it.  Same results
+ * as fa_rotary on q and k followed by fa_append_kvcache (keys round to their
+ * own type between the two).  q, k and v share one dtype. */
+typedef struct fa_step_args {
+  int64_t size;                /* sizeof(fa_step_args) */
+  fa_append_args kv;           /* kv.kv[0] / [1]: K / V, both present; kv[0].x not yet rotated */
+  const void* q; void* q_out;  /* [batch, q_seq, q_heads, q_dim] -> contiguous; NULL without rotary */
+  const void* cos_table; const void* sin_table;   /* [table_rows, half_rot] of trig_dtype; NULL: no rotary */
+  int32_t trig_dtype;          /* FA_F16 / FA_BF16 / FA_F32 */
+  int32_t interleaved;
+  int32_t q_advance;           /* query j sits at lengths[b] + j (else all at lengths[b]) */
+  int32_t _pad0;
+  int64_t q_seq, q_heads, q_dim, half_rot, table_rows;
+  int64_t q_stride[4], cos_stride[2], sin_stride[2];
+  const int32_t* leftpad; int64_t leftpad_stride;   /* [batch], or NULL */
+  int32_t* lengths_out;        /* [batch]: lengths + new_tokens - leftpad; NULL: not written */
+} fa_step_args;
+
 /* ------------------------------------------------------------- attention */
 
 /* Attention over packed [T, Hkv, D] or paged [pages, P, Hkv, D] K/V.  Output
@@ -209,6 +229,7 @@ const char* fa_last_error(void);
 int fa_store_kvcache(const fa_store_args* args, void* stream);
 int fa_append_kvcache(const fa_append_args* args, void* stream);
 int fa_rotary(const fa_rotary_args* args, void* stream);
+int fa_rotary_append(const fa_step_args* args, void* stream);
 
 /* Split-KV decode.  With max_seqlen_q <= 1: one query row per request (rows
  * with cu_seqlens_q difference 1; others are skipped).  With max_seqlen_q = R

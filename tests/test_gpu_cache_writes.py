@@ -11,7 +11,7 @@ import torch
 
 import flash_attn_mps_amd as fa
 from flash_attn_mps_amd._cache import append_kvcache, rotary, store_kvcache
-from harness import decode_attention, max_err
+from harness import decode_attention, max_err, seeded
 from oracle import cache as ocache
 from oracle import fp8 as ofp8
 
@@ -236,3 +236,49 @@ def test_decode_kernel_widens_every_fp8_code_exactly(device):
                      block_table=torch.arange(n, device=device, dtype=torch.int32).reshape(n, 1), out=out)
     expected = torch.from_numpy(ofp8.decode(codes.numpy()))
     assert torch.equal(out.cpu()[:, 0, 0], expected) and torch.equal(out.cpu()[:, 0, 63], expected)
+
+
+@pytest.mark.parametrize("dtype,cache_dtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+                                               (torch.float32, torch.float32), (torch.bfloat16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("interleaved", [True, False])
+@pytest.mark.parametrize("new,dim,rot", [(1, 128, 128), (3, 72, 40), (2, 300, 2), (5, 64, None)])
+@pytest.mark.parametrize("layout", ["dense", "remapped", "paged"])
+def test_rotary_append_equals_its_parts(device, dtype, cache_dtype, interleaved, new, dim, rot, layout):
+    """One launch against rotary() + append_kvcache(), bit for bit: partial
+    and absent rotation (rot None), strided q/k/v and tables, positions past
+    the cos/sin table (NaN) and past the cache (not written), rows out of
+    range, left padding, advancing and fixed queries."""
+    from flash_attn_mps_amd._cache import rotary_append
+    b, sq, hq, hk, page = 4, 2, 6, 2, 16
+    q = seeded((b, sq, hq, 2 * dim), 60, dtype, device)[..., ::2]
+    k = seeded((b, new + 1, hk, dim), 61, dtype, device)[:, 1:]
+    v = seeded((b, new, hk, dim + 8), 62, dtype, device)[..., :dim]
+    lengths = torch.tensor([0, 15, 37, 62], dtype=torch.int32, device=device)   # capacity 64, table of 60 positions
+    cos = sin = None
+    if rot is not None:
+        angles = seeded((60, rot), 63, torch.float32, device)
+        cos, sin = angles.cos().to(dtype)[:, ::2], angles.sin().to(dtype)[:, ::2]
+    kw = dict(cache_leftpad=torch.tensor([0, 1, 2, 3], dtype=torch.int32, device=device))
+    if layout == "paged":
+        table = torch.randperm(16, generator=torch.Generator().manual_seed(1)).reshape(4, 4).int()
+        table[1, 1] = 99
+        kw.update(block_table=table.to(device), cache_leftpad=None)
+        shape = (16, page, hk, dim)
+    else:
+        shape = (5, 64, hk, dim)
+        if layout == "remapped":
+            kw.update(cache_batch_idx=torch.tensor([4, 0, 7, 1], dtype=torch.int32, device=device))
+    caches = [[torch.full(shape, 3.0, device=device).to(cache_dtype) for _ in range(2)] for _ in range(2)]
+    for causal in (True, False):
+        got_q, after = rotary_append(q, k, v, *caches[0], lengths, cos, sin, rotary_interleaved=interleaved,
+                                     causal=causal, **kw)
+        want_q, want_k = q, k
+        if cos is not None:
+            want_q, want_k = rotary(q, k, cos, sin, lengths, rotary_interleaved=interleaved, causal=causal)
+        append_kvcache(want_k, v, *caches[1], lengths, **kw)
+        bits = torch.uint8
+        assert torch.equal(got_q.contiguous().view(bits), want_q.contiguous().view(bits))
+        for got, want in zip(*caches):
+            assert torch.equal(got.view(bits), want.view(bits))
+        pad = kw["cache_leftpad"]
+        assert torch.equal(after, lengths + new - (0 if pad is None else pad))
