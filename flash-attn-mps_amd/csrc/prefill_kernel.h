@@ -1512,6 +1512,8 @@ PrefillChoice pick_dims_small(int64_t dq, int64_t dv, bool causal, int score, bo
 // vLLM mm_prefix +36%, rswa +8%, softcap 50 560 -> 519, softcap + window
 // 346 -> 257; E4M3 K/V causal 299 -> 564, non-causal 342 -> 657, softcap
 // 339 -> 444, window 221 -> 255, softcap + window 285 -> 228.
+// (16-bit K/V without ALiBi and mask kinds take the wave pairs of
+// prefill_pair.h before they come here.)
 template <typename T, typename KT>
 PrefillChoice pick_256(bool causal, int score, bool win, int mk) {
   const bool cap = score == 1 || score == 3;
