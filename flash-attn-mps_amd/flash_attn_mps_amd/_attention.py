@@ -28,6 +28,8 @@ kernel variant depends only on dtypes, head dims and feature flags, and a
 key tile that a row cannot see adds exact zeros to its sums.  So a request's
 rows are bit-identical whatever else is in the batch.
 """
+import math
+
 import torch
 
 from . import _lib
@@ -43,75 +45,70 @@ def _as(t, dtype, keep):
     return t
 
 
+def _int32(x):
+    """x wrapped to 32 bits, as a C assignment does (a window of sys.maxsize is unbounded)."""
+    x = int(x)
+    return x if -1 <= x < 1 << 31 else (x + (1 << 31)) % (1 << 32) - (1 << 31)
+
+
+def _float32(x):
+    """x in fp32 range (larger magnitudes become infinite)."""
+    x = float(x)
+    return math.copysign(math.inf, x) if abs(x) > 3.4028235e38 else x
+
+
 def build_args(p, out, lse, max_q=None):
     """The fa_attn_args struct of problem `p` writing `out` / `lse`."""
     keep = p.keep
-    a = _lib.AttnArgs()
-    a.q, a.k, a.v = p.q.data_ptr(), p.k.data_ptr(), p.v.data_ptr()
-    a.out, a.lse = out.data_ptr(), lse.data_ptr()
-    a.q_dtype, a.k_dtype, a.v_dtype = (_lib.DTYPE_CODE[t.dtype] for t in (p.q, p.k, p.v))
-    a.out_dtype = _lib.DTYPE_CODE[out.dtype]
-    a.total_q, a.heads_q, a.head_dim_qk = p.q.shape
-    a.heads_k, a.head_dim_v = p.kv_heads, p.dim_v
-    a.batch = p.batch
-    a.page_size = p.k.shape[1] if p.paged else 0
-    a.max_seqlen_q = p.max_q if max_q is None else max_q
-    a.max_seqlen_k = p.max_k
-    a.q_stride[:] = p.q.stride()
-    a.k_stride[:] = p.k.stride() if p.paged else (0, *p.k.stride())
-    a.v_stride[:] = p.v.stride() if p.paged else (0, *p.v.stride())
-    a.out_stride[:] = out.stride()
-    a.lse_stride[:] = lse.stride()
-    i32 = torch.int32
-    cu_q = _as(p.cu_q, i32, keep)
-    a.cu_seqlens_q, a.cu_q_stride = cu_q.data_ptr(), cu_q.stride(0)
-    for tensor, ptr_field, stride_field in ((p.cu_k, "cu_seqlens_k", "cu_k_stride"),
-                                            (p.used_k, "seqused_k", "used_k_stride"),
-                                            (p.leftpad, "leftpad_k", "leftpad_stride")):
-        t = _as(tensor, i32, keep)
-        if t is not None:
-            setattr(a, ptr_field, t.data_ptr())
-            setattr(a, stride_field, t.stride(0))
-    table = _as(p.table, i32, keep)
-    if table is not None:
-        a.block_table = table.data_ptr()
-        a.bt_stride[:] = table.stride()
+    q, k, v = p.q, p.k, p.v
+    code = _lib.DTYPE_CODE
+    i32, f32 = torch.int32, torch.float32
+    q_shape, k_shape = q.shape, k.shape
+    if len(k_shape) == 4:
+        page, ks, vs = k_shape[1], k.stride(), v.stride()
+    else:
+        page, ks, vs = 0, (0, *k.stride()), (0, *v.stride())
+
+    def vector(t, dtype):
+        """(address, stride) of an optional vector."""
+        t = _as(t, dtype, keep)
+        return (0, 0) if t is None else (t.data_ptr(), t.stride(0))
+
+    def matrix(t, dtype):
+        """(address, strides) of an optional [.., ..] tensor."""
+        t = _as(t, dtype, keep)
+        return (0, 0, 0) if t is None else (t.data_ptr(), *t.stride())
+
     if torch.is_tensor(p.causal):
-        flags = _as(p.causal, torch.bool, keep)
-        a.causal_by_batch, a.causal_stride, a.causal = flags.data_ptr(), flags.stride(0), 0
+        flags, causal = vector(p.causal, torch.bool), 0
     else:
-        a.causal = int(bool(p.causal))
-    a.window_left, a.window_right = (int(w) for w in p.window)
+        flags, causal = (0, 0), int(bool(p.causal))
+    kind, mask_window, mask_clamp, ranges, prefix, window_len = 0, -1, 0, (0, 0, 0), (0, 0), 0
     if p.mask is not None:
-        a.mask_kind = p.mask.kind
-        a.mask_window = int(p.mask.sliding_window_left)
-        a.mask_clamp = int(bool(p.mask.clamp_prefix_to_window))
-        first, second = (_as(t, i32, keep) for t in p.mask_aux)
-        if p.mask.kind == 1:
-            a.mask_ranges = first.data_ptr()
-            a.ranges_stride[:] = first.stride()
+        kind, mask_window, mask_clamp = p.mask.kind, _int32(p.mask.sliding_window_left), int(bool(p.mask.clamp_prefix_to_window))
+        if kind == 1:
+            ranges = matrix(p.mask_aux[0], i32)
+            _as(p.mask_aux[1], i32, keep)
         else:
-            a.mask_prefix, a.prefix_stride = first.data_ptr(), first.stride(0)
-            a.mask_window_len = second.data_ptr()
-    else:
-        a.mask_kind, a.mask_window, a.mask_clamp = 0, -1, 0
-    a.softmax_scale = float(p.dim_qk ** -0.5 if p.scale is None else p.scale)
-    a.softcap = float(p.softcap)
-    f32 = torch.float32
-    alibi = _as(p.alibi, f32, keep)
-    if alibi is not None:
-        a.alibi = alibi.data_ptr()
-        a.alibi_stride[:] = (0, alibi.stride(0)) if alibi.ndim == 1 else alibi.stride()
-    sinks = _as(p.sinks, f32, keep)
-    if sinks is not None:
-        a.sinks, a.sink_stride = sinks.data_ptr(), sinks.stride(0)
-    for name in ("q_descale", "k_descale", "v_descale"):
-        t = _as(getattr(p, name), f32, keep)
-        if t is not None:
-            setattr(a, name, t.data_ptr())
-            getattr(a, name + "_stride")[:] = t.stride()
-    a.num_splits, a.split_span = 1, 0
-    return a
+            prefix, window_len = vector(p.mask_aux[0], i32), vector(p.mask_aux[1], i32)[0]
+    alibi = (0, 0, 0)
+    if p.alibi is not None:
+        alibi = vector(p.alibi, f32) if p.alibi.ndim == 1 else matrix(p.alibi, f32)
+        if len(alibi) == 2:
+            alibi = (alibi[0], 0, alibi[1])
+    window_left, window_right = p.window
+    return _lib.pack_attn(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
+        code[q.dtype], code[k.dtype], code[v.dtype], code[out.dtype],
+        q_shape[0], q_shape[1], k_shape[-2], q_shape[2], v.shape[-1], p.cu_q.numel() - 1,
+        page, p.max_q if max_q is None else max_q, p.max_k,
+        *q.stride(), *ks, *vs, *out.stride(), *lse.stride(),
+        *vector(p.cu_q, i32), *vector(p.cu_k, i32), *vector(p.used_k, i32), *matrix(p.table, i32), *vector(p.leftpad, i32),
+        causal, _int32(window_left), _int32(window_right), kind, mask_window, mask_clamp, *flags,
+        *ranges, *prefix, window_len,
+        q_shape[2] ** -0.5 if p.scale is None else _float32(p.scale), _float32(p.softcap),
+        *alibi, *vector(p.sinks, f32), *matrix(p.q_descale, f32), *matrix(p.k_descale, f32), *matrix(p.v_descale, f32),
+        1, 0, 0, 0, 0, 0)
 
 
 def _fits_prefill(p, out):
@@ -132,11 +129,12 @@ def _fits_prefill(p, out):
 
 
 def _partials(p, a, shape_out, shape_lse):
-    """fp32 split workspace for the generic kernel or the decode kernel."""
-    po = torch.empty(shape_out, dtype=torch.float32, device=p.device)
-    pl = torch.empty(shape_lse, dtype=torch.float32, device=p.device)
-    p.keep += [po, pl]
-    a.partial_out, a.partial_lse = po.data_ptr(), pl.data_ptr()
+    """fp32 split workspace of one call: outputs, then LSEs from the next 256-byte boundary."""
+    outs = -(-math.prod(shape_out) // 64) * 64
+    work = torch.empty(outs + math.prod(shape_lse), dtype=torch.float32, device=p.device)
+    p.keep.append(work)
+    a.partial_out = work.data_ptr()
+    a.partial_lse = a.partial_out + 4 * outs
 
 
 # Head dims of the fp32 matrix-core kernel (attn_f32.hip, which fa_attn_fwd

@@ -7,6 +7,7 @@ pure-PyTorch fallback: if the library is missing or a call fails, a
 RuntimeError is raised.
 """
 import ctypes
+import struct
 from pathlib import Path
 
 import torch
@@ -94,6 +95,31 @@ class AttnArgs(ctypes.Structure):
                 ("flags", _i32), ("_pad1", _i32)]
 
 
+def _packer(struct_type):
+    """A struct.Struct of the C layout: one pack() sets every field (arrays
+    flattened, pointers as ints), where ctypes sets them one by one (~10 us
+    for an attention call's 90 values, 3 us packed)."""
+    codes = {_p: "P", _i32: "i", _i64: "q", _f32: "f"}
+    fmt = ""
+    for _, t in struct_type._fields_:
+        n = getattr(t, "_length_", 1)
+        fmt += codes[getattr(t, "_type_", t) if n > 1 else t] * n
+    s = struct.Struct("@" + fmt)
+    assert s.size == ctypes.sizeof(struct_type)
+    return s
+
+
+_attn_packer = _packer(AttnArgs)
+
+
+def pack_attn(*values):
+    """An AttnArgs from its fields' values in order, arrays flattened."""
+    try:
+        return AttnArgs.from_buffer_copy(_attn_packer.pack(*values))
+    except struct.error as e:
+        raise TypeError(f"attention sizes and scalars: {e}") from e
+
+
 class MergePairArgs(ctypes.Structure):
     _fields_ = [("out", _p), ("a", _p), ("b", _p), ("a_lse", _p), ("b_lse", _p), ("out_lse", _p),
                 ("dtype", _i32), ("_pad0", _i32),
@@ -148,40 +174,52 @@ def load():
         raise RuntimeError(f"{LIB_PATH.name} is not built; run __graft_entry__.build() "
                            "(make -C flash-attn-mps_amd/csrc)")
     lib = ctypes.CDLL(str(LIB_PATH))
-    for name, (struct, restype) in ENTRY_POINTS.items():
+    for name, (args, restype) in ENTRY_POINTS.items():
         fn = getattr(lib, name)
         fn.restype = restype
         if name == "fa_struct_sizes":
             fn.argtypes = [ctypes.POINTER(_i64)]
-        elif struct is not None:
-            fn.argtypes = ([ctypes.POINTER(struct)] if name.endswith("supported")
-                           else [ctypes.POINTER(struct), _p])
+        elif args is not None:
+            fn.argtypes = ([ctypes.POINTER(args)] if name.endswith("supported")
+                           else [ctypes.POINTER(args), _p])
         else:
             fn.argtypes = []
     if lib.fa_abi_version() != ABI_VERSION:
         raise RuntimeError("libfa_gfx950.so ABI version mismatch")
     sizes = (_i64 * 6)()
     lib.fa_struct_sizes(sizes)
-    for struct, size in zip(STRUCTS, sizes):
-        if ctypes.sizeof(struct) != size:
-            raise RuntimeError(f"{struct.__name__}: ctypes size {ctypes.sizeof(struct)} != C size {size}")
+    for args, size in zip(STRUCTS, sizes):
+        if ctypes.sizeof(args) != size:
+            raise RuntimeError(f"{args.__name__}: ctypes size {ctypes.sizeof(args)} != C size {size}")
     _lib = lib
     return lib
 
 
 def stream_of(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's handle, an int (torch.cuda.current_stream builds a
+    Stream object for it, ~2.5 us a call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+_functions = {}
+
+
+def _function(name):
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(load(), name)
+    return fn
 
 
 def call(name, args, device):
-    lib = load()
-    rc = getattr(lib, name)(ctypes.byref(args), stream_of(device))
+    rc = _function(name)(ctypes.byref(args), stream_of(device))
     if rc != 0:
-        raise RuntimeError(f"{name} failed ({rc}): {lib.fa_last_error().decode()}")
+        raise RuntimeError(f"{name} failed ({rc}): {load().fa_last_error().decode()}")
 
 
 def supported(name, args):
-    return bool(getattr(load(), name)(ctypes.byref(args)))
+    return bool(_function(name)(ctypes.byref(args)))
 
 
 def ptr(t):

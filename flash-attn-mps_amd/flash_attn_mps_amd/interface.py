@@ -120,8 +120,8 @@ def flash_attn_func(
         dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
         deterministic, return_attn_probs, return_softmax_lse=True,
     )
-    out = out.unflatten(0, (batch, sq))
-    return _finish(out, _dense_lse(lse, batch, sq), return_softmax_lse)
+    out = out.view(batch, sq, *out.shape[1:])
+    return (out, _dense_lse(lse, batch, sq)) if return_softmax_lse else out
 
 
 def flash_attn_qkvpacked_func(qkv, *args, **kwargs):
@@ -227,5 +227,5 @@ def flash_attn_with_kvcache(
                       causal=causal, window=tuple(window_size), softcap=softcap, alibi=alibi_slopes,
                       splits=num_splits)
     out, lse = solve(problem.validate())
-    out = out.unflatten(0, (batch, sq))
-    return _finish(out, _dense_lse(lse, batch, sq), return_softmax_lse)
+    out = out.view(batch, sq, *out.shape[1:])
+    return (out, _dense_lse(lse, batch, sq)) if return_softmax_lse else out
