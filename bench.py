@@ -210,8 +210,8 @@ def config2(device, steps, warmup, c=None):
 
 def prefill_d256(device, steps, warmup, c=None):
     """Config 2's lengths with 256-dim heads (Gemma-like, Hq/Hkv 16/8), bf16
-    0.5*N(0,1) Q/K/V, causal: the 256-dim MFMA prefill, which runs each work
-    item as two workgroups, one per 128-column half of V."""
+    0.5*N(0,1) Q/K/V, causal: the 256-dim MFMA prefill, in which two waves share
+    32 query rows, each with one 128-column half of V."""
     import torch
     import flash_attn_mps_amd as fa
     c = c or config2_inputs(device)
@@ -231,7 +231,7 @@ def prefill_d256(device, steps, warmup, c=None):
     flops = causal_pairs(lengths, lengths) * hq * 2 * (d + d)
     return dict(ms=ms, call_ms=call_ms, kernel_ms=kernel_ms, flops=flops, tflops=flops / (ms * 1e-3) / 1e12,
                 what="config 2 lengths, Hq/Hkv 16/8, d256 bf16 causal (Gemma-like heads); "
-                     "two V-column halves per work item")
+                     "wave pairs sharing 32 rows")
 
 
 def prefill_fp8(device, steps, warmup, c=None, defer=False):
