@@ -484,6 +484,7 @@ bool fa_f32_supported(const fa_attn_args& a) {
   if (a.q_dtype != FA_F32 || a.k_dtype != FA_F32 || a.v_dtype != FA_F32) return false;
   if (a.heads_k < 1 || a.heads_q % a.heads_k) return false;
   if (!pick_f32(a.head_dim_qk, a.head_dim_v).kern) return false;
+  if (a.num_splits > 1 && ((uintptr_t)a.partial_out & 15)) return false;   // 16-byte partial stores
   return rows_aligned(a.q, a.q_stride, 2) && rows_aligned(a.k, a.k_stride, 3) && rows_aligned(a.v, a.v_stride, 3);
 }
 

@@ -1399,10 +1399,10 @@ template <> struct PrefillTile<128, 128> {
 // second wave per SIMD, at every grid size (one workgroup per CU ran 7-48%
 // slower even on 128-workgroup launches).
 template <> struct PrefillTile<192, 128> { static constexpr int W = 4, NB = 1, MINB = 2, MINB_WIN = 2; };
-// 256/256 (the softcap routes of pick_256): one wave per SIMD (128 KiB of LDS).
+// 256/256 (softcap routes of pick_256): one wave per SIMD (128 KiB of LDS).
 template <> struct PrefillTile<256, 256> { static constexpr int W = 4, NB = 1, MINB = 1, MINB_WIN = 1; };
-// 256-dim 16-bit heads run as two 256/128 halves of V (prefill_vparts): eight
-// waves in 96 KiB of LDS, two per SIMD.
+// 256-dim heads as two 256/128 halves of V (prefill_vparts): eight waves in 96
+// KiB of LDS, two per SIMD.
 template <> struct PrefillTile<256, 128> { static constexpr int W = 8, NB = 1, MINB = 1, MINB_WIN = 1; };
 
 template <int DQ, int DV>
@@ -1459,6 +1459,8 @@ PrefillChoice pick_tile(int score, bool win, int mk) {
                         : prefill_kernel<T, DQ, DV, S::W, S::NB, S::MINB, CAUSAL, false, false, DQT, DVT, KT, true>;
       }
     }
+  } else if constexpr (DQ == 256 && KT::id != FA_E4M3) {
+    return PrefillChoice{nullptr, 0, 0, 0};   // wave pairs (prefill_pair.h)
   } else if (win)
     c.kern = cap ? prefill_kernel<T, DQ, DV, S::W, S::NB, S::MINB_WIN, CAUSAL, true, true, DQT, DVT, KT>
                  : prefill_kernel<T, DQ, DV, S::W, S::NB, S::MINB_WIN, CAUSAL, false, true, DQT, DVT, KT>;

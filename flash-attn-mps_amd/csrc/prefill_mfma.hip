@@ -213,7 +213,8 @@ extern "C" int fa_prefill_fwd(const fa_attn_args* a, void* stream) {
   blocks *= ch.vparts;
   FA_REQUIRE(blocks <= 0x7fffffffll, "fa_prefill_fwd: grid too large");
   const bool split = a->num_splits > 1;
-  FA_REQUIRE(!split || (a->partial_out && a->partial_lse), "fa_prefill_fwd: splits need partial buffers");
+  FA_REQUIRE(!split || (a->partial_out && a->partial_lse && aligned16(a->partial_out)),
+             "fa_prefill_fwd: splits need partial buffers, the outputs' 16-byte aligned");
   FA_REQUIRE(!split || (a->batch <= 65535 && a->max_seqlen_q * a->heads_q <= 0x7fffffffll),
              "fa_prefill_fwd: split grid too large");
   hipError_t err = hipFuncSetAttribute((const void*)ch.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ch.lds);

@@ -186,8 +186,9 @@ typedef struct fa_attn_args {
                                         R = max(1, max_seqlen_q) */
   float* partial_out;                /* num_splits > 1: caller-owned fp32 workspace,
                                         fa_decode_fwd [batch, S, R, Hq, Dv] contiguous,
-                                        fa_attn_fwd [S, total_q, Hq, Dv] contiguous */
-  float* partial_lse;                /* fa_decode_fwd [batch, R, Hq, S], fa_attn_fwd [S, Hq, total_q] */
+                                        fa_attn_fwd / fa_prefill_fwd [S, total_q, Hq, Dv]
+                                        contiguous */
+  float* partial_lse;                /* fa_decode_fwd [batch, R, Hq, S], the others [S, Hq, total_q] */
 
   int32_t flags;                     /* FA_FLAG_* bits */
   int32_t _pad1;
@@ -269,7 +270,9 @@ int fa_decode_fwd_noalloc(const fa_attn_args* args, void* stream);
  * combines with softcap, windows, per-request causality and E4M3 K/V at
  * unpadded 64/128/256-dim heads; head dims 32-256 and 192/128).
  * fa_prefill_supported() says whether the argument
- * combination is compiled in.  With FA_FLAG_SKIP_SINGLE_QUERY in
+ * combination is compiled in; num_splits 2..64 splits the keys (partial_out 16-byte
+ * aligned) where windows, ALiBi and mask kinds are absent and the head dims
+ * are 64, 128 (softcap too), 192/128 or 256.  With FA_FLAG_SKIP_SINGLE_QUERY in
  * args->flags, requests with one query row are left untouched for
  * fa_decode_fwd (no reference counterpart: the reference runs such rows
  * through its prefill tile, flash_attn_mps/_attention.py:149-158). */
