@@ -170,8 +170,8 @@ def rotary_append(q, k, v, k_cache, v_cache, lengths, cos, sin, *, cache_batch_i
                   and q.numel() and k.numel() and v.numel() and lengths.numel() == k.shape[0]
                   and (cos is None or (cos.numel() and cos.dtype in _INPUT_TYPES and sin.dtype == cos.dtype
                                        and cos.device == sin.device == q.device))
-                  and (cache_leftpad is None or (cache_leftpad.dtype == torch.int32 and cache_leftpad.ndim == 1
-                                                 and cache_leftpad.device == q.device)))
+                  and (cache_leftpad is None or (cache_leftpad.dtype == torch.int32 and cache_leftpad.device == q.device
+                                                 and cache_leftpad.shape == k.shape[:1])))
     if not one_launch:
         if cos is not None:
             q, k = rotary(q, k, cos, sin, lengths, rotary_interleaved=rotary_interleaved, causal=causal,

@@ -282,3 +282,15 @@ def test_rotary_append_equals_its_parts(device, dtype, cache_dtype, interleaved,
             assert torch.equal(got.view(bits), want.view(bits))
         pad = kw["cache_leftpad"]
         assert torch.equal(after, lengths + new - (0 if pad is None else pad))
+
+
+def test_leftpad_of_one_value_is_refused_for_more_requests(device):
+    """The appended call is refused by its contract, and nothing reads the
+    one-entry vector per request on the way."""
+    import flash_attn_mps_amd as fa
+    q = torch.zeros(3, 1, 4, 64, dtype=torch.float16, device=device)
+    kv = torch.zeros(3, 1, 2, 64, dtype=torch.float16, device=device)
+    cache = torch.zeros(3, 32, 2, 64, dtype=torch.float16, device=device)
+    with pytest.raises(ValueError, match="leftpad"):
+        fa.flash_attn_with_kvcache(q, cache, cache.clone(), kv, kv, cache_seqlens=4,
+                                   cache_leftpad=torch.ones(1, dtype=torch.int32, device=device))
