@@ -143,6 +143,9 @@ def _append_args(k, v, k_cache, v_cache, cache_seqlens, cache_batch_idx, cache_l
     table = None if block_table is None else block_table.to(torch.int32).contiguous()
     _check_cache_shape(k, k_cache, 2)
     _check_cache_shape(v, v_cache, 2)
+    # Positions are bounded by the K cache's extents in both writes.
+    if v_cache.shape[0] < k_cache.shape[0] or v_cache.shape[1] < k_cache.shape[1]:
+        raise ValueError(f"the V cache {tuple(v_cache.shape)} is smaller than the K cache {tuple(k_cache.shape)}")
     writes = [(x, c, s) for x, c, s in ((k, k_cache, k_scale), (v, v_cache, v_scale)) if x.numel()]
     if not writes:
         return None

@@ -29,3 +29,19 @@ def test_leftpad_of_another_count_is_refused(monkeypatch):
     with pytest.raises(ValueError, match="cache_leftpad"):
         _cache.rotary_append(q, k, k, cache, cache, torch.tensor([3, 5], dtype=torch.int32), None, None,
                              cache_leftpad=torch.tensor([1, 2, 3], dtype=torch.int32))
+
+
+@pytest.mark.parametrize("v_shape,ok", [((2, 16), True), ((3, 32), True), ((1, 16), False), ((2, 8), False)])
+def test_append_bounds_cover_both_caches(monkeypatch, v_shape, ok):
+    """The kernel bounds both writes by the K cache's rows and capacity."""
+    calls = []
+    monkeypatch.setattr(_cache, "_require_gpu", lambda **tensors: None)
+    monkeypatch.setattr(_lib, "call", lambda name, args, device: calls.append(name))
+    k, k_cache, v_cache = torch.zeros(2, 1, 2, 8), torch.zeros(2, 16, 2, 8), torch.zeros(*v_shape, 2, 8)
+    lengths = torch.tensor([3, 5], dtype=torch.int32)
+    if ok:
+        _cache.append_kvcache(k, k, k_cache, v_cache, lengths)
+    else:
+        with pytest.raises(ValueError, match="V cache"):
+            _cache.append_kvcache(k, k, k_cache, v_cache, lengths)
+    assert calls == ["fa_append_kvcache"] * ok
