@@ -11,6 +11,7 @@ packed QKV/KV tensors become views.  The adapted call is a
 :class:`~flash_attn_mps_amd._problem.Problem`, validated in full on the host
 and then solved by the gfx950 kernels (``_attention.solve``).
 """
+import threading
 from collections import OrderedDict
 
 import torch
@@ -21,42 +22,52 @@ from ._problem import MaskSpec, Problem, reject_training  # noqa: F401  (MaskSpe
 PAGE_MULTIPLE = 16   # paged caches: page sizes the FlashAttention contract accepts
 
 
-class _Resident:
-    """Small int32 index tensors of (batch, length) on a device, made once per
-    (device, batch, length) by `make`.
+class _Counting:
+    """The int32 vector 0, 1, 2, ... on each device, made once and kept, and the
+    index tensors that are strided views of it: the offsets 0, L, 2 L, ..., B L
+    of a dense batch and the identity table [B, 1] of a dense cache (request b
+    reads row b).
 
-    Dense layers of one model reuse a handful of shapes, so a small LRU keeps
-    the tensors resident and a call adds no kernel.  Entries are copied from
-    the host, complete when the call that makes them returns (so any stream
-    may read them), and never written again.  While a graph is being captured
-    a missing entry is made by a captured kernel and not kept: its memory
-    belongs to the graph.
+    A call so adds no kernel and no copy, whatever its shape, and nothing that
+    a captured HIP graph or another stream reads is ever freed or written: the
+    vector is copied from the host, complete when the call that makes it
+    returns, and the small LRU holds views of it.  Its 2^20 entries (4 MiB)
+    are the bound of what stays resident; offsets past them, and any made
+    while a graph is captured before the vector exists, come from kernels on
+    the caller's stream (2 launches) and belong to the call or the graph.
     """
 
-    def __init__(self, make, capacity=64):
-        self._make = make
-        self._entries = OrderedDict()
-        self._capacity = capacity
+    def __init__(self, entries=1 << 20, views=64):
+        self._entries, self._capacity = entries, views
+        self._vectors, self._views = {}, OrderedDict()
+        self._lock = threading.Lock()
 
-    def __call__(self, batch, length, device):
-        key = (device.type, device.index, batch, length)
-        hit = self._entries.get(key)
-        if hit is None:
-            if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
-                return self._make(batch, length, device)
-            hit = self._make(batch, length, "cpu").to(device)
-            self._entries[key] = hit
-            if len(self._entries) > self._capacity:
-                self._entries.popitem(last=False)
-        else:
-            self._entries.move_to_end(key)
-        return hit
+    def offsets(self, batch, length, device):
+        return self._view(device, (batch + 1,), (length,), batch * length)
+
+    def rows(self, batch, device):
+        return self._view(device, (batch, 1), (1, 1), batch - 1)
+
+    def _view(self, device, shape, stride, last):
+        key = (device.type, device.index, shape, stride)
+        with self._lock:
+            hit = self._views.get(key)
+            if hit is not None:
+                self._views.move_to_end(key)
+                return hit
+            vector = self._vectors.get(key[:2])
+            if vector is None and not (device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
+                vector = torch.arange(self._entries, dtype=torch.int32).to(device)
+                self._vectors[key[:2]] = vector
+            if vector is None or last >= self._entries:
+                return (torch.arange(shape[0], dtype=torch.int32, device=device) * stride[0]).reshape(shape)
+            view = self._views[key] = vector.as_strided(shape, stride)
+            if len(self._views) > self._capacity:
+                self._views.popitem(last=False)
+            return view
 
 
-# Offsets 0, L, 2 L, ..., B L of a dense batch, and the identity table [B, 1]
-# of a dense cache (request b reads row b).
-_offsets = _Resident(lambda b, n, device: torch.arange(b + 1, dtype=torch.int32, device=device) * n)
-_rows = _Resident(lambda b, n, device: torch.arange(b, dtype=torch.int32, device=device).reshape(b, n))
+_counting = _Counting()
 
 
 def _check_page_size(k):
@@ -114,9 +125,10 @@ def flash_attn_func(
         raise ValueError(f"batch/length/head extents disagree: q {tuple(q.shape)}, "
                          f"k {tuple(k.shape)}, v {tuple(v.shape)}")
     batch, sq, sk = q.shape[0], q.shape[1], k.shape[1]
+    cu_q = _counting.offsets(batch, sq, q.device)
+    cu_k = cu_q if sk == sq else _counting.offsets(batch, sk, q.device)
     out, lse = flash_attn_varlen_func(
-        q.flatten(0, 1), k.flatten(0, 1), v.flatten(0, 1),
-        _offsets(batch, sq, q.device), _offsets(batch, sk, q.device), sq, sk,
+        q.flatten(0, 1), k.flatten(0, 1), v.flatten(0, 1), cu_q, cu_k, sq, sk,
         dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
         deterministic, return_attn_probs, return_softmax_lse=True,
     )
@@ -221,8 +233,8 @@ def flash_attn_with_kvcache(
     elif cache_batch_idx is not None:
         table, max_k = cache_batch_idx.to(torch.int32).reshape(batch, 1), k_cache.shape[1]
     else:
-        table, max_k = _rows(batch, 1, q.device), k_cache.shape[1]
-    problem = Problem(q.flatten(0, 1), k_cache, v_cache, _offsets(batch, sq, q.device), sq, max_k,
+        table, max_k = _counting.rows(batch, q.device), k_cache.shape[1]
+    problem = Problem(q.flatten(0, 1), k_cache, v_cache, _counting.offsets(batch, sq, q.device), sq, max_k,
                       used_k=lengths, table=table, leftpad=cache_leftpad, scale=softmax_scale,
                       causal=causal, window=tuple(window_size), softcap=softcap, alibi=alibi_slopes,
                       splits=num_splits)

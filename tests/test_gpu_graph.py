@@ -246,3 +246,30 @@ def test_graph_fp8_chunked_prefill_mixed_batch(device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), f"replay {it}"
+
+
+def test_graph_of_a_dense_cache_outlives_its_index_tensors(device):
+    """A graph captured after warm calls reads the resident offsets and the
+    identity table: 100 other batch sizes and lengths, and memory filled with
+    large indices after each, leave its replays unchanged."""
+    gen = torch.Generator().manual_seed(75)
+    batch, capacity, hq, hkv, d = 5, 96, 8, 4, 64
+    kc, vc = (torch.randn(batch, capacity, hkv, d, generator=gen).to(torch.bfloat16).to(device) for _ in range(2))
+    q = torch.randn(batch, 1, hq, d, generator=gen).to(torch.bfloat16).to(device)
+    lens = torch.tensor([3, 96, 40, 0, 64], dtype=torch.int32, device=device)
+
+    def call():
+        return fa.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, return_softmax_lse=True)
+
+    graph, (g_out, g_lse) = capture(call)
+    e_out, e_lse = call()
+    for n in range(1, 101):
+        other = torch.zeros(n, 1 + n % 3, 2, 64, dtype=torch.bfloat16, device=device)
+        fa.flash_attn_with_kvcache(other, other, other, cache_seqlens=1)
+        junk = [torch.full((m,), 1 << 20, dtype=torch.int32, device=device) for m in (1, batch, batch + 1, 128)]
+    for it in range(REPLAYS):
+        g_out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(g_out, e_out) and torch.equal(g_lse, e_lse), f"replay {it}"
+    assert len(junk) == 4
