@@ -66,6 +66,15 @@ FA_DEV float descale_of(const float* p, const int64_t* st, int64_t b, int kh) {
   return p ? p[b * st[0] + (int64_t)kh * st[1]] : 1.0f;
 }
 
+// The arguments with window bounds of 2^30 and more (past any two positions'
+// distance) as -1, unbounded: the kernels add bounds to positions in 32 bits.
+inline fa_attn_args fa_bounded(const fa_attn_args& args) {
+  fa_attn_args a = args;
+  if (a.window_left >= 1 << 30) a.window_left = -1;
+  if (a.window_right >= 1 << 30) a.window_right = -1;
+  return a;
+}
+
 // Host-side argument checks shared by fa_attn_fwd / fa_decode_fwd / fa_prefill_fwd.
 int fa_validate_attn(const fa_attn_args* a, const char* who);
 

@@ -362,9 +362,11 @@ int scratch_of_device(void* stream, float** out) {
 
 }  // namespace
 
-extern "C" int fa_decode_fwd(const fa_attn_args* a, void* stream) {
-  const int rc = fa_validate_attn(a, "fa_decode_fwd");
-  return rc ? rc : decode_launch(a, stream, "fa_decode_fwd");
+extern "C" int fa_decode_fwd(const fa_attn_args* args, void* stream) {
+  const int rc = fa_validate_attn(args, "fa_decode_fwd");
+  if (rc) return rc;
+  const fa_attn_args a = fa_bounded(*args);
+  return decode_launch(&a, stream, "fa_decode_fwd");
 }
 
 extern "C" int fa_decode_fwd_noalloc(const fa_attn_args* in, void* stream) {
@@ -372,7 +374,7 @@ extern "C" int fa_decode_fwd_noalloc(const fa_attn_args* in, void* stream) {
   FA_REQUIRE(in->partial_out == nullptr && in->partial_lse == nullptr,
              "fa_decode_fwd_noalloc: partial buffers are library-owned; pass NULL");
   FA_REQUIRE(in->num_splits >= 0, "fa_decode_fwd_noalloc: num_splits must be >= 0");
-  fa_attn_args a = *in;
+  fa_attn_args a = fa_bounded(*in);
   constexpr int64_t cap = FA_DECODE_SCRATCH_BYTES / (int64_t)sizeof(float);
   if (a.num_splits == 0) {
     FA_REQUIRE(a.batch >= 1 && a.heads_k >= 1 && a.heads_q % a.heads_k == 0,

@@ -147,9 +147,10 @@ int fa_validate_attn(const fa_attn_args* a, const char* who) {
   return FA_OK;
 }
 
-extern "C" int fa_attn_fwd(const fa_attn_args* a, void* stream) {
-  int rc = fa_validate_attn(a, "fa_attn_fwd");
+extern "C" int fa_attn_fwd(const fa_attn_args* args, void* stream) {
+  int rc = fa_validate_attn(args, "fa_attn_fwd");
   if (rc) return rc;
+  const fa_attn_args bounded = fa_bounded(*args), *a = &bounded;
   if (a->total_q == 0) return FA_OK;
   FA_REQUIRE(a->num_splits == 1 || (a->partial_out && a->partial_lse), "fa_attn_fwd: splits need partial buffers");
   FA_REQUIRE(a->max_seqlen_q >= 1, "fa_attn_fwd: max_seqlen_q must be positive");

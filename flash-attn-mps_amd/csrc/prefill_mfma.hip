@@ -166,12 +166,13 @@ bool prefill_ok(const fa_attn_args& a) {
 }  // namespace
 
 extern "C" int fa_prefill_supported(const fa_attn_args* a) {
-  return a != nullptr && prefill_ok(*a);
+  return a != nullptr && prefill_ok(fa_bounded(*a));
 }
 
-extern "C" int fa_prefill_fwd(const fa_attn_args* a, void* stream) {
-  int rc = fa_validate_attn(a, "fa_prefill_fwd");
+extern "C" int fa_prefill_fwd(const fa_attn_args* args, void* stream) {
+  int rc = fa_validate_attn(args, "fa_prefill_fwd");
   if (rc) return rc;
+  const fa_attn_args bounded = fa_bounded(*args), *a = &bounded;
   if (!prefill_ok(*a)) {
     fa_set_error("fa_prefill_fwd: combination not supported by the MFMA kernel");
     return FA_ERR_UNSUPPORTED;

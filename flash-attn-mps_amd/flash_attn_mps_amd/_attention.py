@@ -45,10 +45,12 @@ def _as(t, dtype, keep):
     return t
 
 
-def _int32(x):
-    """x wrapped to 32 bits, as a C assignment does (a window of sys.maxsize is unbounded)."""
+def _bound(x):
+    """A window bound as the kernels take it: 2^30 and more (past any two
+    positions' distance, sys.maxsize among them) is -1, unbounded, so that
+    positions plus bounds stay in 32 bits."""
     x = int(x)
-    return x if -1 <= x < 1 << 31 else (x + (1 << 31)) % (1 << 32) - (1 << 31)
+    return x if -1 <= x < 1 << 30 else -1
 
 
 def _float32(x):
@@ -85,7 +87,7 @@ def build_args(p, out, lse, max_q=None):
         flags, causal = (0, 0), int(bool(p.causal))
     kind, mask_window, mask_clamp, ranges, prefix, window_len = 0, -1, 0, (0, 0, 0), (0, 0), 0
     if p.mask is not None:
-        kind, mask_window, mask_clamp = p.mask.kind, _int32(p.mask.sliding_window_left), int(bool(p.mask.clamp_prefix_to_window))
+        kind, mask_window, mask_clamp = p.mask.kind, _bound(p.mask.sliding_window_left), int(bool(p.mask.clamp_prefix_to_window))
         if kind == 1:
             ranges = matrix(p.mask_aux[0], i32)
             _as(p.mask_aux[1], i32, keep)
@@ -104,7 +106,7 @@ def build_args(p, out, lse, max_q=None):
         page, p.max_q if max_q is None else max_q, p.max_k,
         *q.stride(), *ks, *vs, *out.stride(), *lse.stride(),
         *vector(p.cu_q, i32), *vector(p.cu_k, i32), *vector(p.used_k, i32), *matrix(p.table, i32), *vector(p.leftpad, i32),
-        causal, _int32(window_left), _int32(window_right), kind, mask_window, mask_clamp, *flags,
+        causal, _bound(window_left), _bound(window_right), kind, mask_window, mask_clamp, *flags,
         *ranges, *prefix, window_len,
         q_shape[2] ** -0.5 if p.scale is None else _float32(p.scale), _float32(p.softcap),
         *alibi, *vector(p.sinks, f32), *matrix(p.q_descale, f32), *matrix(p.k_descale, f32), *matrix(p.v_descale, f32),
