@@ -88,8 +88,10 @@ FA_DEV uint64_t shfl_u64(uint64_t x, int src) {
 }
 
 // DQ, DV: the tensors' head dims (multiples of 8).  V columns past DV inside
-// the 32-dim blocks re-read real columns and are not stored.
-template <int DQ, int DV, int MINB>
+// the 32-dim blocks re-read real columns and are not stored.  MASKS: the vLLM
+// mask kinds (a.mask_kind 1 or 2), in variants of their own: their second key
+// range and the gaps it leaves would cost the others 4-24 spilled registers.
+template <int DQ, int DV, int MINB, bool MASKS>
 __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa_attn_args a, const F32Shape shp) {
   static_assert(DQ % 8 == 0 && DV % 8 == 0 && DQ <= 256 && DV <= 256, "head dims");
   constexpr int KT = DQ / 8;                       // 16-byte key pieces per lane
@@ -123,39 +125,41 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   const int h0 = kh * group + t0;
 
   // This lane's column: head h0 + chead, query row q0 + crow, and the keys it
-  // sees, [lo, hi) (mask kinds: [0, hi), refined per key below).
+  // sees, [lo, hi) and, with mask kinds, [lo2, hi2) too.
   const int chead = l32 >> rl, crow = l32 & (R - 1);
   const bool col_ok = chead < nheads && q0 + crow < r.q_len;
   const int qa = q0 + crow + r.k_len - r.q_len;
   const int64_t tq = (int64_t)r.q_begin + q0 + (col_ok ? crow : 0);
   const int hq = h0 + (col_ok ? chead : 0);
-  int lo = INT_MAX, hi = INT_MIN, mlo = -1, mhi = -1, mwin = -1;
+  int lo = INT_MAX, hi = 0, lo2 = INT_MAX, hi2 = 0;
   if (col_ok) {
     lo = 0, hi = r.k_len;
-    if (a.mask_kind == 0) {
+    auto from_window = [&](int w) { return max(qa - min(w, 1 << 30) + 1, 0); };   // keys of the last w positions
+    if (!MASKS) {
       if (r.causal) hi = min(hi, qa + 1);
       if (a.window_right >= 0) hi = min(hi, qa + a.window_right + 1);
       if (a.window_left >= 0) lo = max(qa - a.window_left, 0);
-    } else if (a.mask_kind == 1) {
-      mlo = a.mask_ranges[tq * a.ranges_stride[0]];
-      mhi = a.mask_ranges[tq * a.ranges_stride[0] + a.ranges_stride[1]];
-      mwin = a.mask_window;
-      hi = min(hi, max(qa, mlo >= 0 ? mhi : -1) + 1);
-    } else {
-      mhi = a.mask_prefix[b * a.prefix_stride];
-      mwin = a.mask_window_len[0];
-      hi = min(hi, qa + 1);
+    } else if (a.mask_kind == 1) {   // the causal window, and the row's range
+      const int first = a.mask_window >= 0 ? from_window(a.mask_window) : 0;
+      const int from = a.mask_ranges[tq * a.ranges_stride[0]];
+      const int to = a.mask_ranges[tq * a.ranges_stride[0] + a.ranges_stride[1]];
+      lo = first, hi = min(hi, qa + 1);
+      if (from >= 0) lo2 = a.mask_clamp ? max(from, first) : from, hi2 = min(to, r.k_len - 1) + 1;
+    } else {                         // the prefix, and the causal window
+      lo2 = from_window(a.mask_window_len[0]), hi2 = min(hi, qa + 1);
+      hi = min(hi2, a.mask_prefix[b * a.prefix_stride]);
     }
-    if (hi <= lo) lo = INT_MAX, hi = INT_MIN;   // a row without keys bounds nothing
+    if (hi <= lo) lo = INT_MAX, hi = 0;   // a range without keys bounds nothing
+    if (hi2 <= lo2) lo2 = INT_MAX, hi2 = 0;
   }
   // Keys of the workgroup, [kbeg, kend), and those every column sees.
-  const int kbeg = __builtin_amdgcn_readfirstlane(wave_min_i(lo));
-  const int kend = __builtin_amdgcn_readfirstlane(wave_max_i(hi));
+  const int kbeg = __builtin_amdgcn_readfirstlane(wave_min_i(min(lo, lo2)));
+  const int kend = __builtin_amdgcn_readfirstlane(wave_max_i(max(hi, hi2)));
   const bool bounds = col_ok && hi > lo;
   const int full_lo = __builtin_amdgcn_readfirstlane(wave_max_i(bounds ? lo : INT_MIN));
   const int full_hi = __builtin_amdgcn_readfirstlane(wave_min_i(bounds ? hi : INT_MAX));
   // A column without keys among columns that have some: masked everywhere.
-  const bool any_empty = __any(col_ok && !bounds) || a.mask_kind != 0;
+  const bool any_empty = __any(col_ok && !bounds) || MASKS;
   // This split's rounds of 128 keys.
   const int rnd0 = kbeg < kend ? kbeg / F32_ROUND : 0;
   const int nrnd = kbeg < kend ? (kend + F32_ROUND - 1) / F32_ROUND - rnd0 : 0;
@@ -181,10 +185,30 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   const float* const vhead = (const float*)a.v + (int64_t)kh * a.v_stride[2];
   const int P = (int)a.page_size, lp = shp.log2_page;
   const int32_t* const trow = P ? a.block_table + b * a.bt_stride[0] : nullptr;
-  // Row offsets (elements) of key k0 + l32 in K and V.  Keys outside
-  // [kbeg, kend) take a row inside it: what lies there is never read.
-  auto rows_of = [&](int k0, uint64_t& kr, uint64_t& vr) {
-    const int key = min(max(k0 + l32, kbeg), kend - 1);
+  // Mask kinds: the keys of the stage at k0 that some column sees, as bits
+  // (without them, the stage's keys between kbeg and kend).
+  auto seen_of = [&](int k0) -> uint32_t {
+    auto ones = [](int n) { return n >= 32 ? ~0u : (1u << max(n, 0)) - 1u; };
+    uint32_t mine = hi > lo ? ones(hi - k0) & ~ones(lo - k0) : 0u;
+    if (hi2 > lo2) mine |= ones(hi2 - k0) & ~ones(lo2 - k0);
+#pragma unroll
+    for (int m = 16; m >= 1; m >>= 1) mine |= (uint32_t)__shfl_xor((int)mine, m);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)mine);
+  };
+  // This wave's first round from `rnd` on with such a key, and its keys.
+  auto next_round = [&](int rnd, uint32_t& seen) {
+    if constexpr (MASKS) {
+      seen = 0u;
+      for (; rnd < re; ++rnd)
+        if ((seen = seen_of(F32_ROUND * rnd + F32_STAGE * wave))) break;
+    }
+    return rnd;
+  };
+  // Row offsets (elements) of key k0 + l32 in K and V.  Keys that no column
+  // sees take a row that one does: their table entries and rows, which may
+  // hold anything, are never read.
+  auto rows_of = [&](int k0, uint32_t seen, uint64_t& kr, uint64_t& vr) {
+    const int key = !MASKS ? min(max(k0 + l32, kbeg), kend - 1) : (seen >> l32) & 1 ? k0 + l32 : kbeg;
     const int64_t pos = (int64_t)r.k_base + r.left + key;
     if (P) {
       const int page = lp >= 0 ? (int)pos >> lp : (int)pos / P;
@@ -231,8 +255,11 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
 
   // The first keys, then the queries: both round trips to memory run together.
   uint64_t kr = 0, vr = 0, kn, vn;
+  int rnd = rb;
+  uint32_t seen = 0;
   if (rb < re) {
-    rows_of(F32_ROUND * rb + F32_STAGE * wave, kr, vr);
+    rnd = next_round(rb, seen);
+    rows_of(F32_ROUND * rnd + F32_STAGE * wave, seen, kr, vr);
     load_k(kr, q0c);
   }
   // Q^T operands in LDS: piece t of lane (column l32, half hh) is dims
@@ -250,9 +277,12 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   }
   __syncthreads();
   if (rb < re) {
-    for (int rnd = rb; rnd < re; ++rnd) {
+    int next;
+    for (; rnd < re; rnd = next) {
       const int k0 = F32_ROUND * rnd + F32_STAGE * wave;
-      rows_of(k0 + F32_ROUND, kn, vn);   // the next stage's rows (past the last one: clamped, unused)
+      uint32_t seen_next = 0u;   // the next stage's rows (past the last one: a valid row, unused)
+      next = next_round(rnd + 1, seen_next);
+      rows_of(F32_ROUND * next + F32_STAGE * wave, seen_next, kn, vn);
       f32x16 s;
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = 0.0f;
@@ -292,15 +322,8 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
       if (k0 < full_lo || k0 + F32_STAGE > full_hi || any_empty) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int key = key0 + 8 * (i >> 2) + (i & 3);
-          bool see = key >= lo && key < hi;
-          if (a.mask_kind == 1) {
-            const int diff = qa - key;
-            const bool in_win = mwin < 0 || diff < mwin;
-            see = see && ((diff >= 0 && in_win) || (mlo >= 0 && key >= mlo && key <= mhi && (!a.mask_clamp || in_win)));
-          } else if (a.mask_kind == 2) {
-            see = see && (key < mhi || qa - key < mwin);
-          }
+          const int key = 8 * (i >> 2) + (i & 3);   // from key0
+          const bool see = (key >= lo - key0 && key < hi - key0) || (MASKS && key >= lo2 - key0 && key < hi2 - key0);
           s[i] = see ? s[i] : -INFINITY;
         }
       }
@@ -327,10 +350,11 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
       l_run += psum;
       auto pv = [&](auto q) {
         constexpr int Q = decltype(q)::value;
-        if (edge) {   // rows that are not the stage's own: no value of theirs may reach O
+        if (MASKS ? seen != ~0u : edge) {   // rows that are not the stage's own: no value of theirs may reach O
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const bool own = key0 + 8 * Q + i >= kbeg && key0 + 8 * Q + i < kend;
+            const int key = key0 + 8 * Q + i;
+            const bool own = MASKS ? (seen >> (key - k0)) & 1 : key >= kbeg && key < kend;
 #pragma unroll
             for (int u = 0; u < VL; ++u)
 #pragma unroll
@@ -357,6 +381,7 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
       kr = kn, vr = vn;
       load_k(kr, q0c);
       pv(q3c);
+      seen = seen_next;
     }
   }
 
@@ -451,21 +476,22 @@ struct F32Choice {
 
 // Workgroups per CU (waves per SIMD): 168 registers at three (d128 spills
 // 14), 128 at four; d256 holds 128 for O^T alone and runs one.
-template <int DQ, int DV, int MINB> F32Choice f32_choice() {
-  return F32Choice{attn_f32_kernel<DQ, DV, MINB>, f32_lds_bytes<DQ, DV>()};
+template <int DQ, int DV, int MINB> F32Choice f32_choice(bool masks) {
+  return F32Choice{masks ? attn_f32_kernel<DQ, DV, MINB, true> : attn_f32_kernel<DQ, DV, MINB, false>,
+                   f32_lds_bytes<DQ, DV>()};
 }
 
-F32Choice pick_f32(int64_t dq, int64_t dv) {
-  if (dq == 192 && dv == 128) return f32_choice<192, 128, 2>();
+F32Choice pick_f32(int64_t dq, int64_t dv, bool masks) {
+  if (dq == 192 && dv == 128) return f32_choice<192, 128, 2>(masks);
   if (dq != dv) return F32Choice{nullptr, 0};
   switch (dq) {
-    case 32: return f32_choice<32, 32, 4>();
-    case 64: return f32_choice<64, 64, 4>();
-    case 72: return f32_choice<72, 72, 3>();
-    case 80: return f32_choice<80, 80, 3>();
-    case 96: return f32_choice<96, 96, 3>();
-    case 128: return f32_choice<128, 128, 3>();
-    case 256: return f32_choice<256, 256, 1>();
+    case 32: return f32_choice<32, 32, 4>(masks);
+    case 64: return f32_choice<64, 64, 4>(masks);
+    case 72: return f32_choice<72, 72, 3>(masks);
+    case 80: return f32_choice<80, 80, 3>(masks);
+    case 96: return f32_choice<96, 96, 3>(masks);
+    case 128: return f32_choice<128, 128, 3>(masks);
+    case 256: return f32_choice<256, 256, 1>(masks);
     default: return F32Choice{nullptr, 0};
   }
 }
@@ -483,13 +509,13 @@ bool rows_aligned(const void* p, const int64_t* st, int n) {
 bool fa_f32_supported(const fa_attn_args& a) {
   if (a.q_dtype != FA_F32 || a.k_dtype != FA_F32 || a.v_dtype != FA_F32) return false;
   if (a.heads_k < 1 || a.heads_q % a.heads_k) return false;
-  if (!pick_f32(a.head_dim_qk, a.head_dim_v).kern) return false;
+  if (!pick_f32(a.head_dim_qk, a.head_dim_v, a.mask_kind != 0).kern) return false;
   if (a.num_splits > 1 && ((uintptr_t)a.partial_out & 15)) return false;   // 16-byte partial stores
   return rows_aligned(a.q, a.q_stride, 2) && rows_aligned(a.k, a.k_stride, 3) && rows_aligned(a.v, a.v_stride, 3);
 }
 
 int fa_f32_launch(const fa_attn_args& a, void* stream) {
-  const F32Choice ch = pick_f32(a.head_dim_qk, a.head_dim_v);
+  const F32Choice ch = pick_f32(a.head_dim_qk, a.head_dim_v, a.mask_kind != 0);
   const int64_t group = a.heads_q / a.heads_k;
   F32Shape shp;
   shp.log2_rows = 0;

@@ -107,3 +107,64 @@ def test_rows_do_not_depend_on_the_batch(device):
     alone, lse1 = attention(q[:8], k[:500], v[:500], cu_seqlens_q=cu_q[:2], cu_seqlens_k=cu_k[:2], max_seqlen_q=8,
                             max_seqlen_k=500, **run)
     assert torch.equal(both[:8], alone) and torch.equal(lse[:, :8], lse1)
+
+
+@pytest.mark.parametrize("mask", ["prefix", "rolling", "prefix_rows", "clamped"])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_masked_keys_that_no_row_sees(device, mask, splits, dim):
+    """Mask kinds leave keys unseen before the first window, between a prefix
+    and the windows, and between rows' own ranges: whole pages (whose table
+    entries then lead elsewhere) and single keys inside a 32-key stage.  They
+    hold NaN and infinities here, and no result may show them."""
+    page, q_lens, k_lens = 16, [40, 3], [700, 333]
+    total = sum(q_lens)
+    cols = -(-max(k_lens) // page)
+    cu_q, used = offsets(q_lens, device), torch.tensor(k_lens, dtype=torch.int32, device=device)
+    if mask == "rolling":
+        spec, aux = vllm.rswa_mask(), [torch.tensor([50, 7], dtype=torch.int32, device=device),
+                                       torch.tensor([21], dtype=torch.int32, device=device)]
+    else:
+        ranges = torch.full((total, 2), -1, dtype=torch.int32)
+        if mask == "prefix_rows":
+            ranges[5:9] = torch.tensor([[300, 310], [77, 77], [0, 3], [640, 2 ** 31 - 1]], dtype=torch.int32)
+        elif mask == "clamped":
+            ranges[:] = torch.tensor([0, 650], dtype=torch.int32)
+        ranges[41] = torch.tensor([100, 120], dtype=torch.int32)
+        spec, aux = vllm.mm_prefix_mask(20, mask == "clamped"), [ranges.to(device), cu_q]
+    # The keys each request's rows see, by the definition of the masks.
+    seen, row = [torch.zeros(n, dtype=torch.bool) for n in k_lens], 0
+    for b, (nq, nk) in enumerate(zip(q_lens, k_lens)):
+        key = torch.arange(nk)
+        for i in range(nq):
+            diff = i + nk - nq - key
+            if mask == "rolling":
+                see = (diff >= 0) & ((key < int(aux[0][b])) | (diff < 21))
+            else:
+                first, last = ranges[row].tolist()
+                see = (diff >= 0) & (diff < 20)
+                if first >= 0:
+                    see |= (key >= first) & (key <= last) & ((diff < 20) if mask == "clamped" else True)
+            seen[b] |= see
+            row += 1
+    table = torch.full((2, cols), -1, dtype=torch.int64)
+    poison = 2 * cols   # the page of unseen pages' table entries
+    order = torch.randperm(2 * cols, generator=torch.Generator().manual_seed(5))
+    k, v = (torch.full((2 * cols + 1, page, 2, dim), float(x), device=device) for x in ("nan", "inf"))
+    for b, nk in enumerate(k_lens):
+        for c in range(cols):
+            pos = torch.arange(min(c * page, nk), min((c + 1) * page, nk))
+            if not seen[b][pos].any():
+                table[b, c] = poison
+                continue
+            table[b, c] = order[b * cols + c]
+            own = pos[seen[b][pos]] % page
+            for t, seed in ((k, 970), (v, 980)):
+                t[table[b, c], own.to(device)] = seeded((len(own), 2, dim), seed + 100 * b + c, torch.float32, device)
+    table = table.int()
+    q = seeded((total, 4, dim), 990, torch.float32, device)
+    got, lse = attention(q, k, v, cu_seqlens_q=cu_q, seqused_k=used, max_seqlen_q=40, max_seqlen_k=700,
+                         block_table=table.to(device), causal=True, mask_mod=spec, aux_tensors=aux, num_splits=splits)
+    clean = [t.nan_to_num(0, posinf=0) for t in (k, v)]
+    ref, ref_lse = oracle_attention(q, *clean, cu_q, used_k=used, block_table=table, causal=True, mask=spec, aux=aux)
+    assert_parity(got, lse, ref, ref_lse, out_bar=BAR)
