@@ -40,6 +40,11 @@
 //   K/V go through registers: at 16 bytes per clock and CU they leave the
 //   load path three quarters idle, and LDS tiles would only add barriers.
 //   Two accumulators for S^T instead of one chain: no change.
+// * A product with weight 0 still meets its V, so a NaN or an infinity in V
+//   reaches every row of the block.  The outputs show it: a block with one
+//   that is not finite runs its rows again one by one (f32_row), over the keys
+//   each sees, at the generic kernel's speed.  The check costs the others one
+//   barrier (2 x 1024 causal 16/8 d128 114 us with and without).
 // * Measured (generic kernel before): 2 x 1024 tokens causal, 16/8 heads,
 //   d128 4971 -> 111 us (77 TFLOP/s; 1024 workgroups for 256 CUs); decode of
 //   4 requests x 2048 keys 252 + 14 (merge) -> 16 + 4 us.
@@ -85,6 +90,67 @@ FA_DEV uint64_t shfl_u64(uint64_t x, int src) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)(uint32_t)x);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)(uint32_t)(x >> 32));
   return (uint64_t)hi << 32 | lo;
+}
+
+// One row (query row tq at position qa, head h, of KV head kh) over its keys of
+// [t0, t1), one key per lane and only the values of keys with weight, as the
+// generic kernel does: for blocks whose products met a value that is not
+// finite (0 * inf in the rows that do not see it).
+template <int DQ, int DV>
+FA_DEV void f32_row(const fa_attn_args& a, int64_t b, const RequestInfo& r, int kh, int64_t h, int64_t tq, int qa, int split,
+                    int lo, int hi, int lo2, int hi2, int t0, int t1, float scale, float slope, int lane) {
+  const float* const q = (const float*)a.q + tq * a.q_stride[0] + h * a.q_stride[1];
+  float m = a.sinks && split == 0 ? a.sinks[h * a.sink_stride] : -INFINITY, l = m > -INFINITY ? 1.0f : 0.0f;
+  constexpr int ACC = (DV + 63) / 64;
+  float acc[ACC];
+#pragma unroll
+  for (int i = 0; i < ACC; ++i) acc[i] = 0.0f;
+  for (; t0 < t1; t0 += 64) {
+    const int t = t0 + lane;
+    const bool valid = t < t1 && ((t >= lo && t < hi) || (t >= lo2 && t < hi2));
+    float s = -INFINITY;
+    if (valid) {
+      const float* const k = (const float*)a.k + kv_offset(a, a.k_stride, b, r, t, kh);
+      float dot = 0.0f;
+      for (int d = 0; d < DQ; d += 4) {
+        const f32x4 x = *(const f32x4*)(q + d), y = *(const f32x4*)(k + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dot = fmaf(x[e], y[e], dot);
+      }
+      s = dot * scale;
+      if (a.softcap > 0.0f) s = a.softcap * tanhf(s / a.softcap);
+      s -= slope * (float)abs(qa - t);
+    }
+    const float m_new = fmaxf(m, wave_max(s));
+    const float ref = m_new == -INFINITY ? 0.0f : m_new;
+    const float factor = expf(m - ref), p = valid ? expf(s - ref) : 0.0f;
+    l = l * factor + wave_sum(p);
+#pragma unroll
+    for (int i = 0; i < ACC; ++i) acc[i] *= factor;
+    const int n = min(64, t1 - t0);
+    for (int j = 0; j < n; ++j) {
+      const float pj = readlane_f(p, j);
+      if (pj == 0.0f) continue;
+      const float* const v = (const float*)a.v + kv_offset(a, a.v_stride, b, r, t0 + j, kh);
+#pragma unroll
+      for (int i = 0; i < ACC; ++i)
+        if (lane + 64 * i < DV) acc[i] = fmaf(pj, v[lane + 64 * i], acc[i]);
+    }
+    m = m_new;
+  }
+  const float norm = l > 0.0f ? descale_of(a.v_descale, a.v_descale_stride, b, kh) / l : 0.0f;
+  const float lse = l > 0.0f ? m + logf(l) : -INFINITY;
+  const int S = a.num_splits;
+#pragma unroll
+  for (int i = 0; i < ACC; ++i) {
+    const int d = lane + 64 * i;
+    if (d >= DV) continue;
+    if (S > 1) a.partial_out[((split * a.total_q + tq) * a.heads_q + h) * DV + d] = acc[i] * norm;
+    else store_any(a.out, tq * a.out_stride[0] + h * a.out_stride[1] + d * a.out_stride[2], a.out_dtype, acc[i] * norm);
+  }
+  if (lane != 0) return;
+  if (S > 1) a.partial_lse[((int64_t)split * a.heads_q + h) * a.total_q + tq] = lse;
+  else a.lse[h * a.lse_stride[0] + tq * a.lse_stride[1]] = lse;
 }
 
 // DQ, DV: the tensors' head dims (multiples of 8).  V columns past DV inside
@@ -320,10 +386,14 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
       }
       const bool edge = k0 < kbeg || k0 + F32_STAGE > kend;
       if (k0 < full_lo || k0 + F32_STAGE > full_hi || any_empty) {
+        // Bounds relative to the stage cost the fewest registers to 64 dims,
+        // absolute keys beyond (16 x 8192 keys, 16/8 heads d64 120.5 / 132.5
+        // us; 32/8 d128 204.8 / 201.9; 2 x 1024 causal 16/8 d128 115.4 / 113.2).
+        const int from = NB < 4 ? key0 : 0;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int key = 8 * (i >> 2) + (i & 3);   // from key0
-          const bool see = (key >= lo - key0 && key < hi - key0) || (MASKS && key >= lo2 - key0 && key < hi2 - key0);
+          const int key = key0 - from + 8 * (i >> 2) + (i & 3);
+          const bool see = (key >= lo - from && key < hi - from) || (MASKS && key >= lo2 - from && key < hi2 - from);
           s[i] = see ? s[i] : -INFINITY;
         }
       }
@@ -442,27 +512,64 @@ __global__ __launch_bounds__(64 * F32_WAVES, MINB) void attn_f32_kernel(const fa
   if (wave == 1) put(1);
   if (wave == 0) put(0);
   __syncthreads();
+  // O of this thread's output pieces.  One that is not finite comes from a
+  // value of the block's rows that is not (every column's sum then holds it,
+  // those that give it weight 0 as NaN) or from the row's own scores.
+  constexpr int D4 = DV / 4, PIECES = (F32_COLS * D4 + 64 * F32_WAVES - 1) / (64 * F32_WAVES);
+  f32x4 O[PIECES];
+  float probe = 0.0f;
+  auto column_row = [&](int c, int& head) {   // column c's query row, -1 without one
+    head = h0 + (c >> rl);
+    const int row = q0 + (c & (R - 1));
+    return (c >> rl) < nheads && row < r.q_len ? row : -1;
+  };
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int idx = tid + 64 * F32_WAVES * i, c = idx / D4, d = 4 * (idx - c * D4);
+    int h;
+    if (idx >= F32_COLS * D4 || column_row(c, h) < 0) continue;
+    O[i] = *(const f32x4*)(co + c * ROW + d) + *(const f32x4*)(co + (F32_COLS + c) * ROW + d);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) probe = fmaf(O[i][e], 0.0f, probe);
+  }
+  int* const flags = (int*)cm;   // every wave has read the maxima
+  if (lane == 0) flags[wave] = 0;
+  if (__any(probe != 0.0f) && lane == 0) flags[wave] = 1;
+  __syncthreads();
+  if (__builtin_expect(flags[0] | flags[1] | flags[2] | flags[3], 0)) {
+    for (int c = wave; c < F32_COLS; c += F32_WAVES) {
+      int h;
+      const int row = column_row(c, h);
+      if (row < 0) continue;
+      const float slope_c = a.alibi ? a.alibi[b * a.alibi_stride[0] + (int64_t)h * a.alibi_stride[1]] : 0.0f;
+      f32_row<DQ, DV>(a, b, r, kh, h, (int64_t)r.q_begin + row, row + r.k_len - r.q_len, split,
+                      __builtin_amdgcn_readlane(lo, c), __builtin_amdgcn_readlane(hi, c),
+                      __builtin_amdgcn_readlane(lo2, c), __builtin_amdgcn_readlane(hi2, c),
+                      max(kbeg, F32_ROUND * rb), min(kend, F32_ROUND * re), scale, slope_c, lane);
+    }
+    return;
+  }
   const float lse = L > 0.0f ? M * LN2 + logf(L) : -INFINITY;
   if (wave == 0 && hh == 0 && col_ok) {
     if (S > 1) a.partial_lse[((int64_t)split * a.heads_q + hq) * a.total_q + tq] = lse;
     else a.lse[hq * a.lse_stride[0] + tq * a.lse_stride[1]] = lse;
   }
-  constexpr int D4 = DV / 4;
-  for (int idx = tid; idx < F32_COLS * D4; idx += 64 * F32_WAVES) {
-    const int c = idx / D4, d = 4 * (idx - c * D4);
-    const int ch = c >> rl, cr = q0 + (c & (R - 1));
-    if (ch >= nheads || cr >= r.q_len) continue;
-    const f32x4 O = *(const f32x4*)(co + c * ROW + d) + *(const f32x4*)(co + (F32_COLS + c) * ROW + d);
-    const int64_t t = (int64_t)r.q_begin + cr, h = h0 + ch;
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int idx = tid + 64 * F32_WAVES * i, c = idx / D4, d = 4 * (idx - c * D4);
+    int head;
+    const int row = idx < F32_COLS * D4 ? column_row(c, head) : -1;
+    if (row < 0) continue;
+    const int64_t t = (int64_t)r.q_begin + row, h = head;
     if (S > 1) {   // partials [S][T][Hq][Dv], LSEs [S][Hq][T], as the generic kernel's
-      *(f32x4*)(a.partial_out + ((split * a.total_q + t) * a.heads_q + h) * DV + d) = O;
+      *(f32x4*)(a.partial_out + ((split * a.total_q + t) * a.heads_q + h) * DV + d) = O[i];
     } else {
       const int64_t off = t * a.out_stride[0] + h * a.out_stride[1] + (int64_t)d * a.out_stride[2];
       if (shp.vec_out) {
-        *(f32x4*)((float*)a.out + off) = O;
+        *(f32x4*)((float*)a.out + off) = O[i];
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) store_any(a.out, off + e * a.out_stride[2], a.out_dtype, O[e]);
+        for (int e = 0; e < 4; ++e) store_any(a.out, off + e * a.out_stride[2], a.out_dtype, O[i][e]);
       }
     }
   }
@@ -475,7 +582,7 @@ struct F32Choice {
 };
 
 // Workgroups per CU (waves per SIMD): 168 registers at three (d128 spills
-// 14), 128 at four; d256 holds 128 for O^T alone and runs one.
+// 13), 128 at four; d256 holds 128 for O^T alone and runs one.
 template <int DQ, int DV, int MINB> F32Choice f32_choice(bool masks) {
   return F32Choice{masks ? attn_f32_kernel<DQ, DV, MINB, true> : attn_f32_kernel<DQ, DV, MINB, false>,
                    f32_lds_bytes<DQ, DV>()};

@@ -168,3 +168,49 @@ def test_masked_keys_that_no_row_sees(device, mask, splits, dim):
     clean = [t.nan_to_num(0, posinf=0) for t in (k, v)]
     ref, ref_lse = oracle_attention(q, *clean, cu_q, used_k=used, block_table=table, causal=True, mask=spec, aux=aux)
     assert_parity(got, lse, ref, ref_lse, out_bar=BAR)
+
+
+@pytest.mark.parametrize("dq,dv", [(32, 32), (64, 64), (72, 72), (128, 128), (192, 128), (256, 256)])
+@pytest.mark.parametrize("case", ["causal", "window", "rows2", "clamped", "splits"])
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(device, dq, dv, case):
+    """A NaN and infinities in V at keys that only some rows of a 32-row block
+    see: those rows show them in their dims, the others and the other dims
+    nothing of them."""
+    q_lens, k_lens = ([2, 2], [300, 131]) if case == "rows2" else ([40, 70], [45, 260])
+    q, k, v, cu_q, cu_k = _packed(device, q_lens, k_lens, 6, 2, dq, dv, 995)
+    total, last = sum(q_lens), max(q_lens)
+    kw = dict(causal=True, num_splits=3 if case == "splits" else 1)
+    if case == "window":
+        kw.update(window_size=(9, 0))
+    elif case == "clamped":
+        ranges = torch.full((total, 2), -1, dtype=torch.int32)
+        ranges[7] = torch.tensor([20, 44], dtype=torch.int32)
+        kw.update(mask_mod=vllm.mm_prefix_mask(15), aux_tensors=[ranges.to(device), cu_q])
+    names = dict(window_size="window", mask_mod="mask", aux_tensors="aux")
+    ref, ref_lse = oracle_attention(q, k, v, cu_q, cu_k, **{names.get(n, n): x for n, x in kw.items() if n != "num_splits"})
+    # (key from the request's end, dim, value); NaN in KV head 0 only.
+    poison = [(1, 3, float("nan"), 0), (1, 5, float("inf"), None), (1 + last // 2, 9, float("-inf"), None)]
+    bad = torch.zeros(total, 6, dv, dtype=torch.bool)
+    weight = {}
+    for back, dim, value, head in poison:
+        probe = torch.zeros_like(v)
+        for end in cu_k[1:].tolist():
+            probe[end - back, slice(None) if head is None else head, dim] = 1.0
+        weight[dim], _ = oracle_attention(q, k, probe, cu_q, cu_k, **{names.get(n, n): x for n, x in kw.items() if n != "num_splits"})
+        bad[weight[dim] > 0] = True
+        for end in cu_k[1:].tolist():
+            v[end - back, slice(None) if head is None else head, dim] = value
+    assert bad.any() and not bad[..., 3].all() and not bad[..., 7].any()
+    got, lse = attention(q, k, v, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=last, max_seqlen_k=max(k_lens), **kw)
+    got = got.cpu()
+    assert torch.equal(~got.isfinite(), bad)
+    assert got[..., 3][bad[..., 3]].isnan().all() and (got[..., 5][bad[..., 5]] == float("inf")).all()
+    assert (got[..., 9][bad[..., 9]] == float("-inf")).all()
+    # The clean reference, without the poisoned keys' dims.
+    untouched = torch.ones(dv, dtype=torch.bool)
+    untouched[[3, 5, 9]] = False
+    assert_parity(got[..., untouched], lse, ref[..., untouched], ref_lse, torch.float32, out_bar=BAR)
+    clean = torch.where(bad, torch.zeros((), dtype=torch.float64), ref)
+    for _, dim, _, head in poison:   # rows without weight on a poisoned key: as with any finite value there
+        rows = ~bad[..., dim]
+        assert (got[..., dim][rows].double() - clean[..., dim][rows]).abs().max() <= BAR if rows.any() else True
