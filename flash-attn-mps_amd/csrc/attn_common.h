@@ -78,6 +78,10 @@ inline fa_attn_args fa_bounded(const fa_attn_args& args) {
 // Host-side argument checks shared by fa_attn_fwd / fa_decode_fwd / fa_prefill_fwd.
 int fa_validate_attn(const fa_attn_args* a, const char* who);
 
+// fa_merge_partials for the splits of one call: a NaN LSE makes the row NaN,
+// with LSE -inf, as one split would (fp32 rows over at most 256 dims).
+int fa_merge_splits(const fa_merge_partials_args* a, void* stream);
+
 // The fp32 matrix-core kernel (attn_f32.hip): whether it takes these
 // (validated) arguments, and its launch with fa_attn_fwd's split partials.
 bool fa_f32_supported(const fa_attn_args& a);

@@ -139,8 +139,9 @@ FA_DEV void f32_row(const fa_attn_args& a, int64_t b, const RequestInfo& r, int 
     m = m_new;
   }
   const float norm = l > 0.0f ? descale_of(a.v_descale, a.v_descale_stride, b, kh) / l : 0.0f;
-  const float lse = l > 0.0f ? m + logf(l) : -INFINITY;
   const int S = a.num_splits;
+  // A NaN sum is no split without keys: its LSE is NaN for the merge.
+  const float lse = l > 0.0f || (S > 1 && l != 0.0f) ? m + logf(l) : -INFINITY;
 #pragma unroll
   for (int i = 0; i < ACC; ++i) {
     const int d = lane + 64 * i;

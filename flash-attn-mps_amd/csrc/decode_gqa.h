@@ -619,7 +619,8 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
     const float norm = L > 0.0f ? vdsc / L : 0.0f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) cm[w * GQA_HEADS + tid] = fw[w] * norm;
-    cl[tid] = L > 0.0f ? M * LN2 + logf(L) : -INFINITY;
+    // E4M3 queries: a split's NaN sum gives a NaN LSE, which the merge keeps.
+    cl[tid] = L > 0.0f || (QF8 && S > 1 && L != 0.0f) ? M * LN2 + logf(L) : -INFINITY;
   }
   __syncthreads();
   // hc / ntok for hc < 32 and 1 <= ntok <= 16 as a multiply by

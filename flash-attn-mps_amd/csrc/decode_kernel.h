@@ -729,7 +729,9 @@ __global__ __launch_bounds__(DEC_THREADS, FA_DEC_MINB) void decode_kernel(const 
       O += sm_acc[w][g][d] * f;
     }
     const float norm = L > 0.0f ? vscale[half_of(g)] / L : 0.0f;
-    const float lse = L > 0.0f ? M * LN2 + logf(L) : -INFINITY;
+    // E4M3 queries: a split's NaN sum gives a NaN LSE, which the merge keeps.
+    const bool keep_nan = CT::id == FA_F16 && KT::id == FA_E4M3 && a.q_dtype == FA_E4M3 && S > 1;
+    const float lse = L > 0.0f || (keep_nan && L != 0.0f) ? M * LN2 + logf(L) : -INFINITY;
     const int h = h0 + g;
     if (S == 1) {
       store_any(a.out, tq * a.out_stride[0] + (int64_t)h * a.out_stride[1] + (int64_t)d * a.out_stride[2], a.out_dtype,

@@ -52,7 +52,9 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const fa_attn_args a,
   const float* plse = a.partial_lse + row * S;
   const float* po = a.partial_out + (b * S * rows_b + (row - b * rows_b)) * DV;
   // A zero-weight split (empty, its partial never written) is read like the
-  // others but dropped by a select, so its contents never reach the sum.
+  // others but dropped by a select, so its contents never reach the sum.  A NaN
+  // LSE (E4M3 queries: a split whose sum is NaN) makes the row NaN with LSE
+  // -inf, as one split would.
   float x0[GROUP][DIMS];
 #pragma unroll
   for (int u = 0; u < GROUP; ++u)
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const fa_attn_args a,
   for (int u = 0; u < GROUP; ++u) {
     const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u));
 #pragma unroll
-    for (int k = 0; k < DIMS; ++k) acc[k] = ws > 0.0f ? fmaf(ws, x0[u][k], acc[k]) : acc[k];
+    for (int k = 0; k < DIMS; ++k) acc[k] = ws != 0.0f ? fmaf(ws, x0[u][k], acc[k]) : acc[k];
   }
   for (int s0 = 0; s0 < nv; s0 += 64) {
     if (s0) {
@@ -94,11 +96,11 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const fa_attn_args a,
 #pragma unroll
       for (int u = 0; u < GROUP; ++u)
 #pragma unroll
-        for (int k = 0; k < DIMS; ++k) acc[k] = ws[u] > 0.0f ? fmaf(ws[u], x[u][k], acc[k]) : acc[k];
+        for (int k = 0; k < DIMS; ++k) acc[k] = ws[u] != 0.0f ? fmaf(ws[u], x[u][k], acc[k]) : acc[k];
     }
     for (; j < cnt; ++j) {
       const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
-      if (ws > 0.0f) {   // zero-weight splits are never read
+      if (ws != 0.0f) {   // zero-weight splits are never read
         const float* src = po + (int64_t)(s0 + j) * pitch;
 #pragma unroll
         for (int k = 0; k < DIMS; ++k)

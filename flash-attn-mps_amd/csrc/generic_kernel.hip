@@ -192,5 +192,5 @@ extern "C" int fa_attn_fwd(const fa_attn_args* args, void* stream) {
   m.partial_lse_stride[2] = 1;
   for (int i = 0; i < 3; ++i) m.out_stride[i] = a->out_stride[i];
   for (int i = 0; i < 2; ++i) m.lse_stride[i] = a->lse_stride[i];
-  return fa_merge_partials(&m, stream);
+  return fa_merge_splits(&m, stream);
 }

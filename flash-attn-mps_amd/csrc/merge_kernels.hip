@@ -11,7 +11,7 @@
 // In-place merging (out or out_lse aliasing an input) is safe: each element
 // is read and written by the same lane, and the LSE inputs are read by the
 // whole wave before lane 0 writes the merged LSE.
-#include "fa_device.h"
+#include "attn_common.h"
 
 namespace {
 
@@ -62,6 +62,7 @@ struct MergePartialsParams {
   int64_t splits, tokens, heads, dim;
   int64_t ps[4], pls[3], os[3], ls[2];
   int32_t part_dtype, out_dtype;
+  bool splits_of_call;   // fa_merge_splits
 };
 
 __global__ __launch_bounds__(256) void merge_partials_kernel(const MergePartialsParams p) {
@@ -92,7 +93,8 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(const MergePartials
 // weights once per wave (split s0 + j on lane j, broadcast with readlane)
 // and GROUP partial rows in flight, where the kernel above recomputes every
 // weight from memory for each 64 dims and waits for one row at a time.
-// Splits are added in order.
+// Splits are added in order.  In a merge of one call's splits a NaN LSE (the
+// split's sum is NaN) keeps its NaN weight.
 template <int DIMS, int GROUP>
 __global__ __launch_bounds__(256) void merge_rows_kernel(const MergePartialsParams p) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const MergePartialsPara
   const float* const lse = p.plse + h * p.pls[1] + t * p.pls[2];
   const float* const part = (const float*)p.part + t * p.ps[1] + h * p.ps[2];
   const float lse0 = lane < S ? lse[lane * p.pls[0]] : -INFINITY;
-  float peak = lse0;
+  float peak = fmaxf(lse0, -INFINITY);   // never NaN
   for (int s = lane + 64; s < S; s += 64) peak = fmaxf(peak, lse[s * p.pls[0]]);
   peak = wave_max(peak);
   float acc[DIMS], denom = 0.0f;
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const MergePartialsPara
   for (int k = 0; k < DIMS; ++k) acc[k] = 0.0f;
   for (int s0 = 0; s0 < S; s0 += 64) {
     const float l = s0 == 0 ? lse0 : s0 + lane < S ? lse[(s0 + lane) * p.pls[0]] : -INFINITY;
-    const float w = merge_weight(l, peak);
+    const float w = p.splits_of_call && l != l ? l : merge_weight(l, peak);
     denom += w;
     const int cnt = min(64, S - s0);
     for (int j = 0; j < cnt; j += GROUP) {
@@ -125,19 +127,20 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const MergePartialsPara
       for (int u = 0; u < GROUP; ++u) {
         const float ws = j + u < cnt ? readlane_f(w, j + u) : 0.0f;
 #pragma unroll
-        for (int k = 0; k < DIMS; ++k) acc[k] = ws > 0.0f ? fmaf(ws, x[u][k], acc[k]) : acc[k];
+        for (int k = 0; k < DIMS; ++k) acc[k] = ws != 0.0f ? fmaf(ws, x[u][k], acc[k]) : acc[k];
       }
     }
   }
   denom = wave_sum(denom);
-  const bool empty = peak == -INFINITY;
+  const bool empty = peak == -INFINITY && denom == 0.0f;
 #pragma unroll
   for (int k = 0; k < DIMS; ++k) {
     const int d = lane + 64 * k;
     if (d < dim)
       store_any(p.out, t * p.os[0] + h * p.os[1] + d * p.os[2], p.out_dtype, empty ? 0.0f : acc[k] / denom);
   }
-  if (lane == 0) p.lse[h * p.ls[0] + t * p.ls[1]] = empty ? -INFINITY : peak + logf(denom);
+  if (lane == 0)
+    p.lse[h * p.ls[0] + t * p.ls[1]] = empty || (p.splits_of_call && denom != denom) ? -INFINITY : peak + logf(denom);
 }
 
 }  // namespace
@@ -164,7 +167,9 @@ extern "C" int fa_merge_pair(const fa_merge_pair_args* a, void* stream) {
   return fa_check_launch("fa_merge_pair");
 }
 
-extern "C" int fa_merge_partials(const fa_merge_partials_args* a, void* stream) {
+namespace {
+
+int merge_partials(const fa_merge_partials_args* a, void* stream, bool splits_of_call) {
   FA_REQUIRE(a && a->out && a->lse && (a->splits == 0 || (a->partial && a->partial_lse)),
              "fa_merge_partials: null argument");
   FA_REQUIRE(a->out_dtype == FA_F16 || a->out_dtype == FA_BF16 || a->out_dtype == FA_F32,
@@ -178,6 +183,7 @@ extern "C" int fa_merge_partials(const fa_merge_partials_args* a, void* stream) 
   for (int i = 0; i < 3; ++i) { p.pls[i] = a->partial_lse_stride[i]; p.os[i] = a->out_stride[i]; }
   for (int i = 0; i < 2; ++i) p.ls[i] = a->lse_stride[i];
   p.part_dtype = a->partial_dtype; p.out_dtype = a->out_dtype;
+  p.splits_of_call = splits_of_call;
   const int64_t rows = p.tokens * p.heads;
   if (rows == 0) return FA_OK;
   FA_REQUIRE(fa_ceil_div(rows, 4) <= 0x7fffffffll, "fa_merge_partials: too many rows");
@@ -187,3 +193,11 @@ extern "C" int fa_merge_partials(const fa_merge_partials_args* a, void* stream) 
   hipLaunchKernelGGL(kern, dim3((unsigned)fa_ceil_div(rows, 4)), dim3(256), 0, (hipStream_t)stream, p);   // a wave per row
   return fa_check_launch("fa_merge_partials");
 }
+
+}  // namespace
+
+extern "C" int fa_merge_partials(const fa_merge_partials_args* a, void* stream) {
+  return merge_partials(a, stream, false);
+}
+
+int fa_merge_splits(const fa_merge_partials_args* a, void* stream) { return merge_partials(a, stream, true); }

@@ -1349,7 +1349,8 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
       const float inv = lt > 0.0f ? vdsc / lt : 0.0f;
       const int64_t tq = (int64_t)r.q_begin + row;
       if constexpr (SPLIT) {
-        // Partials [S][T][Hq][Dv] (normalised), LSEs [S][Hq][T].
+        // Partials [S][T][Hq][Dv] (normalised), LSEs [S][Hq][T] (NaN where
+        // the sum is: the merge must not take that for a split without keys).
         const int64_t dv = TWO_PARTS ? 2 * DVT : DVT;
         float* pp = a.partial_out + ((split * a.total_q + tq) * a.heads_q + h) * dv + (TWO_PARTS ? vpart * DVT : 0) + 4 * hh;
 #pragma unroll
@@ -1360,7 +1361,7 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
                                                       o[nb][db][4 * g + 2] * inv, o[nb][db][4 * g + 3] * inv};
         if (hh == 0 && (!TWO_PARTS || vpart == 0))
           a.partial_lse[((int64_t)split * a.heads_q + h) * a.total_q + tq] =
-              lt > 0.0f ? m_run[nb] * LN2 + logf(lt) : -INFINITY;
+              lt == 0.0f ? -INFINITY : m_run[nb] * LN2 + logf(lt);
         continue;
       }
       uint16_t* op = (uint16_t*)a.out + tq * a.out_stride[0] + (int64_t)h * a.out_stride[1] + (TWO_PARTS ? vpart * DVT : 0) + 4 * hh;

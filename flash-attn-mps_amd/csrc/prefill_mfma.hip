@@ -52,7 +52,8 @@ bool split_ok(const fa_attn_args& a) {
 // Merge of the split partials: one wave per (request, row, head) row, split
 // weights on lanes, GROUP partial rows in flight; DIMS dims per lane.  The
 // rows of single-query requests under FA_FLAG_SKIP_SINGLE_QUERY are the
-// decode kernel's and stay untouched.
+// decode kernel's and stay untouched.  A split whose LSE is NaN makes the row
+// NaN, with LSE -inf, as one split would.
 template <int DIMS, int GROUP>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const fa_attn_args a) {
   const int lane = threadIdx.x & 63, S = a.num_splits, DV = (int)a.head_dim_v;
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const fa_attn_args a
     for (int u = 0; u < GROUP; ++u) {
       const float ws = s0 + u < S ? readlane_f(w, s0 + u) : 0.0f;
 #pragma unroll
-      for (int k = 0; k < DIMS; ++k) acc[k] = ws > 0.0f ? fmaf(ws, x[u][k], acc[k]) : acc[k];
+      for (int k = 0; k < DIMS; ++k) acc[k] = ws != 0.0f ? fmaf(ws, x[u][k], acc[k]) : acc[k];
     }
   }
   const float denom = wave_sum(w), inv = denom > 0.0f ? 1.0f / denom : 0.0f;
