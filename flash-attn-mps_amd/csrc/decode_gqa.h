@@ -35,10 +35,10 @@
 //   XOR-swizzled); K operands are widened in registers after 8-byte reads,
 //   V^T comes through ds_read_b64_tr_b8 and is widened the same way.
 // * Supports 16-bit queries over K/V of their type or E4M3 (with descales),
-//   E4M3 queries over E4M3 K/V (one row per request), head dims 64 and 128 (Dqk = Dv), outputs of the query's type, packed or
-//   paged K/V (page size a multiple of 16), sinks, softcap, windows, 1-16
-//   query rows per request; the host keeps other combinations on the VALU
-//   kernel.  Neighbouring KV heads (64-dim, or 128-dim E4M3) can run in
+//   E4M3 queries over E4M3 K/V (one row per request), head dims 64 and 128
+//   (Dqk = Dv), outputs of the query's type, packed or paged K/V (page size
+//   a multiple of 16), sinks, softcap, windows, 1-16 query rows per request;
+//   the host keeps other combinations on the VALU kernel.  Neighbouring KV heads (64-dim, or 128-dim E4M3) can run in
 //   pairs whose rows the slots hold as one row (PACK below), so that each
 //   DMA instruction reads runs of two head rows.
 #ifndef FA_DECODE_GQA_H
@@ -68,7 +68,7 @@ template <int D, bool FP8> constexpr int gqa_slot_bytes() { return FP8 ? 32 * D 
 template <int D, bool FP8, int PACK> constexpr int gqa_slots() { return FP8 && PACK == 1 ? 4 : 2; }
 template <int D, bool FP8, int PACK> constexpr int gqa_lds_bytes() {
   const int ring = 4 * gqa_slots<D, FP8, PACK>() * gqa_slot_bytes<D, FP8>();
-  const int combine = 4 * GQA_HEADS * (D / PACK + 4 + 2) * 4;
+  const int combine = 4 * GQA_HEADS * (D / PACK + 4 + 2) * 4 + 16;   // rows, maxima and sums; four flags
   return ring > combine ? ring : combine;
 }
 
@@ -108,6 +108,57 @@ FA_DEV void wait_dma_groups(int n) {
     if (n >= MAXN) wait_dma_older_than<MAXN * PER>();
     else wait_dma_groups<PER, MAXN - 1>(n);
   }
+}
+
+// One head's row over keys [t0, t1) (E4M3 queries, keys and values), one key
+// per lane and only its own KV head's rows, as the generic kernel does: for
+// workgroups of paired heads whose sums met a NaN, which the zero queries and
+// probabilities of the other head's half do not hide (0 * NaN).
+template <int D>
+FA_DEV void e4m3_row(const fa_attn_args& a, int64_t b, const RequestInfo& r, int kh, int h, int split, int t0, int t1,
+                     float scale, int lane) {
+  const int64_t tq = r.q_begin, S = a.num_splits;
+  const int64_t q0 = tq * a.q_stride[0] + (int64_t)h * a.q_stride[1];
+  float m = a.sinks && split == 0 ? a.sinks[(int64_t)h * a.sink_stride] : -INFINITY, l = m > -INFINITY ? 1.0f : 0.0f;
+  constexpr int ACC = D / 64;
+  float acc[ACC];
+#pragma unroll
+  for (int i = 0; i < ACC; ++i) acc[i] = 0.0f;
+  for (; t0 < t1; t0 += 64) {
+    const bool valid = t0 + lane < t1;
+    float s = -INFINITY;
+    if (valid) {
+      const int64_t k0 = kv_offset(a, a.k_stride, b, r, t0 + lane, kh);
+      float dot = 0.0f;
+      for (int d = 0; d < D; ++d) dot = fmaf(load_elem<E4M3T>(a.q, q0 + d), load_elem<E4M3T>(a.k, k0 + d), dot);
+      s = dot * scale;
+      if (a.softcap > 0.0f) s = a.softcap * tanhf(s / a.softcap);
+    }
+    const float m_new = fmaxf(m, wave_max(s)), ref = m_new == -INFINITY ? 0.0f : m_new;
+    const float factor = expf(m - ref), p = valid ? expf(s - ref) : 0.0f;
+    l = l * factor + wave_sum(p);
+#pragma unroll
+    for (int i = 0; i < ACC; ++i) acc[i] *= factor;
+    for (int j = 0; j < min(64, t1 - t0); ++j) {
+      const float pj = readlane_f(p, j);
+      if (pj == 0.0f) continue;
+      const int64_t v0 = kv_offset(a, a.v_stride, b, r, t0 + j, kh);
+#pragma unroll
+      for (int i = 0; i < ACC; ++i) acc[i] = fmaf(pj, load_elem<E4M3T>(a.v, v0 + lane + 64 * i), acc[i]);
+    }
+    m = m_new;
+  }
+  const float norm = l > 0.0f ? descale_of(a.v_descale, a.v_descale_stride, b, kh) / l : 0.0f;
+  const float lse = l > 0.0f || (S > 1 && l != 0.0f) ? m + logf(l) : -INFINITY;
+#pragma unroll
+  for (int i = 0; i < ACC; ++i) {
+    const int d = lane + 64 * i;
+    if (S > 1) a.partial_out[((b * S + split) * a.heads_q + h) * D + d] = acc[i] * norm;
+    else store_any(a.out, tq * a.out_stride[0] + (int64_t)h * a.out_stride[1] + d * a.out_stride[2], a.out_dtype, acc[i] * norm);
+  }
+  if (lane != 0) return;
+  if (S > 1) a.partial_lse[(b * a.heads_q + h) * S + split] = lse;
+  else a.lse[(int64_t)h * a.lse_stride[0] + tq * a.lse_stride[1]] = lse;
 }
 
 // KT: K/V storage type, T or E4M3.  E4M3 slots hold the raw K rows (16 rows
@@ -583,10 +634,21 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
   __syncthreads();
   float* const cm = (float*)smem;                      // [4][32]
   float* const cl = cm + 4 * GQA_HEADS;                // [4][32]
+  constexpr bool PROBE = QF8 && PACK > 1;   // [4]: whether a wave's sums are all finite
+  int* const finite = (int*)(cl + 4 * GQA_HEADS);
   // [4][32][DH + 4]: the 4-float pad puts the 32 head columns' 16-byte
   // stores of one instruction on distinct bank groups.
   constexpr int CO_ROW = DH + 4;
-  float* const co = cl + 4 * GQA_HEADS;
+  float* const co = cl + 4 * GQA_HEADS + (PROBE ? 4 : 0);
+  if constexpr (PROBE) {
+    float probe = lt * 0.0f;
+#pragma unroll
+    for (int db = 0; db < DBH; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) probe = fmaf(o[db][i], 0.0f, probe);
+    const bool ok = __all(probe == 0.0f);
+    if (lane == 0) finite[wave] = ok;
+  }
   if (hh == 0) {
     cm[wave * GQA_HEADS + l32] = m_run;
     cl[wave * GQA_HEADS + l32] = lt;
@@ -599,6 +661,17 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
       *(float4*)(co + ((int64_t)wave * GQA_HEADS + l32) * CO_ROW + 32 * db + 8 * g + 4 * hh) =
           float4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
   __syncthreads();
+  if constexpr (PROBE) {
+    if (__builtin_expect(!(finite[0] & finite[1] & finite[2] & finite[3]), 0)) {
+      for (int c = wave; c < nheads; c += 4) {
+        const int own = PACK * kh + part_of(c);
+        const float sc = a.softmax_scale * descale_of(a.q_descale, a.q_descale_stride, b, own) *
+                         descale_of(a.k_descale, a.k_descale_stride, b, own);
+        e4m3_row<DH>(a, b, r, own, h0 + c, split, begin, end, sc, lane);
+      }
+      return;
+    }
+  }
   // Per column, once: the combined max, the four waves' weights times the
   // output scale (written over cm) and the LSE (over cl's first row).  Each
   // column belongs to one thread here, which reads all its entries before

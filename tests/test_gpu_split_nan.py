@@ -68,7 +68,8 @@ def test_rows_of_a_chunk(device, monkeypatch, qt, kt, dq, dv, splits):
     _check(got, lse, ref, ref_lse, bad, 1e-4 if qt == torch.float32 else None)
 
 
-@pytest.mark.parametrize("heads,kv_heads,dim", [(12, 3, 128), (4, 4, 128), (4, 4, 256), (12, 3, 64)])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(12, 3, 128), (4, 4, 128), (4, 4, 256), (12, 3, 64),
+                                                (16, 2, 128), (16, 4, 64), (16, 8, 128), (16, 16, 64)])
 @pytest.mark.parametrize("mixed,splits", [(True, 0), (True, 1), (False, 0), (False, 1), (False, 3)])
 def test_single_rows_of_e4m3_queries(device, heads, kv_heads, dim, mixed, splits):
     """Alone and beside a 40-row request; matrix-core and VALU decode."""
@@ -109,3 +110,27 @@ def test_merge_of_caller_states_with_nan_lse(device, splits, dim):
     assert (out[2, 1] == 0).all() and torch.isneginf(lse[1, 2])
     assert (out[1, 0] == 0).all() and torch.isneginf(lse[0, 1])
     assert out[0, 1].isfinite().all() and out[2, 0].isfinite().all()
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 2, 128), (64, 4, 128), (16, 4, 64), (16, 16, 64), (16, 8, 128)])
+@pytest.mark.parametrize("head", [0, 1])
+@pytest.mark.parametrize("splits", [0, 1])
+def test_a_nan_in_one_kv_head_stays_with_its_queries(device, heads, kv_heads, dim, head, splits):
+    """E4M3 queries over neighbouring KV heads that run in pairs: a NaN in V
+    (one dim) and in K (another request) of either head of a pair."""
+    k_lens = [300, 131, 700]
+    k, v = (_values((sum(k_lens), kv_heads, dim), s, E4M3, device) for s in (2, 3))
+    q = _values((3, heads, dim), 4, E4M3, device)
+    cu, cu_k = offsets([1, 1, 1], device), offsets(k_lens, device)
+    ref, ref_lse = oracle_attention(q.float(), k.float(), v.float(), cu, cu_k, causal=True)
+    v = _poison(v, (77, head, 9))
+    k = _poison(k, (300 + 100, head, 1))
+    got, lse = attention(q, k, v, cu_seqlens_q=cu, cu_seqlens_k=cu_k, max_seqlen_q=1, max_seqlen_k=700, causal=True,
+                         num_splits=splits)
+    group = heads // kv_heads
+    own = slice(head * group, (head + 1) * group)
+    assert got[0, own, 9].isnan().all()
+    got[0, own, 9] = ref[0, own, 9].to(got)
+    bad = torch.zeros(3, heads, dtype=torch.bool)
+    bad[1, own] = True
+    _check(got, lse, ref, ref_lse, bad)
