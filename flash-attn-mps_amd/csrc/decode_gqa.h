@@ -178,14 +178,17 @@ FA_DEV void e4m3_row(const fa_attn_args& a, int64_t b, const RequestInfo& r, int
 // with each column's probabilities zeroed for the other head's half, so
 // every column accumulates only its own head's values.  Descales are per
 // column (its KV head).
-// QF8: E4M3 queries (with E4M3 K/V, T = fp16, which holds both exactly).
-// Probabilities then stay at fp32 accuracy, as in the kernels that compute
-// them on the VALU: P = hi + lo, two fp16 values (22 bits; the remainder is
-// below 2^-24 of the largest), and P.V runs on both.  The matrix cores have
-// the room: 24 MFMAs a stage at d128 are 768 cycles per 8 KiB and SIMD, four
-// times the rate HBM delivers.
+// QF8: E4M3 queries (with E4M3 K/V, T = bf16, which holds both exactly).
+// Probabilities then stay in fp32, as in the kernels that compute them on the
+// VALU: P is the sum of three bf16 values (8 bits each and fp32's exponents,
+// so the sum is exact) and P.V runs on all three; the softcap is
+// fp32's too (softcap_rel).  The matrix cores have the room: 32 MFMAs a stage at d128 are 1024 cycles per 8
+// KiB and SIMD, three times the rate HBM delivers.  Against
+// two fp16 terms, which drop what lies 2^25 below the running maximum: 32 x
+// 8192 keys 32/8 d128 105.8 -> 110.4 us a call, 64 x 16384 64/8 366.6 -> 370.5.
+// Two waves per SIMD are asked for, which the softcap variants would lose.
 template <typename T, int D, bool CAP, typename KT = T, int PACK = 1, bool QF8 = false>
-__global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_attn_args a, const int span) {
+__global__ __launch_bounds__(GQA_THREADS, QF8 ? 2 : 1) void decode_gqa_kernel(const fa_attn_args a, const int span) {
   static_assert(D == 64 || D == 128 || D == 256, "rows of 64, 128 or 256 elements");
   static_assert((PACK == 1 && D <= 128) || (PACK == 2 && (D == 128 || (D == 256 && KT::id == FA_E4M3))),
                 "paired heads: 64-dim heads, or 128-dim E4M3 heads");
@@ -201,8 +204,8 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
   constexpr int KBYTES = KG * KGROUP, SLOT = gqa_slot_bytes<D, FP8>(), NSLOT = gqa_slots<D, FP8, PACK>();
   static_assert(NSLOT >= 2, "a stage's two slots");
   constexpr bool RING2 = NSLOT == 4;      // slots hold two stages (E4M3, unpaired)
-  static_assert(!QF8 || (FP8 && T::id == FA_F16), "E4M3 queries: E4M3 K/V, fp16 products");
-  constexpr int PT = QF8 ? 2 : 1;         // 16-bit terms of a probability
+  static_assert(!QF8 || (FP8 && T::id == FA_BF16), "E4M3 queries: E4M3 K/V, bf16 products");
+  constexpr int PT = QF8 ? 3 : 1;         // 16-bit terms of a probability
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
@@ -275,7 +278,7 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
   const int ckh = PACK * kh + cpart;
   const float kdsc = descale_of(a.q_descale, a.q_descale_stride, b, ckh) * descale_of(a.k_descale, a.k_descale_stride, b, ckh);
   const float c_scale = a.softmax_scale * kdsc * LOG2E;   // raw dot -> log2 units
-  const float cap_in = CAP ? 2.0f * LOG2E * a.softmax_scale * kdsc / a.softcap : 0.0f;
+  const float cap_in = CAP ? (QF8 ? 1.0f : 2.0f * LOG2E) * a.softmax_scale * kdsc / a.softcap : 0.0f;
   const float cap_out = a.softcap * LOG2E;
   // A sink logit seeds the state of one wave of split 0 (max = sink, sum = 1).
   const bool seed = a.sinks && split == 0 && wave == 0;
@@ -526,12 +529,23 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
     }
     // s[e] = score of storage position st_pos(i) + 16 (e >> 3) + 8 hh + (e & 7).
     const int p0 = st_pos(i) + 8 * hh;
+    if constexpr (CAP && QF8) {
+      auto each = [&](auto f) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          float x = s[e];
+          f(x);
+          s[e] = x;
+        }
+      };
+      fa_decode::softcap_rel(each, cap_in, cap_out);
+    }
     float mx = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       float v = s[e];
-      if constexpr (CAP) v = cap_out * (1.0f - 2.0f * __builtin_amdgcn_rcpf(fast_exp2(cap_in * v) + 1.0f));
-      else v *= c_scale;
+      if constexpr (CAP && !QF8) v = cap_out * (1.0f - 2.0f * __builtin_amdgcn_rcpf(fast_exp2(cap_in * v) + 1.0f));
+      else if constexpr (!CAP) v *= c_scale;
       const int pos = p0 + 16 * (e >> 3) + (e & 7);
       v = (pos >= col_lo && pos < col_hi) ? v : -INFINITY;
       s[e] = v;
@@ -576,8 +590,8 @@ __global__ __launch_bounds__(GQA_THREADS, 1) void decode_gqa_kernel(const fa_att
 #pragma unroll
           for (int u = 0; u < PACK; ++u) pop[u][c][t][q] = PACK == 1 || cpart == u ? w : 0u;
           if constexpr (QF8) {
-            x -= f16_bits_to_f32(w & 0xffffu);
-            y -= f16_bits_to_f32(w >> 16);
+            x -= bf16_bits_to_f32(w & 0xffffu);
+            y -= bf16_bits_to_f32(w >> 16);
           }
         }
       }

@@ -83,7 +83,7 @@ GqaChoice pick_decode_gqa(const fa_attn_args& a) {
     return none;
   // P.V runs on probabilities rounded to the query's type: fp32 outputs
   // (held to fp32 accuracy) take the VALU kernel, which keeps P in fp32.
-  // E4M3 queries (P as two fp16 terms) write either 16-bit type; their
+  // E4M3 queries (P as three bf16 terms) write either 16-bit type; their
   // multi-row calls run as prefill.
   const bool fp8q = a.q_dtype == FA_E4M3;
   if (fp8q) {
@@ -102,7 +102,7 @@ GqaChoice pick_decode_gqa(const fa_attn_args& a) {
   for (int i = 0; i < 2; ++i)
     if (a.k_stride[i] * kvb >= (1ll << 31) / 16 || a.v_stride[i] * kvb >= (1ll << 31) / 16) return none;
   const bool cap = a.softcap > 0.0f, fp8 = a.k_dtype == FA_E4M3;
-  if (fp8q) return choose_dim<F16T, E4M3T, true>(a, cap);
+  if (fp8q) return choose_dim<BF16T, E4M3T, true>(a, cap);
   if (a.q_dtype == FA_BF16) return fp8 ? choose_dim<BF16T, E4M3T>(a, cap) : choose_dim<BF16T, BF16T>(a, cap);
   return fp8 ? choose_dim<F16T, E4M3T>(a, cap) : choose_dim<F16T, F16T>(a, cap);
 }

@@ -195,6 +195,41 @@ FA_DEV uint32_t pack_pair_bits(float lo, float hi) {
   else return (uint32_t)f32_to_f16_bits(lo) | ((uint32_t)f32_to_f16_bits(hi) << 16);
 }
 
+// The softcap of E4M3 queries, out * tanh(in * x) for each score x that
+// each(f) hands to f by reference, with tanh within 2.2 * 2^-24 relative:
+// these calls are held to tanhf's accuracy, and 1 - 2 / (e^2x + 1) alone loses
+// small scores under a large cap.  Below 3/4 tanh is the odd series x + x^3
+// g(x^2), g the interpolation of (tanh(x) / x - 1) / x^2 at the six Chebyshev
+// nodes of [0, 9/16]; a wave with a larger argument adds the quotient.  64 x
+// 16384 keys, cap 30, us a call: 64/8 d128 398, 16/8 d128 386 (tanhf 507 /
+// 492, the quotient alone 362 / 367).
+template <typename Each>
+FA_DEV void softcap_rel(Each each, float in, float out) {
+  auto series = [](float x) {
+    const float u = x * x;
+    float g = fmaf(u, 0.0019095024f, -0.0079338076f);
+    g = fmaf(g, u, 0.021615319f);
+    g = fmaf(g, u, -0.053935852f);
+    g = fmaf(g, u, 0.13333179f);
+    g = fmaf(g, u, -0.33333331f);
+    return fmaf(x * u, g, x);
+  };
+  float most = 0.0f;
+  each([&](float& x) {
+    x *= in;
+    most = fmaxf(most, fabsf(x));
+  });
+  if (__any(most >= 0.75f)) {
+    each([&](float& x) {
+      const float m = fabsf(x);
+      const float large = fmaf(-2.0f, __builtin_amdgcn_rcpf(fast_exp2(2.0f * LOG2E * m) + 1.0f), 1.0f);
+      x = out * (m < 0.75f ? series(x) : copysignf(large, x));
+    });
+  } else {
+    each([&](float& x) { x = out * series(x); });
+  }
+}
+
 // First key any of a request's q_len query rows sees (the rows are the last
 // q_len positions; a left window starts at the first row's position - WL).
 FA_DEV int decode_vis_begin(const fa_attn_args& a, int k_len, int q_len = 1) {
@@ -397,7 +432,8 @@ __global__ __launch_bounds__(DEC_THREADS, FA_DEC_MINB) void decode_kernel(const 
                 descale_of(a.k_descale, a.k_descale_stride, b, kv) * (CAP ? 1.0f : LOG2E);
     vscale[u] = descale_of(a.v_descale, a.v_descale_stride, b, kv);
   }
-  const float cap_in = CAP ? 2.0f * LOG2E / a.softcap : 0.0f, cap_out = a.softcap * LOG2E;
+  constexpr bool E4M3Q = CT::id == FA_F16 && KT::id == FA_E4M3;   // variants that E4M3 queries share
+  const float cap_rel = CAP ? 1.0f / a.softcap : 0.0f, cap_in = 2.0f * LOG2E * cap_rel, cap_out = a.softcap * LOG2E;
   // ALiBi: -slope |q_pos - key| in log2 units after the softcap
   // (flash_attn_mps/kernels/attention.metal:47-51); the query sits at key
   // position k_len - 1, storage row qrow, so the bias is slope (row - qrow).
@@ -617,10 +653,20 @@ __global__ __launch_bounds__(DEC_THREADS, FA_DEC_MINB) void decode_kernel(const 
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         float v = row16_sum(s[g][i]) * sscale[half_of(g)];
-        if constexpr (CAP) v = cap_out * (1.0f - 2.0f * __builtin_amdgcn_rcpf(fast_exp2(v * cap_in) + 1.0f));
+        if constexpr (CAP && !E4M3Q) v = cap_out * (1.0f - 2.0f * __builtin_amdgcn_rcpf(fast_exp2(v * cap_in) + 1.0f));
         if constexpr (ALIBI) v = fmaf(slope2[g], (float)(rp + i - qrow), v);
         s[g][i] = v;
       }
+    if constexpr (CAP && E4M3Q) {
+      auto each = [&](auto f) {
+#pragma unroll
+        for (int g = 0; g < GT; ++g)
+#pragma unroll
+          for (int i = 0; i < NT; ++i) f(s[g][i]);
+      };
+      if (a.q_dtype == FA_E4M3) softcap_rel(each, cap_rel, cap_out);
+      else each([&](float& v) { v = cap_out * (1.0f - 2.0f * __builtin_amdgcn_rcpf(fast_exp2(v * cap_in) + 1.0f)); });
+    }
     if (!full) {
 #pragma unroll
       for (int i = 0; i < NT; ++i) {

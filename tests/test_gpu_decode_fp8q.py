@@ -2,7 +2,7 @@
 (matrix-core and VALU) against the float64 oracle.
 
 Tolerance: E4M3 products are exact and probabilities are held to fp32
-accuracy (as two fp16 terms on the matrix cores), so beside the output's own
+accuracy (as three bf16 terms on the matrix cores), so beside the output's own
 rounding (half an ulp: 2^-11 |out| in fp16, 2^-8 in bf16, 2^-25 for fp16
 subnormals) only fp32 sums differ: score errors of ~256 * 2^-24 * |score| <=
 6e-5, twice that relative on an output of magnitude up to max|v|.
@@ -99,3 +99,42 @@ def test_features(device, heads, kv_heads, dim, feature):
                                     block_table=table, causal=True, **{names.get(n, n): x for n, x in kw.items()}, **desc)
     vmax = float(v.float().nan_to_num(0).abs().amax() * desc["v_descale"].max())
     _check(got[:3], lse[:, :3], ref[:3], ref_lse[:, :3], vmax)
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 2, 128), (12, 3, 128), (16, 4, 64), (4, 4, 128), (4, 4, 256)])
+def test_small_probabilities_keep_their_weight(device, heads, kv_heads, dim):
+    """Four keys (one of each wave's first stage) score ~18.4 above 8000
+    others, whose probabilities of 2^-26.5 alone make the output: 1.4e-3 with
+    |V| = 64.  Probabilities held as 16-bit fractions of the largest drop them.
+
+    Tolerance: an output of 2^-10 is rounded to fp16 within 2^-21, and the fp32
+    sums err by less than 2^-11 of it."""
+    n = 8000
+    k, v = torch.zeros(n, kv_heads, dim), torch.full((n, kv_heads, dim), 64.0)
+    peaks = [0, 32, 64, 96]
+    k[peaks] = 1.625 * (128 / dim) ** 0.5 if dim != 256 else 1.125   # both E4M3 values at 64 (2.25) and 256
+    if dim == 64:
+        k[peaks] = 2.25
+    v[peaks] = 0.0
+    q = torch.ones(1, heads, dim)
+    q, k, v = (t.to(E4M3).to(device) for t in (q, k, v))
+    cu, cu_k = offsets([1], device), offsets([n], device)
+    got, lse = attention(q, k, v, cu_seqlens_q=cu, cu_seqlens_k=cu_k, max_seqlen_q=1, max_seqlen_k=n, num_splits=1)
+    ref, ref_lse = oracle_attention(q, k.float(), v.float(), cu, cu_k)
+    assert 2.0 ** -11 < ref.max() < 2.0 ** -8
+    assert ((got.cpu().double() - ref).abs() <= 2.0 ** -21 + 2.0 ** -10 * ref).all()
+    assert (lse.cpu().double() - ref_lse).abs().max() <= 1e-5
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim", [(16, 2, 128), (12, 3, 128), (16, 4, 64), (4, 4, 128), (4, 4, 256)])
+def test_small_scores_under_a_large_softcap(device, heads, kv_heads, dim):
+    """Scores of ~N(0, 1) under a cap of 4000: tanhf keeps their relative
+    accuracy (2^-22 of |score| <= 6 beside the dot's own ~16 * 2^-24), a
+    difference of nearly equal numbers only 2^-24 of the cap."""
+    n = 300
+    q, k, v = (_e4m3(shape, 50 + i, device, 1.0) for i, shape in
+               enumerate([(1, heads, dim), (n, kv_heads, dim), (n, kv_heads, dim)]))
+    cu, cu_k = offsets([1], device), offsets([n], device)
+    _, lse = attention(q, k, v, cu_seqlens_q=cu, cu_seqlens_k=cu_k, max_seqlen_q=1, max_seqlen_k=n, softcap=4000.0)
+    _, ref_lse = oracle_attention(q, k.float(), v.float(), cu, cu_k, softcap=4000.0)
+    assert (lse.cpu().double() - ref_lse).abs().max() <= 6e-6
