@@ -147,17 +147,25 @@ _F32_COLUMNS = 32
 _F32_ROUND = 128
 
 
+def _rows_aligned(t):
+    """Whether every 16-byte piece of an fp32 tensor's rows is aligned (mirrors
+    rows_aligned in attn_f32.hip)."""
+    strides = t.stride()
+    return t.data_ptr() % 16 == 0 and strides[-1] == 1 and not any(s % 4 for s in strides[:-1])
+
+
 def f32_splits(p):
     """Key splits of an fp32 call on the matrix-core kernel (a round of 128
-    keys or more each); None for calls of other types or head dims (the
-    generic kernel's rule).  One query row per request is bound by memory and
+    keys or more each); None for calls it does not take: other types, head
+    dims or alignments (the generic kernel's rule).  One query row per request is bound by memory and
     wants two workgroups per compute unit (4 x 2048 keys, 16/8 heads: 4 / 8 /
     16 splits 39.0 / 28.6 / 28.2 us a call; 4 x 8192: 8 / 16 / 32 splits 64.4 /
     58.3 / 73.5).  More rows are bound by the matrix cores, and partials cost
     more than idle compute units until most of them idle (2 x 256 tokens, 256
     workgroups: 1 / 2 splits 19.5 / 29.4 us; 1 x 2048: 177 / 204)."""
     f32 = torch.float32
-    if not (p.q.dtype == p.k.dtype == p.v.dtype == f32 and (p.dim_qk, p.dim_v) in _F32_DIMS):
+    if not (p.q.dtype == p.k.dtype == p.v.dtype == f32 and (p.dim_qk, p.dim_v) in _F32_DIMS
+            and _rows_aligned(p.q) and _rows_aligned(p.k) and _rows_aligned(p.v)):
         return None
     rows = 1
     while rows < _F32_COLUMNS and rows < p.max_q:
