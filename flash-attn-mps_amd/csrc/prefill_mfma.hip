@@ -217,8 +217,9 @@ extern "C" int fa_prefill_fwd(const fa_attn_args* args, void* stream) {
   const bool split = a->num_splits > 1;
   FA_REQUIRE(!split || (a->partial_out && a->partial_lse && aligned16(a->partial_out)),
              "fa_prefill_fwd: splits need partial buffers, the outputs' 16-byte aligned");
-  FA_REQUIRE(!split || (a->batch <= 65535 && a->max_seqlen_q * a->heads_q <= 0x7fffffffll),
-             "fa_prefill_fwd: split grid too large");
+  // The merge's rows per request: max_seqlen_q may be far above any request's.
+  const int64_t merge_rows = (a->max_seqlen_q < a->total_q ? a->max_seqlen_q : a->total_q) * a->heads_q;
+  FA_REQUIRE(!split || (a->batch <= 65535 && merge_rows <= 0x7fffffffll), "fa_prefill_fwd: split grid too large");
   hipError_t err = hipFuncSetAttribute((const void*)ch.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ch.lds);
   if (err != hipSuccess) {
     fa_set_error("fa_prefill_fwd: cannot reserve %zu bytes of LDS: %s", ch.lds, hipGetErrorString(err));
@@ -233,7 +234,7 @@ extern "C" int fa_prefill_fwd(const fa_attn_args* args, void* stream) {
   void (*merge)(const fa_attn_args) = a->head_dim_v == 64    ? prefill_merge_kernel<1, 8>
                                       : a->head_dim_v == 128 ? prefill_merge_kernel<2, 8>
                                                              : prefill_merge_kernel<4, 4>;
-  hipLaunchKernelGGL(merge, dim3((unsigned)fa_ceil_div(a->max_seqlen_q * a->heads_q, 4), (unsigned)a->batch), dim3(256), 0,
+  hipLaunchKernelGGL(merge, dim3((unsigned)fa_ceil_div(merge_rows, 4), (unsigned)a->batch), dim3(256), 0,
                      (hipStream_t)stream, *a);
   return fa_check_launch("fa_prefill_fwd");
 }

@@ -86,3 +86,19 @@ def test_the_plan_and_the_kernel_agree(device, dq, dv, kt, softcap):
     for extra in (dict(num_splits=1), dict(deterministic=True), dict(window_size=(100, 0)),
                   dict(alibi_slopes=torch.ones(4, device=device))):
         assert _attention.prefill_splits(problem(q, k, v, **{**kw, **extra})) == 1
+
+
+@pytest.mark.parametrize("max_q", [40, 1 << 20, 1 << 30])
+def test_a_loose_row_bound(device, monkeypatch, max_q):
+    """max_seqlen_q far above any request's rows: the merge's grid follows the
+    rows there are (2^30 rows of 4 heads were refused, 2^20 of 3 requests ran
+    three million idle workgroups)."""
+    q_lens, k_lens = [40, 3, 17], [700, 64, 131]
+    k, v, table = _paged(device, k_lens, 2, 128, 128, torch.bfloat16)
+    q = _values((60, 4, 128), 8, torch.bfloat16, device)
+    _split_everything(monkeypatch, 4)
+    cu, used = offsets(q_lens, device), torch.tensor(k_lens, dtype=torch.int32, device=device)
+    got, lse = attention(q, k, v, cu_seqlens_q=cu, seqused_k=used, max_seqlen_q=max_q, max_seqlen_k=700,
+                         block_table=table.to(device), causal=True)
+    ref, ref_lse = oracle_attention(q, k, v, cu, used_k=used, block_table=table, causal=True)
+    assert_parity(got, lse, ref, ref_lse)
