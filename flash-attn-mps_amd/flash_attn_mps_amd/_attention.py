@@ -117,8 +117,8 @@ def _fits_prefill(p, out):
     """Features the MFMA route takes at all (the kernel is asked about the rest,
     vLLM mask kinds and left padding included): 16-bit queries over same-type
     or E4M3 K/V with output in the query's type, or E4M3 queries over E4M3 K/V
-    with fp16/bf16 output (S on the FP8 MFMA).  The kernel never splits a row,
-    so deterministic calls qualify."""
+    with fp16/bf16 output (S on the FP8 MFMA).  Deterministic calls qualify:
+    prefill_splits keeps them, and num_splits=1, at one split."""
     if p.splits not in (0, 1):
         return False
     fp8 = torch.float8_e4m3fn

@@ -1,21 +1,23 @@
-"""256-dim MFMA prefill run as two V-column halves vs the fp64 oracle.
+"""256-dim MFMA prefill vs the fp64 oracle.
 
-fa_prefill_fwd runs 256-dim heads as two workgroups per work item, one per
-128-column half of V and of the output (prefill_vparts in
-prefill_kernel.h; the one-pass 256/256 tile stays for 16-bit softcaps and for
-E4M3 softcaps with a window).  Both halves recompute S; only the first
-writes the LSE.  These cases pin the part decoding against both work-list
-modes (compact up to 256 requests, the per-pair grid beyond), one and two
-query heads per workgroup, strided V and output views (the second half's
-columns start DVT elements into the row, whatever the strides), spare
-output rows and columns that must stay unwritten, and E4M3 K/V on both
-routes.  Bar: this build's (max-abs <= 1e-2 bf16, LSE <= 1e-4) on rows that
-see at least 32 keys, plus the all-rows check of assert_parity.
+16-bit K/V without ALiBi, mask kinds and key splits run as wave pairs
+(prefill_pair.h; edges in test_gpu_prefill_pair.py); the others as two
+workgroups per work item, one per 128-column half of V and of the output
+(prefill_vparts in prefill_kernel.h; the one-pass 256/256 tile stays for
+16-bit softcaps with ALiBi or a mask kind and for E4M3 softcaps with a
+window).  Both halves recompute S; only the first writes the LSE.  These
+cases pin, on either route, the work-list modes (compact up to 256 requests,
+the per-pair grid beyond) and one and two query heads per workgroup, strided
+V and output views (the second half's columns start DVT elements into the
+row, whatever the strides), spare output rows and columns that must stay
+unwritten, and E4M3 K/V on both its routes.  Bar: this build's (max-abs <=
+1e-2 bf16, LSE <= 1e-4) on rows that see at least 32 keys, plus the all-rows
+check of assert_parity.
 """
 import pytest
 import torch
 
-from flash_attn_mps_amd import _lib, vllm
+from flash_attn_mps_amd import _attention, _lib, vllm
 from harness import assert_parity, attention, kernel_args, offsets, oracle_attention
 
 pytestmark = pytest.mark.gpu
@@ -179,3 +181,31 @@ def test_d256_halves_requests_alone_and_batched(device, kv_dtype):
         assert torch.equal(o1, out[qo:qo + n]), f"request {i}: output"
         assert torch.equal(l1, lse[:, qo:qo + n]), f"request {i}: LSE"
         qo, ko = qo + n, ko + m
+
+
+@pytest.mark.parametrize("route", ["alibi", "e4m3", "splits"])
+@pytest.mark.parametrize("batch,hq,hkv", [(9, 16, 8), (9, 16, 16), (20, 12, 4), (13, 6, 2), (257, 8, 2), (257, 6, 2)])
+def test_d256_halves_work_list(device, monkeypatch, route, batch, hq, hkv):
+    """The work-list modes of test_d256_halves_work_list_modes on routes that
+    run V halves: ALiBi, E4M3 K/V and key splits."""
+    g = torch.Generator().manual_seed(batch * 10 + hq + hkv)
+    q_lens = torch.randint(2, 160, (batch,), generator=g)
+    q_lens[::7] = 0
+    k_lens = (q_lens + torch.randint(0, 90, (batch,), generator=g)).tolist()
+    q_lens, spare = q_lens.tolist(), 40
+    kt = E4M3 if route == "e4m3" else torch.bfloat16
+    q = (torch.randn(sum(q_lens) + spare, hq, 256, generator=g) * 0.5).to(torch.bfloat16).to(device)
+    k = (torch.randn(sum(k_lens), hkv, 256, generator=g) * 0.5).to(kt).to(device)
+    v = (torch.randn(sum(k_lens), hkv, 256, generator=g) * VALUE_SCALE).to(kt).to(device)
+    slopes = 2.0 ** (-8.0 * torch.arange(1, hq + 1) / hq) if route == "alibi" else None
+    cuq, cuk = offsets(q_lens, device), offsets(k_lens, device)
+    kw = dict(cu_seqlens_q=cuq, cu_seqlens_k=cuk, max_seqlen_q=max(q_lens), max_seqlen_k=max(k_lens), causal=True,
+              alibi_slopes=None if slopes is None else slopes.to(device))
+    assert _route_mfma(q, k, v, **kw)
+    if route == "splits":
+        monkeypatch.setattr(_attention, "prefill_splits", lambda p: 3)
+    out, lse = attention(q, k, v, out=torch.full_like(q, float("nan")), **kw)
+    ref, ref_lse = oracle_attention(q, k.float(), v.float(), cuq, cuk, causal=True, alibi=slopes)
+    rows = torch.arange(sum(q_lens))
+    assert_parity(out[rows], lse[:, rows], ref[rows], ref_lse[:, rows], torch.bfloat16)
+    assert torch.isnan(out[sum(q_lens):].float()).all(), "spare rows past the last request were written"
