@@ -57,7 +57,10 @@ class _Counting:
                 return hit
             vector = self._vectors.get(key[:2])
             if vector is None and not (device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
-                vector = torch.arange(self._entries, dtype=torch.int32).to(device)
+                # On the host whatever torch's default device is, so that the copy is what makes it.
+                vector = torch.arange(self._entries, dtype=torch.int32, device="cpu").to(device)
+                if type(vector) is not torch.Tensor:   # a tracer's stand-in: no later call may see it
+                    return vector.as_strided(shape, stride)
                 self._vectors[key[:2]] = vector
             if vector is None or last >= self._entries:
                 return (torch.arange(shape[0], dtype=torch.int32, device=device) * stride[0]).reshape(shape)

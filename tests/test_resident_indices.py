@@ -57,3 +57,15 @@ def test_threads_share_one_vector():
     for t in threads:
         t.join()
     assert len(seen) == 2400 and all(seen) and len(c._vectors) == 1
+
+
+@pytest.mark.parametrize("context", ["fake", "default device"])
+def test_a_mode_around_the_first_call_leaves_nothing_behind(context):
+    """Under a tracer's stand-in tensors nothing is kept (they would be every
+    later call's offsets), and torch's default device does not place the vector."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    c = _Counting(entries=100)
+    with FakeTensorMode() if context == "fake" else torch.device("meta"):
+        first = c.offsets(2, 3, CPU)
+    assert (type(first) is torch.Tensor) == (context != "fake") and first.shape == (3,)
+    assert c.offsets(2, 3, CPU).tolist() == [0, 3, 6]
