@@ -433,7 +433,8 @@ __global__ __launch_bounds__(DEC_THREADS, FA_DEC_MINB) void decode_kernel(const 
     vscale[u] = descale_of(a.v_descale, a.v_descale_stride, b, kv);
   }
   constexpr bool E4M3Q = CT::id == FA_F16 && KT::id == FA_E4M3;   // variants that E4M3 queries share
-  const float cap_rel = CAP ? 1.0f / a.softcap : 0.0f, cap_in = 2.0f * LOG2E * cap_rel, cap_out = a.softcap * LOG2E;
+  const float cap_rel = CAP && E4M3Q ? 1.0f / a.softcap : 0.0f;
+  const float cap_in = CAP ? 2.0f * LOG2E / a.softcap : 0.0f, cap_out = a.softcap * LOG2E;
   // ALiBi: -slope |q_pos - key| in log2 units after the softcap
   // (flash_attn_mps/kernels/attention.metal:47-51); the query sits at key
   // position k_len - 1, storage row qrow, so the bias is slope (row - qrow).
