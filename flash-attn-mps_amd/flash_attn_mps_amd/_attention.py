@@ -147,11 +147,12 @@ _F32_COLUMNS = 32
 _F32_ROUND = 128
 
 
-def _rows_aligned(t):
-    """Whether every 16-byte piece of an fp32 tensor's rows is aligned (mirrors
+def _rows_aligned(q, k, v):
+    """Whether every 16-byte piece of these fp32 rows is aligned (mirrors
     rows_aligned in attn_f32.hip)."""
-    strides = t.stride()
-    return t.data_ptr() % 16 == 0 and strides[-1] == 1 and not any(s % 4 for s in strides[:-1])
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
+    return (qs[2] == ks[-1] == vs[-1] == 1 and not (q.data_ptr() | k.data_ptr() | v.data_ptr()) & 15
+            and not (qs[0] | qs[1] | ks[0] | ks[1] | ks[-2] | vs[0] | vs[1] | vs[-2]) & 3)
 
 
 def f32_splits(p):
@@ -164,17 +165,18 @@ def f32_splits(p):
     more than idle compute units until most of them idle (2 x 256 tokens, 256
     workgroups: 1 / 2 splits 19.5 / 29.4 us; 1 x 2048: 177 / 204)."""
     f32 = torch.float32
-    if not (p.q.dtype == p.k.dtype == p.v.dtype == f32 and (p.dim_qk, p.dim_v) in _F32_DIMS
-            and _rows_aligned(p.q) and _rows_aligned(p.k) and _rows_aligned(p.v)):
+    q, k, v, max_q = p.q, p.k, p.v, p.max_q
+    if not (q.dtype == k.dtype == v.dtype == f32 and (p.dim_qk, p.dim_v) in _F32_DIMS and _rows_aligned(q, k, v)):
         return None
     rows = 1
-    while rows < _F32_COLUMNS and rows < p.max_q:
+    while rows < _F32_COLUMNS and rows < max_q:
         rows *= 2
-    group = p.heads // p.kv_heads
+    kv_heads, batch = p.kv_heads, p.batch
+    group = p.heads // kv_heads
     tiles = -(-group // min(group, _F32_COLUMNS // rows))
-    row_blocks = min(p.batch * -(-p.max_q // rows), p.tokens // rows + p.batch)
-    blocks = max(1, row_blocks * p.kv_heads * tiles)
-    wanted = -(-512 // blocks) if p.max_q == 1 else 256 // blocks
+    row_blocks = min(batch * -(-max_q // rows), p.tokens // rows + batch)
+    blocks = max(1, row_blocks * kv_heads * tiles)
+    wanted = -(-512 // blocks) if max_q == 1 else 256 // blocks
     return max(1, min(wanted, -(-p.visible_max // _F32_ROUND)))
 
 
