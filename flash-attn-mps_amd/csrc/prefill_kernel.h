@@ -158,6 +158,14 @@ FA_DEV float sum_hh(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Key splits of a request of k_len keys: the a.num_splits that the host planned
+// for a.max_seqlen_k, which may be far above k_len (the capacity of a cache),
+// as far as each gets a.split_span keys (0: any number).  A request with one
+// split is written as by the unsplit kernel, without partials.
+FA_DEV int request_splits(const fa_attn_args& a, int k_len) {
+  return a.split_span > 0 ? min(max(k_len / a.split_span, 1), a.num_splits) : a.num_splits;
+}
+
 // 16 bytes a lane from a buffer straight into LDS at lds + 16 * lane
 // (buffer_load_dwordx4 ... lds: LDS address = m0 + IMM + 16 * lane, global
 // address = base + voffset + IMM).  Written as inline assembly so that the
@@ -351,9 +359,10 @@ FA_DEV bool compact_item(const fa_attn_args& a, int slot, int xcd, int lane, int
 // MK: vLLM mask kind (a.mask_kind; 0 none): each row's visible keys are at
 // most two key ranges (see mask_ranges below); causality and the window
 // fields do not apply, as in the reference (kernels/attention.metal:29-45).
-// SPLIT: a.num_splits workgroups (blockIdx.y) share each work item's key
-// tiles evenly and write fp32 partials for prefill_merge_kernel: for grids
-// that leave CUs idle (a chunk of a few hundred rows behind a long prefix).
+// SPLIT: a.num_splits workgroups (blockIdx.y; request_splits of them at work)
+// share each work item's key tiles evenly and write fp32 partials for
+// prefill_merge_kernel: for grids that leave CUs idle (a chunk of a few hundred
+// rows behind a long prefix).
 template <typename T, int DQ, int DV, int W, int NB, int MINB, bool CAUSAL, bool CAP, bool WIN, int DQT = DQ,
           int DVT = DV, typename KT = T, bool ALIBI = false, typename QT = T, int MK = 0, bool SPLIT = false>
 __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_args a, const PrefillShape shp) {
@@ -541,12 +550,13 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
   }
   int n_tiles = kv_end > 0 ? (kv_end + PF_BN - 1) / PF_BN : 0;
   int tile0 = kv_begin / PF_BN;   // first tile with a visible key
-  const int split = SPLIT ? (int)blockIdx.y : 0;
+  const int split = SPLIT ? (int)blockIdx.y : 0, splits = SPLIT ? request_splits(a, r.k_len) : 1;
   if constexpr (SPLIT) {
     static_assert(MK == 0 && !WIN, "key splits: one run of tiles per work item");
+    if (split >= splits) return;
     const int n = n_tiles;   // tile0 = 0 without windows
-    tile0 = (int)((int64_t)n * split / a.num_splits);
-    n_tiles = (int)((int64_t)n * (split + 1) / a.num_splits);
+    tile0 = (int)((int64_t)n * split / splits);
+    n_tiles = (int)((int64_t)n * (split + 1) / splits);
     kv_end = min(kv_end, n_tiles * PF_BN);
   }
 
@@ -1348,7 +1358,7 @@ __global__ __launch_bounds__(64 * W, MINB) void prefill_kernel(const fa_attn_arg
     if (row < r.q_len) {
       const float inv = lt > 0.0f ? vdsc / lt : 0.0f;
       const int64_t tq = (int64_t)r.q_begin + row;
-      if constexpr (SPLIT) {
+      if (SPLIT && splits > 1) {
         // Partials [S][T][Hq][Dv] (normalised), LSEs [S][Hq][T] (NaN where
         // the sum is: the merge must not take that for a split without keys).
         const int64_t dv = TWO_PARTS ? 2 * DVT : DVT;

@@ -52,18 +52,20 @@ bool split_ok(const fa_attn_args& a) {
 // Merge of the split partials: one wave per (request, row, head) row, split
 // weights on lanes, GROUP partial rows in flight; DIMS dims per lane.  The
 // rows of single-query requests under FA_FLAG_SKIP_SINGLE_QUERY are the
-// decode kernel's and stay untouched.  A split whose LSE is NaN makes the row
-// NaN, with LSE -inf, as one split would.
+// decode kernel's, those of requests with one split are the split kernel's, and
+// both stay untouched.  A split whose LSE is NaN makes the row NaN, with LSE
+// -inf, as one split would.
 template <int DIMS, int GROUP>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const fa_attn_args a) {
-  const int lane = threadIdx.x & 63, S = a.num_splits, DV = (int)a.head_dim_v;
+  const int lane = threadIdx.x & 63, DV = (int)a.head_dim_v;
   const uint32_t idx = blockIdx.x * 4 + (threadIdx.x >> 6), hq = (uint32_t)a.heads_q;
   const int64_t b = blockIdx.y;
-  const int64_t q_begin = load_invariant_i32(a.cu_seqlens_q, b * a.cu_q_stride);
-  const int q_len = load_invariant_i32(a.cu_seqlens_q, (b + 1) * a.cu_q_stride) - (int)q_begin;
+  const RequestInfo r = load_request(a, b);
+  const int64_t q_begin = r.q_begin;
+  const int q_len = r.q_len, S = request_splits(a, r.k_len);
   const int row = (int)(idx / hq);
   const int64_t h = idx - (uint32_t)row * hq;
-  if (row >= q_len || ((a.flags & FA_FLAG_SKIP_SINGLE_QUERY) && q_len == 1)) return;
+  if (S == 1 || row >= q_len || ((a.flags & FA_FLAG_SKIP_SINGLE_QUERY) && q_len == 1)) return;
   const int64_t tq = q_begin + row;
   const float* const part = a.partial_out + (tq * a.heads_q + h) * DV;
   const float* const plse = a.partial_lse + h * a.total_q + tq;

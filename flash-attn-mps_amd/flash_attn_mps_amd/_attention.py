@@ -198,9 +198,11 @@ def prefill_splits(p):
     unit, plus 6 us for the merge and the partials written and read back at
     2.5 TB/s.  Measured (us, 1 split -> the chosen count, bf16, 16-token
     pages): 512 rows behind 24000 keys, 32/8 heads d128 451 -> 211 (4), 64
-    rows 445 -> 46 (16), 2 x 256 behind 4096, 16/8 94 -> 44 (4), 512 behind
-    8192, 16/8 d256 283 -> 116 (4); where the estimate keeps one: 1 x 2048
-    causal 16/8 44 against 56 with two, 4 x 128 behind 1024 35 / 38."""
+    rows 445 -> 46 (16), 2 x 256 behind 4096, 16/8 94 -> 44 (4); d256 16/8,
+    where one split runs the wave pairs, 512 of 8192 keys 297 -> 115 (4), 1024 of
+    2048 84 -> 71 (2), of 8192 294 -> 198 (2); where the estimate keeps one: 1 x
+    2048 causal 16/8 44 against 56 with two, d256 85 / 94, 4 x 128 behind 1024
+    35 / 38."""
     if p.max_k < _PREFILL_SPLIT_MIN_KEYS:
         return 1
     if (p.splits or p.deterministic or p.mask is not None or p.alibi is not None or torch.is_tensor(p.causal)
@@ -208,23 +210,52 @@ def prefill_splits(p):
         return 1
     if p.dim_v != (128 if p.dim_qk == 192 else p.dim_qk) or (p.softcap > 0 and p.dim_qk > 128):
         return 1
-    rows, per_cu, parts, tile_us = _PREFILL_TILE[p.dim_qk]
-    pair = 2 if p.heads // p.kv_heads % 2 == 0 else 1   # heads per workgroup
-    requests = p.batch if p.tokens >= 2 * p.batch else 1
-    blocks = requests * -(-p.tokens // (requests * (rows // pair))) * (p.heads // pair) * parts
-    most = min(per_cu * _COMPUTE_UNITS // blocks, 16)
+    blocks = _prefill_blocks(p)
+    most = min(_PREFILL_TILE[p.dim_qk][1] * _COMPUTE_UNITS // blocks, 16)
     if most < 2 or p.batch > 65535:
         return 1
-    keys_us = p.max_k / 64 * tile_us
-    partial_us = p.tokens * p.heads * p.dim_v * 8 / 2.5e6
-    best, best_us = 1, keys_us
+    best, best_us = 1, p.max_k * _key_us(p, blocks, 1)
     for n in (2, 3, 4, 6, 8, 12, 16):
         if n > most:
             break
-        us = keys_us / n * (0.55 + 0.45 * -(-blocks * n // _COMPUTE_UNITS)) + 6 + n * partial_us
+        us = p.max_k * _key_us(p, blocks, n) + _merge_us(p, n)
         if us < best_us:
             best, best_us = n, us
     return best
+
+
+def _prefill_blocks(p):
+    """Workgroups of an unsplit MFMA prefill call."""
+    rows, _, parts, _ = _PREFILL_TILE[p.dim_qk]
+    pair = 2 if p.heads // p.kv_heads % 2 == 0 else 1   # heads per workgroup
+    requests = p.batch if p.tokens >= 2 * p.batch else 1
+    return requests * -(-p.tokens // (requests * (rows // pair))) * (p.heads // pair) * parts
+
+
+def _key_us(p, blocks, n):
+    """Time of a key in n splits: a tile's, shared by 64 keys, stretched by the
+    workgroups that then share a compute unit (one split: as many as the grid has)."""
+    crowd = 1 if n == 1 else 0.55 + 0.45 * -(-blocks * n // _COMPUTE_UNITS)
+    return _PREFILL_TILE[p.dim_qk][3] / 64 * crowd / n
+
+
+def _merge_us(p, n):
+    return 6 + n * p.tokens * p.heads * p.dim_v * 8 / 2.5e6
+
+
+def prefill_split_span(p, splits):
+    """Keys that a request must have per split.  max_seqlen_k may be the capacity
+    of a cache, far above the lengths there are, which only the kernel sees: by
+    the same estimate `splits` pay from this many keys each, and a request with
+    fewer takes fewer.  Captured graphs, 32/8 heads d128, capacity 32768, us with
+    one split / all planned / this many each: 512 rows planned as four, 600 keys
+    20.7 / 31.9 / 24.7, 1024 27.3 / 33.1 / 32.3, 2048 46.0 / 40.8 / 43.1; 64 rows
+    planned as 16, 200 keys 12.7 / 15.6 / 14.9, 600 19.7 / 15.7 / 15.9.  The merge's
+    launch is what one split still loses (3-4 us)."""
+    blocks = _prefill_blocks(p)
+    gain_us = _key_us(p, blocks, 1) - _key_us(p, blocks, splits)
+    worth = _merge_us(p, splits) / gain_us if gain_us > 0 else p.max_k
+    return max(1, int(min(worth, p.max_k) / splits))
 
 
 _SIDE = {}
@@ -349,7 +380,7 @@ def solve(p):
         splits = prefill_splits(p)
         if splits > 1:
             _partials(p, a, (splits, p.tokens, p.heads, p.dim_v), (splits, p.heads, p.tokens))
-            a.num_splits = splits
+            a.num_splits, a.split_span = splits, prefill_split_span(p, splits)
         if not (mixed and _mixed_batch(p, a, fixed_order=p.deterministic)):
             _lib.call("fa_prefill_fwd", a, p.device)
         return out, lse

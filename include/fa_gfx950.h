@@ -271,7 +271,8 @@ int fa_decode_fwd_noalloc(const fa_attn_args* args, void* stream);
  * unpadded 64/128/256-dim heads; head dims 32-256 and 192/128).
  * fa_prefill_supported() says whether the argument
  * combination is compiled in; num_splits 2..64 splits the keys (partial_out 16-byte
- * aligned) where windows, ALiBi and mask kinds are absent and the head dims
+ * aligned; a request takes as many as leave each split_span keys, with split_span
+ * 0 all of them) where windows, ALiBi and mask kinds are absent and the head dims
  * are 64, 128 (softcap too), 192/128 or 256.  With FA_FLAG_SKIP_SINGLE_QUERY in
  * args->flags, requests with one query row are left untouched for
  * fa_decode_fwd (no reference counterpart: the reference runs such rows

@@ -204,6 +204,7 @@ def test_d256_halves_work_list(device, monkeypatch, route, batch, hq, hkv):
     assert _route_mfma(q, k, v, **kw)
     if route == "splits":
         monkeypatch.setattr(_attention, "prefill_splits", lambda p: 3)
+        monkeypatch.setattr(_attention, "prefill_split_span", lambda p, splits: 0)
     out, lse = attention(q, k, v, out=torch.full_like(q, float("nan")), **kw)
     ref, ref_lse = oracle_attention(q, k.float(), v.float(), cuq, cuk, causal=True, alibi=slopes)
     rows = torch.arange(sum(q_lens))

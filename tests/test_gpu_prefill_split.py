@@ -29,6 +29,7 @@ def _paged(device, k_lens, kv_heads, dq, dv, dtype, page=16):
 
 def _split_everything(monkeypatch, count):
     monkeypatch.setattr(_attention, "prefill_splits", lambda p: count)
+    monkeypatch.setattr(_attention, "prefill_split_span", lambda p, splits: 0)
 
 
 @pytest.mark.parametrize("qt,kt", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
@@ -102,3 +103,32 @@ def test_a_loose_row_bound(device, monkeypatch, max_q):
                          block_table=table.to(device), causal=True)
     ref, ref_lse = oracle_attention(q, k, v, cu, used_k=used, block_table=table, causal=True)
     assert_parity(got, lse, ref, ref_lse)
+
+
+@pytest.mark.parametrize("qt,kt,dq,dv", [(torch.bfloat16, torch.bfloat16, 64, 64), (torch.float16, torch.float16, 128, 128),
+                                         (torch.bfloat16, torch.bfloat16, 192, 128), (torch.bfloat16, torch.bfloat16, 256, 256),
+                                         (torch.bfloat16, E4M3, 128, 128), (E4M3, E4M3, 256, 256)])
+@pytest.mark.parametrize("span,counts", [(0, [4, 4, 4]), (130, [1, 4, 4]), (600, [1, 1, 3]), (2300, [1, 1, 1])])
+def test_requests_far_below_the_key_bound(device, qt, kt, dq, dv, span, counts):
+    """130, 1100 and 2300 keys of a call planned in four splits: a request takes
+    as many as leave each `span` keys, and one split writes no partials."""
+    q_lens, k_lens = [40, 70, 17], [130, 1100, 2300]
+    k, v = _values((sum(k_lens), 2, dq), 2, kt, device), _values((sum(k_lens), 2, dv), 3, kt, device, 0.5)
+    q = _values((127, 4, dq), 4, qt, device)
+    sinks = seeded((4,), 5, torch.float32, device)
+    cu, cu_k = offsets(q_lens, device), offsets(k_lens, device)
+    out_type = torch.bfloat16 if qt == E4M3 else qt
+    out, lse = torch.empty(127, 4, dv, dtype=out_type, device=device), torch.empty(4, 127, device=device)
+    keep = [torch.full((4, 127, 4, dv), 7.0, device=device), torch.full((4, 4, 127), 7.0, device=device)]
+    a = kernel_args(q, k, v, out, lse, keep=keep, cu_seqlens_q=cu, cu_seqlens_k=cu_k, max_seqlen_q=70, max_seqlen_k=1 << 16,
+                    causal=True, s_aux=sinks)
+    a.num_splits, a.split_span = 4, span
+    a.partial_out, a.partial_lse = keep[0].data_ptr(), keep[1].data_ptr()
+    _lib.call("fa_prefill_fwd", a, device)
+    ref, ref_lse = oracle_attention(q.float() if qt == E4M3 else q, k.float(), v.float(), cu, cu_k, causal=True, sinks=sinks)
+    assert_parity(out, lse, ref, ref_lse)
+    for b, count in enumerate(counts):
+        rows = slice(sum(q_lens[:b]), sum(q_lens[:b + 1]))
+        written = count if count > 1 else 0
+        assert (keep[0][written:, rows] == 7).all() and (keep[1][written:, :, rows] == 7).all()
+        assert (keep[1][:written, :, rows] != 7).all()

@@ -56,6 +56,7 @@ def test_rows_of_a_chunk(device, monkeypatch, qt, kt, dq, dv, splits):
     cu_q, cu_k = offsets(q_lens, device), offsets(k_lens, device)
     ref, ref_lse = oracle_attention(q.float() if qt == E4M3 else q, k.float(), v.float(), cu_q, cu_k, causal=True)
     monkeypatch.setattr(_attention, "prefill_splits", lambda p: splits)
+    monkeypatch.setattr(_attention, "prefill_split_span", lambda p, n: 0)
     kw = dict(cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=90, max_seqlen_k=700, causal=True,
               num_splits=splits if qt == torch.float32 else 0)
     bad = torch.zeros(123, 4, dtype=torch.bool)
