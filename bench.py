@@ -1,6 +1,6 @@
 """Benchmark of the flash_attn_mps_amd hot path on one MI355X.
 
-Headline (`value`): bf16 causal varlen prefill TFLOP/s on BASELINE config 2
+Headline (`value`): bf16 causal varlen prefill TFLOP/s on config 2
 (16 sequences, lengths U[256, 4096], Hq/Hkv = 16/8, d = 128, Qwen3-0.6B
 attention shape), one `flash_attn_varlen_func` call per step with Q/K/V
 resident in HBM.  Algorithmic FLOPs = sum over visible (query, key) pairs x

@@ -47,7 +47,7 @@
 //   barrier (2 x 1024 causal 16/8 d128 114 us with and without).
 // * Measured (generic kernel before): 2 x 1024 tokens causal, 16/8 heads,
 //   d128 4971 -> 111 us (77 TFLOP/s; 1024 workgroups for 256 CUs); decode of
-//   4 requests x 2048 keys 252 + 14 (merge) -> 16 + 4 us.
+//   4 requests x 2048 keys 252 + 14 (merge) -> 22 + 4 us.
 #include "attn_common.h"
 
 #include <climits>

@@ -1514,19 +1514,17 @@ PrefillChoice pick_dims_small(int64_t dq, int64_t dv, bool causal, int score, bo
   }
 }
 
-// 256-dim heads: two V-column halves per work item (prefill_vparts),
-// each an eight-wave 256/128 tile at two waves per SIMD (the one-pass
-// 256/256 tile holds four waves, one per SIMD, and spills more).  The halves
-// recompute S, with every tanh of a softcap: 16-bit softcaps, and E4M3
+// 256-dim heads that the wave pairs of prefill_pair.h leave (E4M3 K/V; 16-bit
+// K/V with ALiBi or mask kinds): two V-column halves per work item
+// (prefill_vparts), each an eight-wave 256/128 tile at two waves per SIMD (the
+// one-pass 256/256 tile holds four waves, one per SIMD, and spills more).  The
+// halves recompute S, with every tanh of a softcap: 16-bit softcaps, and E4M3
 // softcaps with a window and no ALiBi, keep the one-pass tile (which has no
-// E4M3 ALiBi instance).  Measured on config 2's
-// lengths at 16/8 heads (TFLOP/s, one-pass -> halves): bf16 causal 456 ->
-// 597, non-causal 629 -> 716, ALiBi 404 -> 519, left window 1023 260 -> 292,
-// vLLM mm_prefix +36%, rswa +8%, softcap 50 560 -> 519, softcap + window
-// 346 -> 257; E4M3 K/V causal 299 -> 564, non-causal 342 -> 657, softcap
-// 339 -> 444, window 221 -> 255, softcap + window 285 -> 228.
-// (16-bit K/V without ALiBi and mask kinds take the wave pairs of
-// prefill_pair.h before they come here.)
+// E4M3 ALiBi instance).  Measured on config 2's lengths at 16/8 heads
+// (TFLOP/s, one-pass -> halves): 16-bit ALiBi 404 -> 519, vLLM mm_prefix +36%,
+// rswa +8%, a softcap without mask or bias 560 -> 519; E4M3 K/V causal 299 ->
+// 564, non-causal 342 -> 657, softcap 339 -> 444, window 221 -> 255, softcap +
+// window 285 -> 228.
 template <typename T, typename KT>
 PrefillChoice pick_256(bool causal, int score, bool win, int mk) {
   const bool cap = score == 1 || score == 3;

@@ -2,14 +2,15 @@
 //
 // What bounds 256-dim heads: O^T of 32 rows is 128 registers and Q 64, so a
 // wave that owns 32 whole rows fills the 512 registers of a SIMD by itself,
-// spills, and has no second wave to overlap its softmax with (one-pass
-// 256/256 tile: 560 TFLOP/s with softcap, 346 with softcap and a window); as
-// two workgroups per V half S and its softmax are computed twice (600
-// TFLOP/s without softcap).  Here two waves share 32 rows: each takes one
+// spills 62 and more, and has no second wave to overlap its softmax with
+// (one-pass 256/256 tile: 560 TFLOP/s with softcap, 346 with softcap and a
+// window); as two workgroups per V half S and its softmax are computed twice
+// (600 TFLOP/s without softcap).  Here two waves share 32 rows: each takes one
 // 32-key half of every 64-key tile for S and the softmax and one 128-column
 // half of V for O^T, and they exchange their probabilities through LDS.
 // Nothing is computed twice, a wave holds 64 + 64 registers of O^T and Q, and
-// two waves fit a SIMD.  (Reference counterpart as prefill_kernel.h.)
+// two waves fit a SIMD (256 registers each, of which 13-15 still spill, 26 with
+// softcap and a window that is not causal).  (Reference counterpart as prefill_kernel.h.)
 //
 // * A workgroup is eight waves, four row blocks of 32 (of one head, or two
 //   blocks of each of two heads of a KV head).  Layouts, DMA, MFMA operand
@@ -28,8 +29,9 @@
 // * Measured, 16 sequences of 256..4096 tokens, 16/8 heads, bf16, TFLOP/s of
 //   visible pairs, before -> here: causal 608 -> 721, softcap 556 -> 562, left
 //   window of 1023 291 -> 581, softcap and window 346 -> 538, not causal 712
-//   -> 828.  What bounds it now: MFMA busy ~30%, VALU ~40% (softcap and
-//   window), the rest waits at the barrier and LDS operand latency.
+//   -> 828.  What bounds it now (counters): causal MFMA busy 29%, VALU 31%, 34%
+//   of wave time waiting; softcap and window 24%, 37%, 31%: two waves per SIMD
+//   do not cover the barrier, the softmax chain and LDS operand latency.
 #ifndef FA_PREFILL_PAIR_H
 #define FA_PREFILL_PAIR_H
 

@@ -5,7 +5,7 @@
   router, the decode path, or just the C-struct builder.
 * `oracle_attention(...)` is the CPU restatement under /oracle, computed in
   float64 (float32 and row chunks for full-size configurations).
-* `assert_parity(...)` is the acceptance bar of this build (north star):
+* `assert_parity(...)` is the acceptance bar of the tests:
   max |out - oracle| <= 2e-3 for fp16 outputs, <= 1e-2 for bf16, <= 1e-4 for
   fp32; max |lse - oracle| <= 1e-4.  Rows whose LSE is -inf in the oracle must
   be -inf in the result too.

@@ -2,7 +2,7 @@
 
 The request shapes, lengths and edge cases are data from the reference's
 own suite (flash_attn_mps tests/test_interface.py, cited per case); the
-checks are this build's: parity at the north-star bar (bf16 1e-2, fp16 2e-3,
+checks are this package's: parity at the harness's bar (bf16 1e-2, fp16 2e-3,
 fp32 1e-4, LSE 1e-4 max-abs), exact cache bytes, untouched sentinels, and
 outputs bit-identical across equivalent entry points.
 """

@@ -1,7 +1,7 @@
 """Single-query split-KV decode on gfx950 against the CPU oracle.
 
 Part of the cases are data from flash_attn_mps tests/test_decode.py (cited
-per case); the rest exercise this build's decode kernel: its 16-token page
+per case); the rest exercise this package's decode kernel: its 16-token page
 walk, padded head dims, head-group tiles and ALiBi.  Checks: parity bar
 (fp16 2e-3, bf16 1e-2, fp32 1e-4, LSE 1e-4 max-abs), NaN-poisoned slots that
 must never be read, sentinels around caller-owned outputs.  Where outputs are

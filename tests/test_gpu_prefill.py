@@ -3,7 +3,7 @@
 Covers the fast-path feature set: bf16/fp16, head dims 64/128/256, causal and
 non-causal, softcap, GQA ratios, packed and paged K/V, q_len != k_len
 (lower-right causality, rows with no visible key), partial query/key tiles,
-and that the MFMA path is the one taken.  Tolerances: this build's bar
+and that the MFMA path is the one taken.  Tolerances: this package's bar
 (max-abs <= 2e-3 fp16, <= 1e-2 bf16, LSE <= 1e-4).
 """
 import pytest
@@ -65,7 +65,7 @@ def test_prefill_gqa_ratios(device, hq, hkv):
                                       return_softmax_lse=True)
     ref, ref_lse = oracle_attention(q, k, v, cuq, cuk, causal=True)
     # The first rows of each request see a few keys (outputs near single V
-    # rows of |v| up to 4): the reference's tolerance there, this build's bar
+    # rows of |v| up to 4): the reference's tolerance there, this package's bar
     # on rows that see 32 keys or more.
     assert_parity(out, lse, ref, ref_lse, torch.bfloat16)
     rows = torch.cat([torch.arange(s + 31, s + n) for s, n in zip(cuq[:-1].tolist(), q_lens)])

@@ -10,7 +10,7 @@ cases pin, on either route, the work-list modes (compact up to 256 requests,
 the per-pair grid beyond) and one and two query heads per workgroup, strided
 V and output views (the second half's columns start DVT elements into the
 row, whatever the strides), spare output rows and columns that must stay
-unwritten, and E4M3 K/V on both its routes.  Bar: this build's (max-abs <=
+unwritten, and E4M3 K/V on both its routes.  Bar: this package's (max-abs <=
 1e-2 bf16, LSE <= 1e-4) on rows that see at least 32 keys, plus the all-rows
 check of assert_parity.
 """

@@ -9,7 +9,7 @@ them); mask descriptors and aux tensors as in flash_attn_mps/vllm.py:11-23 and
 tests/test_vllm.py:40-66.  Left padding (flash_attn_with_kvcache's
 cache_leftpad over a dense cache, interface.py:295-296) shifts a request's
 storage positions.  Every case asserts that fa_prefill_fwd takes the call,
-then holds outputs and LSE to this build's bar (bf16 1e-2, fp16 2e-3 max-abs,
+then holds outputs and LSE to this package's bar (bf16 1e-2, fp16 2e-3 max-abs,
 LSE 1e-4 on every row; -inf LSE where no key is visible).
 """
 import pytest

@@ -1,7 +1,7 @@
 """vLLM FLASH_ATTN / FLASH_ATTN_DIFFKV contract on gfx950 against the CPU oracle.
 
 Request shapes and feature values are data from flash_attn_mps
-tests/test_vllm.py (cited per case); the checks are this build's parity bar
+tests/test_vllm.py (cited per case); the checks are this package's parity bar
 (fp16 2e-3, bf16 1e-2, LSE 1e-4 max-abs), caller-owned outputs with
 untouched sentinels, and bit-exact batch invariance.
 """
