@@ -29,7 +29,7 @@
 // * Measured, 16 sequences of 256..4096 tokens, 16/8 heads, bf16, TFLOP/s of
 //   visible pairs, before -> here: causal 608 -> 721, softcap 556 -> 562, left
 //   window of 1023 291 -> 581, softcap and window 346 -> 538, not causal 712
-//   -> 828.  What bounds it now (counters): causal MFMA busy 29%, VALU 31%, 34%
+//   -> 828.  What bounds it now (counters): causal MFMA busy 30%, VALU 31%, 34%
 //   of wave time waiting; softcap and window 24%, 37%, 31%: two waves per SIMD
 //   do not cover the barrier, the softmax chain and LDS operand latency.
 #ifndef FA_PREFILL_PAIR_H
